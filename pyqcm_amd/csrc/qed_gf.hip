@@ -6,10 +6,14 @@
 //  * CPT / VCA / CDMFT k-sums: for every (w, k) the n x n complex matrix
 //    M = Gc(w)^-1 - V(k) is inverted (G_cpt = M^-1, src_qcm/CPT.cpp:76-86) or factorized
 //    (log|det(V Gc - 1)| = log|det Gc| + log|det M|, src_qcm/lattice_model_instance.cpp:624-643).
-//    n lanes hold one matrix, lane j owns column j in registers; the pivot column is
-//    broadcast with shuffles. Several matrices share a wave (n <= 16 -> >= 4 per wave).
+//    A few lanes hold one matrix, some rows each; 8 to 64 matrices share a wave.
 #include <cmath>
 #include <complex>
+#include <cstring>
+#include <memory>
+#include <mutex>
+#include <thread>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/qed.h"
@@ -31,9 +35,6 @@ __device__ __forceinline__ cplx cinv(cplx a) {
   return {a.re / d, -a.im / d};
 }
 __device__ __forceinline__ double cabs2(cplx a) { return a.re * a.re + a.im * a.im; }
-__device__ __forceinline__ cplx shfl(cplx v, int src) {
-  return {__shfl(v.re, src, 64), __shfl(v.im, src, 64)};
-}
 
 // ---- Lehmann G(z) --------------------------------------------------------------------
 // one workgroup per frequency; thread t accumulates element (b, a) = (t % L, t / L)
@@ -94,203 +95,366 @@ __global__ void k_cf_eval(int n, const int* __restrict__ off, const int* __restr
 }
 
 // ---- batched small complex matrices ---------------------------------------------------
+//
+// An n x n complex matrix (n <= 16, padded to N with an identity block) is held by LN
+// lanes, R = N / LN rows in the registers of each: row i = q + LN s lives in lane q, slot s.
+// Gauss-Jordan with partial pivoting, rows never moved: at step k the unused row with the
+// largest |re| or |im| in column k is the pivot; its lane writes it to LDS, every lane of
+// the group reads it back and eliminates its own rows.
+//
+// What bounds it: the 4 n^3 FP64 multiply-adds of the inversion (1.5 ms for the 8.4 million
+// 12 x 12 matrices of a 128^2 k x 512 w map at 78.6 TFLOP/s) and the LDS broadcast of the
+// pivot row, n 16-byte reads per step and wave. Few lanes with several rows each share one
+// broadcast among more matrices: 4 lanes x 3 rows put 16 matrices in a wave, against 5 when
+// every lane held one column and exchanged it by lane shuffles (n complex shuffles per step
+// and 8 n selects per row exchange; that form took 23.8 ms for the map above, this one
+// 4.6 ms, 25 TFLOP/s). Small sums (4 x 4, 32^2 k x 20 w) are bound by their four launches:
+// 98 us with 16 matrices in turn per group and 80 waves, 4.6 us with one per group.
 
 struct KsumArgs {
-  int n, nw, nterm, nk, mode;
-  const double* ginv;   // nw x n x n complex (column-major per matrix): Gc(w)^-1
-  const double* V0;     // n x n complex
-  const double* Vt;     // nterm x n x n complex
-  const double* nv;     // nterm x 3
-  const double* k;      // nk x 3
+  int n, nw, nk;        // nk: k points of this launch (k0: their first index of nk_all)
+  int k0, nk_all;
+  int chunk;            // matrices per group, one after the other
+  int nchunk;           // chunks per k block (modes 0, 1) or per frequency (modes 2, 3)
+  int part0, parts;     // first partial of this launch, partials per frequency (modes 2, 3)
+  const double* ginv;   // nw x N x N complex (column-major per matrix): Gc(w)^-1
+  const double* vk;     // nk x N x N complex: V(k)
   double* out;
-  double* part;         // partial sums (mode 2: per group n x n; sef: per group scalar)
-  int kchunk;           // k points per group
+  double* part;
 };
 
-// Builds column j of M = Ginv(w) - V(k) into reg[0..N)
-template <int N>
-__device__ __forceinline__ void build_column(const KsumArgs& A, int w, int kk, int j, cplx* col) {
-  const double* gi = A.ginv + ((size_t)w * N * N + (size_t)j * N) * 2;
-  const double* v0 = A.V0 + (size_t)j * N * 2;
-#pragma unroll
-  for (int i = 0; i < N; ++i) col[i] = {gi[2 * i] - v0[2 * i], gi[2 * i + 1] - v0[2 * i + 1]};
-  const double kx = A.k[3 * kk], ky = A.k[3 * kk + 1], kz = A.k[3 * kk + 2];
-  for (int t = 0; t < A.nterm; ++t) {
-    const double ph = 2.0 * M_PI * (kx * A.nv[3 * t] + ky * A.nv[3 * t + 1] + kz * A.nv[3 * t + 2]);
-    double s, c;
-    sincos(ph, &s, &c);
-    const double* vt = A.Vt + ((size_t)t * N * N + (size_t)j * N) * 2;
-#pragma unroll
-    for (int i = 0; i < N; ++i) {
-      cplx v{vt[2 * i], vt[2 * i + 1]};
-      cplx e = cmul(v, cplx{c, s});
-      col[i] = csub(col[i], e);
-    }
-  }
+__device__ __forceinline__ uint32_t dpp_max(uint32_t v, uint32_t w) { return v > w ? v : w; }
+
+// the maximum of v over the LN lanes of a group (LN = 1, 2, 4, 8; aligned groups)
+template <int LN>
+__device__ __forceinline__ uint32_t group_max(uint32_t v) {
+  if constexpr (LN >= 2)  // quad_perm [1,0,3,2]
+    v = dpp_max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xf, 0xf, true));
+  if constexpr (LN >= 4)  // quad_perm [2,3,0,1]
+    v = dpp_max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x4E, 0xf, 0xf, true));
+  if constexpr (LN >= 8)  // row_half_mirror: lane i of eight <-> 7 - i
+    v = dpp_max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x141, 0xf, 0xf, true));
+  return v;
 }
 
-// In-place Gauss-Jordan inversion of the matrix whose column j lives in col (lane base+j of
-// a group of N lanes). Returns log|det| in every lane.
-template <int N>
-__device__ __forceinline__ double gj_invert(cplx* col, int base, int j, bool want_inverse) {
-  int perm[N];
-  double logdet = 0.0;
+__device__ __forceinline__ uint32_t mag_bits(cplx v) {  // monotone in max(|re|, |im|)
+  const uint32_t r = (uint32_t)((uint64_t)__double_as_longlong(v.re) >> 32) << 1;
+  const uint32_t i = (uint32_t)((uint64_t)__double_as_longlong(v.im) >> 32) << 1;
+  return r > i ? r : i;
+}
+
+// log|det| as a product of |pivot|^2 kept in (0, 1) and a power of two
+struct LogDet {
+  double m = 1.0;
+  int e = 0;
+  __device__ __forceinline__ void mul(double c2) {
+    const double p = m * __builtin_amdgcn_frexp_mant(c2);
+    e += __builtin_amdgcn_frexp_exp(c2) + __builtin_amdgcn_frexp_exp(p);
+    m = __builtin_amdgcn_frexp_mant(p);
+  }
+  __device__ __forceinline__ double value() const { return 0.5 * (log(m) + (double)e * M_LN2); }
+};
+
+// One elimination of the group's matrix. INV: the inverse in place, C = (P A)^-1 with the
+// row that was the pivot of step k holding C[k][:], so that A^-1[k][p_j] = C[k][j]; the
+// pivot rows p_j are the nibbles of perm and step[s] is the k of this lane's row s.
+// Otherwise the rows below only (the determinant). buf: N double2 of LDS for the group.
+template <int N, int LN, bool INV>
+__device__ __forceinline__ void eliminate(cplx (&a)[N / LN][N], int q, double2* buf, uint64_t& perm,
+                                          int (&step)[N / LN], LogDet& ld, bool& zero) {
+  constexpr int R = N / LN;
+  perm = 0;
+#pragma unroll
+  for (int s = 0; s < R; ++s) step[s] = -1;
 #pragma unroll
   for (int k = 0; k < N; ++k) {
-    // pivot search in column k (held by lane base+k)
-    int p = k;
-    double best = -1.0;
+    uint32_t key = 0;
 #pragma unroll
-    for (int i = 0; i < N; ++i) {
-      double m = (i >= k) ? cabs2(col[i]) : -1.0;
-      if (m > best) {
-        best = m;
-        p = i;
+    for (int s = 0; s < R; ++s) {
+      const uint32_t m = (mag_bits(a[s][k]) & ~31u) | 16u | (uint32_t)(q + LN * s);
+      key = dpp_max(key, step[s] < 0 ? m : 0u);
+    }
+    key = group_max<LN>(key);
+    const int p = (int)(key & 15u);
+    perm |= (uint64_t)p << (4 * k);
+#pragma unroll
+    for (int s = 0; s < R; ++s) {
+      if (p == q + LN * s) {
+#pragma unroll
+        for (int j = 0; j < N; ++j) {
+          if (!INV && j < k) continue;
+          buf[j] = make_double2(a[s][j].re, a[s][j].im);
+          a[s][j] = {0.0, 0.0};
+        }
+        step[s] = k;
       }
     }
-    p = __shfl(p, base + k, 64);
-    perm[k] = p;
-    // swap rows k and p in every column
-    cplx rk = col[k], rp = col[k];
+    // the reads below see the pivot lane's writes: LDS accesses of a wave complete in
+    // order, the fence keeps the compiler from reusing values of an earlier step
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    cplx rp[N];
 #pragma unroll
-    for (int i = 0; i < N; ++i)
-      if (i == p) rp = col[i];
+    for (int j = 0; j < N; ++j) {
+      if (!INV && j < k) continue;
+      const double2 t = buf[j];
+      rp[j] = {t.x, t.y};
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    const double c2 = cabs2(rp[k]);
+    if (!INV) ld.mul(c2);
+    else zero |= rp[k].re == 0.0 && rp[k].im == 0.0;
+    const double ic2 = 1.0 / c2;
+    const cplx dinv{rp[k].re * ic2, -rp[k].im * ic2};
 #pragma unroll
-    for (int i = 0; i < N; ++i)
-      if (i == p) col[i] = rk;
-    col[k] = rp;
-    // broadcast column k after the swap
-    cplx ck[N];
+    for (int s = 0; s < R; ++s) {
+      cplx f = cmul(a[s][k], dinv);
+      if (INV) {
+        if (p == q + LN * s) f = {-dinv.re, -dinv.im};
+        a[s][k] = {-f.re, -f.im};
+      }
 #pragma unroll
-    for (int i = 0; i < N; ++i) ck[i] = shfl(col[i], base + k);
-    const cplx piv = ck[k];
-    logdet += 0.5 * log(cabs2(piv));
-    if (!want_inverse) {
-      // plain elimination below the pivot (determinant only)
-      const cplx dinv = cinv(piv);
-      const cplx f = cmul(col[k], dinv);
+      for (int j = 0; j < N; ++j) {
+        if (j == k || (!INV && j < k)) continue;
+        a[s][j].re = fma(-f.re, rp[j].re, a[s][j].re);
+        a[s][j].re = fma(f.im, rp[j].im, a[s][j].re);
+        a[s][j].im = fma(-f.re, rp[j].im, a[s][j].im);
+        a[s][j].im = fma(-f.im, rp[j].re, a[s][j].im);
+      }
+    }
+  }
+}
+
+// lanes per matrix for each padded dimension
+template <int N>
+constexpr int lanes_of() {
+  return N == 16 ? 8 : N >= 4 ? 4 : N;
+}
+
+// V(k) = V0 + sum_t Vt e^(2 pi i k.n_t), padded to N x N with zeros; one block per 8 k points
+template <int N>
+__global__ __launch_bounds__(256) void k_vk(int n, int nterm, int nk, const double* __restrict__ V0,
+                                            const double* __restrict__ Vt, const double* __restrict__ nv,
+                                            const double* __restrict__ kk, double* __restrict__ vk) {
+  constexpr int KB = 8, TB = 32;
+  __shared__ double2 ph[KB][TB];
+  const int kb = blockIdx.x * KB;
+  constexpr int E = (KB * N * N + 255) / 256;
+  cplx acc[E];
 #pragma unroll
-      for (int i = 0; i < N; ++i)
-        if (i > k) col[i] = csub(col[i], cmul(ck[i], f));
+  for (int u = 0; u < E; ++u) {
+    const int e = (threadIdx.x + 256 * u) % (N * N), i = e % N, j = e / N;
+    acc[u] = {0.0, 0.0};
+    if (i < n && j < n) acc[u] = {V0[2 * (i + j * n)], V0[2 * (i + j * n) + 1]};
+  }
+  for (int t0 = 0; t0 < nterm; t0 += TB) {
+    const int tc = min(TB, nterm - t0);
+    __syncthreads();
+    for (int u = threadIdx.x; u < KB * TB; u += 256) {
+      const int t = u % TB, kq = min(kb + u / TB, nk - 1);
+      if (t < tc) {
+        const double* v = nv + 3 * (t0 + t);
+        double s, c;
+        sincospi(2.0 * (kk[3 * (size_t)kq] * v[0] + kk[3 * (size_t)kq + 1] * v[1] + kk[3 * (size_t)kq + 2] * v[2]), &s, &c);
+        ph[u / TB][t] = make_double2(c, s);
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < E; ++u) {
+      const int id = threadIdx.x + 256 * u;
+      const int e = id % (N * N), i = e % N, j = e / N, kq = id / (N * N);
+      if (kq >= KB || i >= n || j >= n) continue;
+      for (int t = 0; t < tc; ++t) {
+        const double* m = Vt + 2 * ((size_t)(t0 + t) * n * n + i + (size_t)j * n);
+        const double2 p = ph[kq][t];
+        acc[u] = cadd(acc[u], cmul(cplx{m[0], m[1]}, cplx{p.x, p.y}));
+      }
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < E; ++u) {
+    const int id = threadIdx.x + 256 * u;
+    const int kq = id / (N * N);
+    if (kq >= KB || kb + kq >= nk) continue;
+    reinterpret_cast<double2*>(vk)[(size_t)(kb + kq) * N * N + id % (N * N)] = make_double2(acc[u].re, acc[u].im);
+  }
+}
+
+// Gc(w)^-1 padded with an identity block, log|det Gc(w)| and whether a pivot vanished
+template <int N>
+__global__ __launch_bounds__(64) void k_gc_inverse(int n, int nw, const double* __restrict__ Gc,
+                                                   double* __restrict__ ginv, double* __restrict__ logdet,
+                                                   int* __restrict__ singular) {
+  constexpr int LN = lanes_of<N>(), R = N / LN, G = 64 / LN;
+  __shared__ double2 buf[G][N + 1];
+  const int g = threadIdx.x / LN, q = threadIdx.x % LN;
+  const int w = min((int)blockIdx.x * G + g, nw - 1);
+  const double2* src = reinterpret_cast<const double2*>(Gc) + (size_t)w * n * n;
+  for (int pass = 0; pass < 2; ++pass) {
+    cplx a[R][N];
+#pragma unroll
+    for (int s = 0; s < R; ++s)
+#pragma unroll
+      for (int j = 0; j < N; ++j) {
+        const int i = q + LN * s;
+        a[s][j] = {i == j ? 1.0 : 0.0, 0.0};
+        if (i < n && j < n) {
+          const double2 v = src[i + j * n];
+          a[s][j] = {v.x, v.y};
+        }
+      }
+    uint64_t perm;
+    int step[R];
+    LogDet ld;
+    bool zero = false;
+    if (pass == 0) {
+      if (!logdet) continue;
+      eliminate<N, LN, false>(a, q, buf[g], perm, step, ld, zero);
+      if (q == 0) logdet[w] = ld.value();
       continue;
     }
-    const cplx dinv = cinv(piv);
-    // row k scaled; column k replaced by the eliminator
-    const cplx rowk = (j == k) ? cplx{1.0, 0.0} : col[k];
-    const cplx rs = cmul(rowk, dinv);
+    eliminate<N, LN, true>(a, q, buf[g], perm, step, ld, zero);
+    if (zero) *singular = 1;
+    double2* o = reinterpret_cast<double2*>(ginv) + (size_t)w * N * N;
 #pragma unroll
-    for (int i = 0; i < N; ++i) {
-      if (i == k) {
-        col[i] = rs;
-      } else {
-        cplx base_v = (j == k) ? cplx{0.0, 0.0} : col[i];
-        col[i] = csub(base_v, cmul(ck[i], rs));
-      }
-    }
-  }
-  if (want_inverse) {
-    // undo the row interchanges as column interchanges, last first
+    for (int s = 0; s < R; ++s)
 #pragma unroll
-    for (int k = N - 1; k >= 0; --k) {
-      const int p = perm[k];
-      if (p == k) continue;
-      // lanes k and p exchange their columns
-      const int src = (j == k) ? p : ((j == p) ? k : j);
-#pragma unroll
-      for (int i = 0; i < N; ++i) col[i] = shfl(col[i], base + src);
-    }
-  }
-  return logdet;
-}
-
-// At least two wavefronts per SIMD: the fully unrolled elimination of a 12- or 16-wide
-// matrix otherwise takes over 256 registers and runs one wavefront per SIMD (measured on
-// the 3x4 cluster: 30.7 ms at one, 22.4 ms at two with a few spilled registers, 25.3 ms at
-// three with more spills; 16 wide on 128^2 k x 512 w: 86.3 ms at one, 59.8 ms at two)
-template <int N>
-__global__ __launch_bounds__(256, 2) void k_ksum(KsumArgs A) {
-  constexpr int GPW = 64 / N;  // groups per wave
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int g = lane / N, j = lane % N;
-  const int base = g * N;
-  const bool lane_ok = g < GPW;
-  const int gid = (blockIdx.x * 4 + wave) * GPW + g;  // global group id
-  const int ngroups_k = (A.nk + A.kchunk - 1) / A.kchunk;
-  const int w = gid / ngroups_k, kc = gid % ngroups_k;
-  const bool act = lane_ok && w < A.nw;
-  cplx acc[N];
-#pragma unroll
-  for (int i = 0; i < N; ++i) acc[i] = {0.0, 0.0};
-  double sef = 0.0;
-  if (act) {
-    const int k0 = kc * A.kchunk, k1 = min(A.nk, k0 + A.kchunk);
-    for (int kk = k0; kk < k1; ++kk) {
-      cplx col[N];
-      build_column<N>(A, w, kk, j, col);
-      const double ld = gj_invert<N>(col, base, j, A.mode != 3);
-      if (A.mode == 0) {
-        double* o = A.out + (((size_t)w * A.nk + kk) * N * N + (size_t)j * N) * 2;
-#pragma unroll
-        for (int i = 0; i < N; ++i) {
-          o[2 * i] = col[i].re;
-          o[2 * i + 1] = col[i].im;
-        }
-      } else if (A.mode == 1) {
-        // trace: lane j contributes element (j, j)
-        cplx d{0.0, 0.0};
-#pragma unroll
-        for (int i = 0; i < N; ++i)
-          if (i == j) d = col[i];
-        double tr = d.re, ti = d.im;
-        if constexpr ((N & (N - 1)) == 0) {
-          for (int o = 1; o < N; o <<= 1) {
-            tr += __shfl_xor(tr, o, 64);
-            ti += __shfl_xor(ti, o, 64);
-          }
-        } else {
-          // groups of N lanes do not align with xor butterflies: gather the diagonal
-          double sr = 0.0, si = 0.0;
-#pragma unroll
-          for (int i = 0; i < N; ++i) {
-            sr += __shfl(tr, base + i, 64);
-            si += __shfl(ti, base + i, 64);
-          }
-          tr = sr;
-          ti = si;
-        }
-        if (j == 0) {
-          A.out[2 * ((size_t)w * A.nk + kk)] = tr;
-          A.out[2 * ((size_t)w * A.nk + kk) + 1] = ti;
-        }
-      } else if (A.mode == 2) {
-#pragma unroll
-        for (int i = 0; i < N; ++i) acc[i] = cadd(acc[i], col[i]);
-      } else {
-        sef += ld;
-      }
-    }
-    if (A.mode == 2) {
-      double* o = A.part + (((size_t)w * ngroups_k + kc) * N * N + (size_t)j * N) * 2;
-#pragma unroll
-      for (int i = 0; i < N; ++i) {
-        o[2 * i] = acc[i].re;
-        o[2 * i + 1] = acc[i].im;
-      }
-    } else if (A.mode == 3 && j == 0) {
-      A.part[(size_t)w * ngroups_k + kc] = sef;
-    }
+      for (int j = 0; j < N; ++j)
+        o[step[s] + (size_t)((perm >> (4 * j)) & 15u) * N] = make_double2(a[s][j].re, a[s][j].im);
   }
 }
 
-// sum of partials over k-chunks
-__global__ void k_ksum_reduce(int nw, int nparts, int len, const double* __restrict__ part,
-                              double scale, double* __restrict__ out) {
-  int id = blockIdx.x * blockDim.x + threadIdx.x;
-  if (id >= nw * len) return;
-  int w = id / len, q = id % len;
-  double s = 0.0;
-  for (int p = 0; p < nparts; ++p) s += part[((size_t)w * nparts + p) * len + q];
-  out[id] = s * scale;
+// M(w, k) = Gc(w)^-1 - V(k) for the (w, k) of a launch. MODE 0: the inverses; 1: their
+// traces; 2: their sum over k; 3: the sum over k of log|det|. A group takes `chunk`
+// matrices in turn: one k point and a run of frequencies (modes 0, 1), or one frequency and
+// a run of k blocks (modes 2, 3). Two waves per SIMD, which the 12-wide form just fits
+// (250 registers); the sum over k of wide matrices takes 40 KB of LDS and one wave.
+template <int N, int MODE>
+__global__ __launch_bounds__(64, MODE == 2 && N >= 12 ? 1 : 2) void k_ksum(KsumArgs A) {
+  constexpr int LN = lanes_of<N>(), R = N / LN, G = 64 / LN;
+  __shared__ double2 buf[G][N + 1];
+  __shared__ double2 acc[MODE == 2 ? G : 1][MODE == 2 ? N * N + 1 : 1];
+  const int g = threadIdx.x / LN, q = threadIdx.x % LN;
+  const int b = blockIdx.x;
+  const int nkb = (A.nk + G - 1) / G;
+  const int fix = MODE < 2 ? b % nkb : b / A.nchunk;      // k block / frequency
+  const int c0 = (MODE < 2 ? b / nkb : b % A.nchunk) * A.chunk;
+  const int c1 = min(c0 + A.chunk, MODE < 2 ? A.nw : nkb);
+  if constexpr (MODE == 2) {
+    for (int e = q; e < N * N; e += LN) acc[g][e] = make_double2(0.0, 0.0);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  }
+  LogDet ld;
+  for (int c = c0; c < c1; ++c) {
+    const int w = MODE < 2 ? c : fix;
+    const int kr = (MODE < 2 ? fix : c) * G + g;
+    const bool ok = kr < A.nk;
+    const int kc = ok ? kr : A.nk - 1;
+    const double2* gi = reinterpret_cast<const double2*>(A.ginv) + (size_t)w * N * N;
+    const double2* vk = reinterpret_cast<const double2*>(A.vk) + (size_t)kc * N * N;
+    cplx a[R][N];
+#pragma unroll
+    for (int j = 0; j < N; ++j)
+#pragma unroll
+      for (int s = 0; s < R; ++s) {
+        const double2 x = gi[j * N + q + LN * s], v = vk[j * N + q + LN * s];
+        a[s][j] = {x.x - v.x, x.y - v.y};
+      }
+    uint64_t perm;
+    int step[R];
+    bool zero = false;
+    LogDet one;
+    eliminate<N, LN, MODE != 3>(a, q, buf[g], perm, step, one, zero);
+    if constexpr (MODE == 0) {
+      double2* o = reinterpret_cast<double2*>(A.out) + ((size_t)w * A.nk_all + A.k0 + kc) * A.n * A.n;
+#pragma unroll
+      for (int s = 0; s < R; ++s)
+#pragma unroll
+        for (int j = 0; j < N; ++j) {
+          const int col = (int)((perm >> (4 * j)) & 15u);
+          if (ok && step[s] < A.n && col < A.n) o[step[s] + col * A.n] = make_double2(a[s][j].re, a[s][j].im);
+        }
+    } else if constexpr (MODE == 1) {
+      cplx d{0.0, 0.0};
+#pragma unroll
+      for (int s = 0; s < R; ++s)
+#pragma unroll
+        for (int j = 0; j < N; ++j)
+          if (step[s] < A.n && (int)((perm >> (4 * j)) & 15u) == step[s]) d = cadd(d, a[s][j]);
+#pragma unroll
+      for (int o = 1; o < LN; o <<= 1) {
+        d.re += __shfl_xor(d.re, o, 64);
+        d.im += __shfl_xor(d.im, o, 64);
+      }
+      if (ok && q == 0)
+        reinterpret_cast<double2*>(A.out)[(size_t)w * A.nk_all + A.k0 + kc] = make_double2(d.re, d.im);
+    } else if constexpr (MODE == 2) {
+      // element (step, p_j) has one owner in the group
+      if (ok) {
+#pragma unroll
+        for (int s = 0; s < R; ++s)
+#pragma unroll
+          for (int j = 0; j < N; ++j) {
+            double2* t = &acc[g][step[s] + (int)((perm >> (4 * j)) & 15u) * N];
+            const double2 v = *t;
+            *t = make_double2(v.x + a[s][j].re, v.y + a[s][j].im);
+          }
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+    } else {
+      if (ok) {
+        ld.mul(one.m);
+        ld.e += one.e;
+      }
+    }
+  }
+  if constexpr (MODE == 2) {
+    double2* o = reinterpret_cast<double2*>(A.part) + ((size_t)fix * A.parts + A.part0 + b % A.nchunk) * N * N;
+    for (int e = threadIdx.x; e < N * N; e += 64) {
+      double2 t = make_double2(0.0, 0.0);
+      for (int h = 0; h < G; ++h) {
+        t.x += acc[h][e].x;
+        t.y += acc[h][e].y;
+      }
+      o[e] = t;
+    }
+  }
+  if constexpr (MODE == 3) {
+    double v = q == 0 ? ld.value() : 0.0;
+    v = wave_sum(v);
+    if (threadIdx.x == 0) A.part[(size_t)fix * A.parts + A.part0 + b % A.nchunk] = v;
+  }
+}
+
+// sums of the partials over the k chunks: out[w][i + j n] from parts x (N x N complex), or
+// out[w] from parts (n = 0); one wave per output
+__global__ __launch_bounds__(64) void k_ksum_reduce(int parts, int n, int N, const double* __restrict__ part,
+                                                    double scale, double* __restrict__ out) {
+  const int lane = threadIdx.x;
+  if (n == 0) {
+    double s = 0.0;
+    for (int p = lane; p < parts; p += 64) s += part[(size_t)blockIdx.x * parts + p];
+    s = wave_sum(s);
+    if (lane == 0) out[blockIdx.x] = s * scale;
+    return;
+  }
+  const int w = blockIdx.x / n, j = blockIdx.x % n;  // one column of one frequency
+  const double2* src = reinterpret_cast<const double2*>(part) + (size_t)w * parts * N * N + (size_t)j * N;
+  for (int i = 0; i < n; ++i) {
+    double re = 0.0, im = 0.0;
+    for (int p = lane; p < parts; p += 64) {
+      const double2 v = src[(size_t)p * N * N + i];
+      re += v.x;
+      im += v.y;
+    }
+    re = wave_sum(re);
+    im = wave_sum(im);
+    if (lane == 0) reinterpret_cast<double2*>(out)[(size_t)w * n * n + (size_t)j * n + i] = make_double2(re * scale, im * scale);
+  }
 }
 
 template <class T>
@@ -298,47 +462,6 @@ DevBuf up(const T* p, size_t n) {
   DevBuf b(std::max<size_t>(n, 1) * sizeof(T));
   if (n) QED_HIP(hipMemcpyAsync(b.p, p, n * sizeof(T), hipMemcpyHostToDevice, stream()));
   return b;
-}
-
-template <int N>
-void launch_ksum(KsumArgs A, int ngroups) {
-  constexpr int GPW = 64 / N;
-  const int waves = (ngroups + GPW - 1) / GPW;
-  const int blocks = (waves + 3) / 4;
-  k_ksum<N><<<blocks, 256, 0, stream()>>>(A);
-}
-
-void ksum_dispatch(KsumArgs A, int ngroups) {
-  switch (A.n) {
-    case 1: launch_ksum<1>(A, ngroups); break;
-    case 2: launch_ksum<2>(A, ngroups); break;
-    case 4: launch_ksum<4>(A, ngroups); break;
-    case 5: case 6: case 7: case 8: launch_ksum<8>(A, ngroups); break;
-    case 12: launch_ksum<12>(A, ngroups); break;  // 5 groups of 12 lanes per wave
-    case 16: launch_ksum<16>(A, ngroups); break;
-    default: fail("lattice k-sum: cluster Green function dimension above 16 is not supported");
-  }
-  QED_HIP(hipGetLastError());
-}
-
-// Pads n x n complex matrices to N x N (identity padding for inverse-like uses, zero for V)
-std::vector<double> pad_mats(const double* src, int count, int n, int N, bool identity) {
-  std::vector<double> out((size_t)count * N * N * 2, 0.0);
-  for (int c = 0; c < count; ++c) {
-    for (int j = 0; j < N; ++j)
-      for (int i = 0; i < N; ++i) {
-        double re = 0.0, im = 0.0;
-        if (i < n && j < n) {
-          re = src[(((size_t)c * n * n) + i + (size_t)j * n) * 2];
-          im = src[(((size_t)c * n * n) + i + (size_t)j * n) * 2 + 1];
-        } else if (identity && i == j) {
-          re = 1.0;
-        }
-        out[(((size_t)c * N * N) + i + (size_t)j * N) * 2] = re;
-        out[(((size_t)c * N * N) + i + (size_t)j * N) * 2 + 1] = im;
-      }
-  }
-  return out;
 }
 
 int padded_dim(int n) {
@@ -350,28 +473,26 @@ int padded_dim(int n) {
   fail("lattice k-sum: cluster Green function dimension above 16 is not supported");
 }
 
-// Gc(w)^-1 for each frequency (host, n <= 16), padded to N
-std::vector<double> inverse_gc(const double* Gc, int nw, int n, int N, std::vector<double>* logdet) {
-  std::vector<double> out((size_t)nw * N * N * 2, 0.0);
-  if (logdet) logdet->assign(nw, 0.0);
-  std::vector<std::complex<double>> a((size_t)n * n);
-  for (int w = 0; w < nw; ++w) {
-    for (size_t q = 0; q < (size_t)n * n; ++q)
-      a[q] = {Gc[((size_t)w * n * n + q) * 2], Gc[((size_t)w * n * n + q) * 2 + 1]};
-    if (logdet) {
-      std::vector<std::complex<double>> b(a);
-      (*logdet)[w] = clogabsdet(n, b.data());
-    }
-    if (!cinverse(n, a.data())) fail("cluster Green function is singular at a requested frequency");
-    for (int j = 0; j < N; ++j)
-      for (int i = 0; i < N; ++i) {
-        std::complex<double> v = (i < n && j < n) ? a[i + (size_t)j * n]
-                                                  : std::complex<double>(i == j ? 1.0 : 0.0, 0.0);
-        out[(((size_t)w * N * N) + i + (size_t)j * N) * 2] = v.real();
-        out[(((size_t)w * N * N) + i + (size_t)j * N) * 2 + 1] = v.imag();
-      }
+template <class F>
+void with_dim(int N, F&& f) {
+  switch (N) {
+    case 1: f(std::integral_constant<int, 1>{}); break;
+    case 2: f(std::integral_constant<int, 2>{}); break;
+    case 4: f(std::integral_constant<int, 4>{}); break;
+    case 8: f(std::integral_constant<int, 8>{}); break;
+    case 12: f(std::integral_constant<int, 12>{}); break;
+    default: f(std::integral_constant<int, 16>{}); break;
   }
-  return out;
+}
+
+template <int N>
+void launch_ksum(const KsumArgs& A, int mode, int blocks) {
+  switch (mode) {
+    case 0: k_ksum<N, 0><<<blocks, 64, 0, stream()>>>(A); break;
+    case 1: k_ksum<N, 1><<<blocks, 64, 0, stream()>>>(A); break;
+    case 2: k_ksum<N, 2><<<blocks, 64, 0, stream()>>>(A); break;
+    default: k_ksum<N, 3><<<blocks, 64, 0, stream()>>>(A); break;
+  }
 }
 
 // device time of the last CPT k-sum (HIP events on the library stream)
@@ -380,25 +501,194 @@ double& last_ksum_ms() {
   return ms;
 }
 
-struct KsumTimer {
-  hipEvent_t a = nullptr, b = nullptr;
-  KsumTimer() {
-    QED_HIP(hipEventCreate(&a));
-    QED_HIP(hipEventCreate(&b));
-    QED_HIP(hipEventRecord(a, stream()));
+// Device memory, pinned host memory and events of one k-sum call. Calls take a free one and
+// give it back (concurrent calls have one each); at most kKeep are kept, and none with more
+// than kKeepBytes of either memory, so that small calls allocate nothing.
+struct KsumSpace {
+  DevBuf dev;
+  unsigned char* pin = nullptr;
+  size_t pin_bytes = 0;
+  hipEvent_t ev[2] = {nullptr, nullptr};
+  KsumSpace() = default;
+  KsumSpace(const KsumSpace&) = delete;
+  ~KsumSpace() {
+    if (pin) (void)hipHostFree(pin);
+    for (hipEvent_t e : ev)
+      if (e) (void)hipEventDestroy(e);
   }
-  void stop() {
-    QED_HIP(hipEventRecord(b, stream()));
-    QED_HIP(hipEventSynchronize(b));
-    float ms = 0.0f;
-    QED_HIP(hipEventElapsedTime(&ms, a, b));
-    last_ksum_ms() = ms;
-  }
-  ~KsumTimer() {
-    if (a) (void)hipEventDestroy(a);
-    if (b) (void)hipEventDestroy(b);
+  void reserve(size_t d, size_t p) {
+    if (dev.bytes < d) dev.alloc(d);
+    if (pin_bytes < p) {
+      if (pin) (void)hipHostFree(pin);
+      pin = nullptr;
+      pin_bytes = 0;
+      QED_HIP(hipHostMalloc((void**)&pin, p, hipHostMallocDefault));
+      pin_bytes = p;
+    }
+    for (hipEvent_t& e : ev)
+      if (!e) QED_HIP(hipEventCreate(&e));
   }
 };
+
+class KsumLease {
+ public:
+  KsumLease() {
+    std::lock_guard<std::mutex> lk(mutex());
+    if (!idle().empty()) {
+      s_ = std::move(idle().back());
+      idle().pop_back();
+    } else {
+      s_ = std::make_unique<KsumSpace>();
+    }
+  }
+  ~KsumLease() {
+    (void)hipStreamSynchronize(stream());  // also after a failure: nothing may still use the memory
+    if (s_->dev.bytes > kKeepBytes || s_->pin_bytes > kKeepBytes) return;
+    std::lock_guard<std::mutex> lk(mutex());
+    if (idle().size() < kKeep) idle().push_back(std::move(s_));
+  }
+  KsumSpace* operator->() { return s_.get(); }
+
+ private:
+  static constexpr size_t kKeep = 4, kKeepBytes = size_t(64) << 20;
+  static std::mutex& mutex() {
+    static std::mutex m;
+    return m;
+  }
+  static std::vector<std::unique_ptr<KsumSpace>>& idle() {  // never destroyed: the runtime may be gone by then
+    static auto* v = new std::vector<std::unique_ptr<KsumSpace>>();
+    return *v;
+  }
+  std::unique_ptr<KsumSpace> s_;
+};
+
+// Copies bytes from the device to caller memory through the pinned buffer, in pieces: while
+// one piece is on its way the threads copy the previous one out (the caller's pages are
+// often touched for the first time here, which is what a single thread is slow at).
+void copy_out(unsigned char* dst, const unsigned char* src_dev, size_t bytes, unsigned char* pin, size_t pin_bytes) {
+  const size_t piece = pin_bytes / 2;
+  const int nt = bytes >= (size_t(8) << 20) ? 8 : 1;
+  auto send = [&](size_t i) {
+    const size_t o = i * piece;
+    if (o < bytes)
+      QED_HIP(hipMemcpyAsync(pin + (i & 1) * piece, src_dev + o, std::min(piece, bytes - o), hipMemcpyDeviceToHost, stream()));
+  };
+  send(0);
+  for (size_t i = 0; i * piece < bytes; ++i) {
+    QED_HIP(hipStreamSynchronize(stream()));
+    send(i + 1);
+    const size_t o = i * piece, len = std::min(piece, bytes - o);
+    const unsigned char* from = pin + (i & 1) * piece;
+    const size_t per = ((len + nt - 1) / nt + 4095) & ~size_t(4095);
+    std::vector<std::thread> th;
+    for (int t = 1; t < nt && t * per < len; ++t)
+      th.emplace_back([=] { std::memcpy(dst + o + t * per, from + t * per, std::min(per, len - t * per)); });
+    std::memcpy(dst + o, from, std::min(per, len));
+    for (auto& t : th) t.join();
+  }
+}
+
+// The k-sums of mode 0 to 3 (see k_ksum) for host inputs: one upload, Gc^-1 and V(k) on the
+// device, the sums, one download in the caller's layout.
+void ksum(int n, int nw, const double* Gc, const double* V0, int nterm, const double* Vt, const double* nv, int nk,
+          const double* k, int mode, double* out) {
+  const int N = padded_dim(n), LN = N == 16 ? 8 : N >= 4 ? 4 : N, G = 64 / LN;
+  const size_t n2 = 2 * (size_t)n * n, N2 = 2 * (size_t)N * N;  // doubles per matrix
+  // V(k) of as many k points at a time as 256 MB hold
+  const int kmax = (int)std::max<size_t>(G, std::min<size_t>(nk, (size_t(256) << 20) / (N2 * 8) / G * G));
+  // Matrices per group: about 4096 waves (two per SIMD of 256 CUs, twice over), one matrix
+  // each when there are fewer
+  const long nkb_all = (nk + G - 1) / G;
+  const long runs = mode < 2 ? nw : (kmax + G - 1) / G;
+  const int chunk = (int)std::max<long>(1, std::min<long>(runs, nkb_all * nw / 4096));
+  int parts = 0;
+  for (int k0 = 0; k0 < nk; k0 += kmax)
+    if (mode >= 2) parts += ((std::min(kmax, nk - k0) + G - 1) / G + chunk - 1) / chunk;
+  const size_t out_len = mode == 0 ? (size_t)nw * nk * n2 : mode == 1 ? (size_t)nw * nk * 2 : mode == 2 ? nw * n2 : (size_t)nw;
+  // inputs in the order of the upload, then the device's own arrays (doubles)
+  size_t off = 0;
+  auto take = [&](size_t len) {
+    const size_t o = off;
+    off += (len + 31) & ~size_t(31);
+    return o;
+  };
+  const size_t o_gc = take(nw * n2), o_v0 = take(n2), o_vt = take(nterm * n2), o_nv = take(3 * (size_t)nterm),
+               o_k = take(3 * (size_t)nk), n_in = off;
+  const size_t o_gi = take(nw * N2), o_vk = take(kmax * N2),
+               o_part = take(mode == 2 ? nw * (size_t)parts * N2 : mode == 3 ? nw * (size_t)parts : 0),
+               o_ld = take(nw + 1), o_out = take(out_len);
+  // small results come down with log|det Gc| and the singular flag in one copy; large ones
+  // after them, in pieces
+  const size_t n_down = off - o_ld;
+  const bool small = n_down * 8 <= (size_t(1) << 20);
+  KsumLease L;
+  const size_t piece = size_t(16) << 20;
+  L->reserve(off * 8, std::max(n_in, small ? n_down : std::max<size_t>(nw + 1, 2 * piece / 8)) * 8);
+  double* d = L->dev.as<double>();
+  double* h = reinterpret_cast<double*>(L->pin);
+  std::memcpy(h + o_gc, Gc, nw * n2 * 8);
+  std::memcpy(h + o_v0, V0, n2 * 8);
+  if (nterm > 0) {
+    std::memcpy(h + o_vt, Vt, nterm * n2 * 8);
+    std::memcpy(h + o_nv, nv, 3 * (size_t)nterm * 8);
+  }
+  std::memcpy(h + o_k, k, 3 * (size_t)nk * 8);
+  hipStream_t st = stream();
+  QED_HIP(hipMemcpyAsync(d, h, n_in * 8, hipMemcpyHostToDevice, st));
+  double* ld = d + o_ld;
+  int* singular = reinterpret_cast<int*>(ld + nw);
+  QED_HIP(hipMemsetAsync(singular, 0, 8, st));
+  QED_HIP(hipEventRecord(L->ev[0], st));
+  with_dim(N, [&](auto dim) {
+    constexpr int M = decltype(dim)::value;
+    k_gc_inverse<M><<<(nw + G - 1) / G, 64, 0, st>>>(n, nw, d + o_gc, d + o_gi, mode == 3 ? ld : nullptr, singular);
+    int part0 = 0;
+    for (int k0 = 0; k0 < nk; k0 += kmax) {
+      KsumArgs A{};
+      A.n = n;
+      A.nw = nw;
+      A.nk = std::min(kmax, nk - k0);
+      A.k0 = k0;
+      A.nk_all = nk;
+      A.chunk = chunk;
+      const int nkb = (A.nk + G - 1) / G;
+      A.nchunk = ((mode < 2 ? nw : nkb) + chunk - 1) / chunk;
+      A.part0 = part0;
+      A.parts = parts;
+      A.ginv = d + o_gi;
+      A.vk = d + o_vk;
+      A.out = d + o_out;
+      A.part = d + o_part;
+      k_vk<M><<<(A.nk + 7) / 8, 256, 0, st>>>(n, nterm, A.nk, d + o_v0, d + o_vt, d + o_nv, d + o_k + 3 * (size_t)k0, d + o_vk);
+      launch_ksum<M>(A, mode, (mode < 2 ? nkb : nw) * A.nchunk);
+      if (mode >= 2) part0 += A.nchunk;
+    }
+  });
+  if (mode == 2) k_ksum_reduce<<<nw * n, 64, 0, st>>>(parts, n, N, d + o_part, 1.0 / nk, d + o_out);
+  if (mode == 3) k_ksum_reduce<<<nw, 64, 0, st>>>(parts, 0, 0, d + o_part, 1.0 / nk, d + o_out);
+  QED_HIP(hipGetLastError());
+  QED_HIP(hipEventRecord(L->ev[1], st));
+  QED_HIP(hipMemcpyAsync(h, ld, (small ? n_down : (size_t)nw + 1) * 8, hipMemcpyDeviceToHost, st));
+  QED_HIP(hipStreamSynchronize(st));
+  int bad = 0;
+  std::memcpy(&bad, h + nw, sizeof(int));
+  if (bad) fail("cluster Green function is singular at a requested frequency");
+  if (small) {
+    std::memcpy(out, h + (o_out - o_ld), out_len * 8);
+    // log|det(V G - 1)| = log|det G| + log|det(G^-1 - V)|  (padding blocks contribute log 1 = 0)
+    if (mode == 3)
+      for (int w = 0; w < nw; ++w) out[w] += h[w];
+  } else {
+    std::vector<double> logdet(h, h + nw);
+    copy_out(reinterpret_cast<unsigned char*>(out), reinterpret_cast<const unsigned char*>(d + o_out), out_len * 8, L->pin,
+             2 * piece);
+    if (mode == 3)
+      for (int w = 0; w < nw; ++w) out[w] += logdet[w];
+  }
+  float ms = 0.0f;
+  QED_HIP(hipEventElapsedTime(&ms, L->ev[0], L->ev[1]));
+  if (mode < 3) last_ksum_ms() = ms;
+}
 
 }  // namespace
 
@@ -448,61 +738,7 @@ int qed_cpt_batch(int n, int nw, const double* Gc, const double* V0, int nterm, 
   return guard([&] {
     if (mode < 0 || mode > 2) fail("cpt_batch: mode must be 0, 1 or 2");
     if (n <= 0 || nw <= 0 || nk <= 0) return;
-    const int N = padded_dim(n);
-    std::vector<double> ginv = inverse_gc(Gc, nw, n, N, nullptr);
-    std::vector<double> v0 = pad_mats(V0, 1, n, N, false);
-    std::vector<double> vt = pad_mats(Vt, nterm, n, N, false);
-    DevBuf dgi = upload(ginv), dv0 = upload(v0), dvt = upload(vt.empty() ? std::vector<double>{0} : vt);
-    DevBuf dnv = up(nv, (size_t)3 * nterm), dk = up(k, (size_t)3 * nk);
-    KsumArgs A{};
-    A.n = N;
-    A.nw = nw;
-    A.nterm = nterm;
-    A.nk = nk;
-    A.mode = mode;
-    A.ginv = dgi.as<double>();
-    A.V0 = dv0.as<double>();
-    A.Vt = dvt.as<double>();
-    A.nv = dnv.as<double>();
-    A.k = dk.as<double>();
-    A.kchunk = (mode == 2) ? std::max(1, nk / 64) : 1;
-    const int ngk = (nk + A.kchunk - 1) / A.kchunk;
-    const int ngroups = nw * ngk;
-    DevBuf dout, dpart;
-    size_t out_len;
-    if (mode == 0) out_len = (size_t)nw * nk * N * N * 2;
-    else if (mode == 1) out_len = (size_t)nw * nk * 2;
-    else out_len = (size_t)nw * N * N * 2;
-    dout.alloc(out_len * 8);
-    if (mode == 2) dpart.alloc((size_t)ngroups * N * N * 2 * 8);
-    A.out = dout.as<double>();
-    A.part = dpart.as<double>();
-    KsumTimer timer;
-    ksum_dispatch(A, ngroups);
-    if (mode == 2) {
-      int len = N * N * 2;
-      k_ksum_reduce<<<(nw * len + 255) / 256, 256, 0, stream()>>>(nw, ngk, len, dpart.as<double>(), 1.0 / nk,
-                                                                 dout.as<double>());
-      QED_HIP(hipGetLastError());
-    }
-    timer.stop();
-    std::vector<double> h(out_len);
-    QED_HIP(hipMemcpyAsync(h.data(), dout.p, out_len * 8, hipMemcpyDeviceToHost, stream()));
-    QED_HIP(hipStreamSynchronize(stream()));
-    // unpad
-    if (mode == 1) {
-      std::copy(h.begin(), h.end(), out);
-      // padded identity blocks add (N - n) to the trace of M^-1
-      for (size_t q = 0; q < (size_t)nw * nk; ++q) out[2 * q] -= (N - n);
-    } else {
-      size_t cnt = (mode == 0) ? (size_t)nw * nk : (size_t)nw;
-      for (size_t c = 0; c < cnt; ++c)
-        for (int j = 0; j < n; ++j)
-          for (int i = 0; i < n; ++i) {
-            out[((c * n * n) + i + (size_t)j * n) * 2] = h[((c * N * N) + i + (size_t)j * N) * 2];
-            out[((c * n * n) + i + (size_t)j * n) * 2 + 1] = h[((c * N * N) + i + (size_t)j * N) * 2 + 1];
-          }
-    }
+    ksum(n, nw, Gc, V0, nterm, Vt, nv, nk, k, mode, out);
   });
 }
 
@@ -510,37 +746,7 @@ int qed_sef_batch(int n, int nw, const double* Gc, const double* V0, int nterm, 
                   const double* nv, int nk, const double* k, double* out) {
   return guard([&] {
     if (n <= 0 || nw <= 0 || nk <= 0) return;
-    const int N = padded_dim(n);
-    std::vector<double> logdetG;
-    std::vector<double> ginv = inverse_gc(Gc, nw, n, N, &logdetG);
-    std::vector<double> v0 = pad_mats(V0, 1, n, N, false);
-    std::vector<double> vt = pad_mats(Vt, nterm, n, N, false);
-    DevBuf dgi = upload(ginv), dv0 = upload(v0), dvt = upload(vt.empty() ? std::vector<double>{0} : vt);
-    DevBuf dnv = up(nv, (size_t)3 * nterm), dk = up(k, (size_t)3 * nk);
-    KsumArgs A{};
-    A.n = N;
-    A.nw = nw;
-    A.nterm = nterm;
-    A.nk = nk;
-    A.mode = 3;
-    A.ginv = dgi.as<double>();
-    A.V0 = dv0.as<double>();
-    A.Vt = dvt.as<double>();
-    A.nv = dnv.as<double>();
-    A.k = dk.as<double>();
-    A.kchunk = std::max(1, nk / 256);
-    const int ngk = (nk + A.kchunk - 1) / A.kchunk;
-    DevBuf dpart((size_t)nw * ngk * 8), dout((size_t)nw * 8);
-    A.part = dpart.as<double>();
-    A.out = dout.as<double>();
-    ksum_dispatch(A, nw * ngk);
-    k_ksum_reduce<<<(nw + 255) / 256, 256, 0, stream()>>>(nw, ngk, 1, dpart.as<double>(), 1.0 / nk,
-                                                         dout.as<double>());
-    QED_HIP(hipGetLastError());
-    QED_HIP(hipMemcpyAsync(out, dout.p, nw * 8, hipMemcpyDeviceToHost, stream()));
-    QED_HIP(hipStreamSynchronize(stream()));
-    // log|det(V G - 1)| = log|det G| + log|det(G^-1 - V)|  (padding blocks contribute log 1 = 0)
-    for (int w = 0; w < nw; ++w) out[w] += logdetG[w];
+    ksum(n, nw, Gc, V0, nterm, Vt, nv, nk, k, 3, out);
   });
 }
 

@@ -356,7 +356,7 @@ def cpt_batch(Geff, V0, nv, mats, k, mode="full"):
     if m == 0:
         return _from_cm(out, (nw, nk, n, n))
     if m == 1:
-        return out.view(np.complex128).reshape(nw, nk).copy()
+        return out.view(np.complex128).reshape(nw, nk)
     return _from_cm(out, (nw, n, n))
 
 
