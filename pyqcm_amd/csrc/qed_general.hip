@@ -97,9 +97,13 @@ __device__ __forceinline__ int between_parity(uint64_t s, uint64_t a, uint64_t b
 
 // y[I] += sum_J H[I, J] x[J]: every term applied to basis state I gives <J|T|I>, which is
 // H[I, J] since the term list is Hermitian and real
+template <int EP>
 __global__ __launch_bounds__(256) void k_hv_general(const uint64_t* __restrict__ st, uint32_t n, LocateTables loc,
                                                     const GTerm* __restrict__ terms, int nterms,
-                                                    const double* __restrict__ x, double* __restrict__ y) {
+                                                    const double* __restrict__ x, double* __restrict__ y, LzStep lz) {
+  double2 sc = make_double2(0.0, 0.0);
+  double dot = 0.0;
+  if constexpr (EP != 0) sc = lz_scalars(lz);
   for (uint32_t I = blockIdx.x * blockDim.x + threadIdx.x; I < n; I += gridDim.x * blockDim.x) {
     const uint64_t s = st[I];
     double diag = 0.0, acc = 0.0;
@@ -129,7 +133,13 @@ __global__ __launch_bounds__(256) void k_hv_general(const uint64_t* __restrict__
         acc += between_parity(s, t.mr, t.mc) ? v : -v;
       }
     }
-    y[I] += diag * x[I] + acc;
+    const double xi = x[I];
+    lz_update<EP>(lz, sc, diag * xi + acc, xi, y + I, EP == 2 ? lz.psi + I : nullptr, dot);
+  }
+  if constexpr (EP == 1) {
+    __shared__ double red[4];
+    dot = block_sum(dot, red);
+    if (threadIdx.x == 0) lz.pa[blockIdx.x] = dot;
   }
 }
 
@@ -178,15 +188,24 @@ uint32_t grid_of(uint64_t n) { return (uint32_t)std::min<uint64_t>(std::max<uint
 
 }  // namespace
 
-void hv_general(const qed_sector& s, const double* x, double* y, int variant) {
+template <int EP>
+static int launch_general(const qed_sector& s, const double* x, double* y, int variant, const LzStep& L) {
   auto T = std::static_pointer_cast<GeneralTables>(s.general);
-  const uint32_t n = (uint32_t)s.D;
-  if (n == 0) return;
+  const uint32_t n = (uint32_t)s.D, grid = grid_of(n);
+  if (n == 0) return 0;
   LocateTables loc = T->loc();
   if (variant == 0) loc.tabled = 0;  // the binary search (reference form of the lookup)
-  k_hv_general<<<grid_of(n), 256, 0, stream()>>>(T->states.as<uint64_t>(), n, loc, T->terms.as<GTerm>(), T->nterms,
-                                                 x, y);
+  k_hv_general<EP><<<grid, 256, 0, stream()>>>(T->states.as<uint64_t>(), n, loc, T->terms.as<GTerm>(), T->nterms, x, y, L);
   QED_HIP(hipGetLastError());
+  return (int)grid;
+}
+
+void hv_general(const qed_sector& s, const double* x, double* y, int variant) {
+  launch_general<0>(s, x, y, variant, LzStep{});
+}
+
+int hv_step_general(const qed_sector& s, const double* x, double* y, const LzStep& L) {
+  return L.kind == 1 ? launch_general<1>(s, x, y, -1, L) : launch_general<2>(s, x, y, -1, L);
 }
 
 void diag_general(const qed_sector& s, double* d) {

@@ -193,11 +193,14 @@ constexpr int kG = 8;
 
 // Row r of y += H x for one sector: the body shared by the single-sector kernel and the
 // batched multi-sector kernel. smem: nvu amplitudes, then (LDSX) the row X[r, :].
-template <int BS, bool LDSX>
+// EP: the epilogue of one Lanczos step (LzStep), 0 for y += H x.
+template <int BS, bool LDSX, int EP = 0>
 __device__ __forceinline__ void ell_row(const HvView& v, const uint32_t* __restrict__ up_ell,
                                         uint32_t Wu, const uint32_t* __restrict__ dn_ell,
                                         uint32_t Wd, const double* __restrict__ x,
-                                        double* __restrict__ y, uint32_t r, double* smem) {
+                                        double* __restrict__ y, uint32_t r, double* smem,
+                                        const LzStep* lz = nullptr, double2 sc = double2{0.0, 0.0},
+                                        double* dot = nullptr) {
   const uint32_t du = v.du;
   const uint32_t nvu = v.up_nvals;
   double* vals_s = smem;
@@ -235,7 +238,11 @@ __device__ __forceinline__ void ell_row(const HvView& v, const uint32_t* __restr
 #pragma unroll
       for (int q = 0; q < kG; ++q) acc2 += v.dn_vals[e[q] >> kTargetBits] * xv[q];
     }
-    yr[c] += acc + acc2;
+    if constexpr (EP == 0) {
+      yr[c] += acc + acc2;
+    } else {
+      lz_update<EP>(*lz, sc, acc + acc2, xsrc[c], yr + c, EP == 2 ? lz->psi + (uint64_t)r * du + c : nullptr, *dot);
+    }
   }
 }
 
@@ -243,13 +250,27 @@ __device__ __forceinline__ void ell_row(const HvView& v, const uint32_t* __restr
 // from the row staged in LDS. Down-spin hops: the row's neighbour list is uniform across
 // the workgroup; 8 neighbour rows are requested before any of them is consumed so that
 // each wave keeps 8 row loads in flight.
-template <int BS, bool LDSX>
+template <int BS, bool LDSX, int EP = 0>
 __global__ __launch_bounds__(BS) void k_hv_ell(HvView v, const uint32_t* __restrict__ up_ell,
                                                uint32_t Wu, const uint32_t* __restrict__ dn_ell,
                                                uint32_t Wd, const double* __restrict__ x,
-                                               double* __restrict__ y) {
+                                               double* __restrict__ y, LzStep lz = LzStep{}) {
   extern __shared__ double smem[];
-  ell_row<BS, LDSX>(v, up_ell, Wu, dn_ell, Wd, x, y, blockIdx.x, smem);
+  if constexpr (EP == 0) {
+    ell_row<BS, LDSX>(v, up_ell, Wu, dn_ell, Wd, x, y, blockIdx.x, smem);
+  } else {
+    __shared__ double red[BS / 64];
+    const double2 sc = lz_scalars(lz);
+    double dot = 0.0;
+    for (uint32_t r = blockIdx.x; r < v.dd; r += gridDim.x) {
+      ell_row<BS, LDSX, EP>(v, up_ell, Wu, dn_ell, Wd, x, y, r, smem, &lz, sc, &dot);
+      __syncthreads();
+    }
+    if (EP == 1) {
+      dot = block_sum(dot, red);
+      if (threadIdx.x == 0) lz.pa[blockIdx.x] = dot;
+    }
+  }
 }
 
 // Batched H.v over many sectors ("jobs") in one persistent launch: the rows of all jobs
@@ -410,17 +431,14 @@ __global__ __launch_bounds__(256) void k_hv_tileB_batch(const HvJob* __restrict_
 
 // Same product, two adjacent columns per thread: 16-byte loads of the down-spin neighbour
 // rows and of the ELL entry pairs (needs an even up dimension).
-// LZ (one Lanczos step fused into the product): y <- lz[0] (H x) + lz[1] y, and the
-// workgroup's part of <x, y_new> in lz_part[row] (the scalars are device values, so that
-// a step needs no host round trip before it starts).
-template <int BS, bool DOWN = true, bool LZ = false>
+// EP: the epilogue of one Lanczos step (LzStep), 0 for y += H x.
+template <int BS, int EP = 0>
 __global__ __launch_bounds__(BS) void k_hv_ell2(HvView v, const uint32_t* __restrict__ up_ell,
                                                 uint32_t Wu, const uint32_t* __restrict__ dn_ell,
                                                 uint32_t Wd, const double* __restrict__ x,
                                                 double* __restrict__ y,
                                                 const uint32_t* __restrict__ order = nullptr,
-                                                const double* __restrict__ lz = nullptr,
-                                                double* __restrict__ lz_part = nullptr) {
+                                                LzStep lz = LzStep{}) {
   extern __shared__ double smem[];
   const uint32_t du = v.du;
   const uint32_t nvu = v.up_nvals;
@@ -440,6 +458,8 @@ __global__ __launch_bounds__(BS) void k_hv_ell2(HvView v, const uint32_t* __rest
   const uint32_t* dl = dn_ell + (uint64_t)r * Wd;
   double2* yr = reinterpret_cast<double2*>(y + (uint64_t)r * du);
   double dotp = 0.0;
+  double2 sc = make_double2(0.0, 0.0);
+  if constexpr (EP != 0) sc = lz_scalars(lz);
   for (uint32_t c2 = threadIdx.x; c2 < dh; c2 += BS) {
     const uint32_t c = 2 * c2;
     double a0 = (dg + v.diag_up[c] + interaction(v, v.bup[c], sd)) * xs[c];
@@ -456,7 +476,7 @@ __global__ __launch_bounds__(BS) void k_hv_ell2(HvView v, const uint32_t* __rest
       }
     }
     double b0 = 0.0, b1 = 0.0;
-    for (uint32_t g = 0; DOWN && g < dgroups; g += kG) {
+    for (uint32_t g = 0; g < dgroups; g += kG) {
       uint32_t e[kG];
       double2 xv[kG];
 #pragma unroll
@@ -472,19 +492,16 @@ __global__ __launch_bounds__(BS) void k_hv_ell2(HvView v, const uint32_t* __rest
       }
     }
     double2 yo = yr[c2];
-    if (LZ) {
-      yo.x = lz[0] * (a0 + b0) + lz[1] * yo.x;
-      yo.y = lz[0] * (a1 + b1) + lz[1] * yo.y;
-      dotp += xs[c] * yo.x + xs[c + 1] * yo.y;
-    } else {
-      yo.x += a0 + b0;
-      yo.y += a1 + b1;
-    }
+    double2 po = make_double2(0.0, 0.0);
+    if constexpr (EP == 2) po = reinterpret_cast<double2*>(lz.psi + (uint64_t)r * du)[c2];
+    lz_update<EP>(lz, sc, a0 + b0, xs[c], &yo.x, &po.x, dotp);
+    lz_update<EP>(lz, sc, a1 + b1, xs[c + 1], &yo.y, &po.y, dotp);
     yr[c2] = yo;
+    if constexpr (EP == 2) reinterpret_cast<double2*>(lz.psi + (uint64_t)r * du)[c2] = po;
   }
-  if (LZ) {
+  if constexpr (EP == 1) {
     const double t = block_sum(dotp, smem + ((nvu + 1u) & ~1u) + du);
-    if (threadIdx.x == 0) lz_part[r] = t;
+    if (threadIdx.x == 0) lz.pa[blockIdx.x] = t;
   }
 }
 
@@ -698,18 +715,11 @@ static void set_lds_attributes() {
                               hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
     (void)hipFuncSetAttribute((const void*)k_hv_rows<256, false, true>,
                               hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-    (void)hipFuncSetAttribute((const void*)k_hv_ell<1024, true>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-    (void)hipFuncSetAttribute((const void*)k_hv_ell<256, true>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-    (void)hipFuncSetAttribute((const void*)k_hv_ell2<512>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-    (void)hipFuncSetAttribute((const void*)k_hv_ell2<512, false>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-    (void)hipFuncSetAttribute((const void*)k_hv_ell2<512, true, true>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-
-
+    for (const void* f : {(const void*)k_hv_ell<1024, true>, (const void*)k_hv_ell<1024, true, 1>,
+                          (const void*)k_hv_ell<1024, true, 2>, (const void*)k_hv_ell<256, true>,
+                          (const void*)k_hv_ell<256, true, 1>, (const void*)k_hv_ell<256, true, 2>,
+                          (const void*)k_hv_ell2<512>, (const void*)k_hv_ell2<512, 1>, (const void*)k_hv_ell2<512, 2>})
+      (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
   });
 }
 
@@ -782,7 +792,6 @@ void hv(const qed_sector& s, const double* x, double* y, int variant) {
     return;
   }
   set_lds_attributes();
-  if (variant < 0) variant = s.hv_variant;
   if (variant < 0) variant = 12;
   if (variant >= 20 && variant <= 22) {
     // split-halves passes (20 both; 21 row pass only, 22 tile pass only: timing splits)
@@ -857,20 +866,44 @@ void hv(const qed_sector& s, const double* x, double* y, int variant) {
 }
 
 
-bool hv_lanczos(const qed_sector& s, const double* x, double* y, const double* lz, double* lz_part) {
-  if (s.D == 0 || s.hv_variant >= 0 || !s.factorized()) return false;
-  // the default row kernel (tiled row order); the LZ epilogue needs LDS for the row, the
-  // amplitudes and eight doubles of reduction scratch
-  const size_t lds2 = ((size_t)s.du + s.up_nvals + 1 + 16) * sizeof(double);
-  if (s.du % 2 != 0 || s.du < 4096 || lds2 > lds_budget()) return false;
+template <int BS, bool LDSX>
+static void launch_ell_step(const qed_sector& s, const HvView& v, uint32_t grid, size_t sh, const double* x, double* y,
+                            const LzStep& L) {
+  const uint32_t* ue = s.up_ell.as<uint32_t>();
+  const uint32_t* de = s.dn_ell.as<uint32_t>();
+  if (L.kind == 1) k_hv_ell<BS, LDSX, 1><<<grid, BS, sh, stream()>>>(v, ue, s.up_w, de, s.dn_w, x, y, L);
+  else k_hv_ell<BS, LDSX, 2><<<grid, BS, sh, stream()>>>(v, ue, s.up_w, de, s.dn_w, x, y, L);
+}
+
+int hv_step(const qed_sector& s, const double* x, double* y, const LzStep& L) {
+  if (s.D == 0) return 0;
+  if (s.mixed) return hv_step_mixed(s, x, y, L);
+  if (s.general) return hv_step_general(s, x, y, L);
   set_lds_attributes();
-  ensure_row_order(s);
-  HvView v = view(s);
-  k_hv_ell2<512, true, true><<<s.dd, 512, lds2, stream()>>>(v, s.up_ell.as<uint32_t>(), s.up_w,
-                                                          s.dn_ell.as<uint32_t>(), s.dn_w, x, y,
-                                                          s.row_order.as<uint32_t>(), lz, lz_part);
+  const HvView v = view(s);
+  // the kernels of hv(); the reduction needs eight more doubles of LDS
+  const size_t lds2 = ((size_t)s.du + s.up_nvals + 1 + 16) * sizeof(double);
+  const uint32_t grid = std::min(s.dd, kLzRows);
+  if (s.du % 2 == 0 && s.du >= 4096 && lds2 <= lds_budget() && grid == s.dd) {
+    ensure_row_order(s);
+    const uint32_t* ue = s.up_ell.as<uint32_t>();
+    const uint32_t* de = s.dn_ell.as<uint32_t>();
+    const uint32_t* ord = s.row_order.as<uint32_t>();
+    if (L.kind == 1) k_hv_ell2<512, 1><<<grid, 512, lds2, stream()>>>(v, ue, s.up_w, de, s.dn_w, x, y, ord, L);
+    else k_hv_ell2<512, 2><<<grid, 512, lds2, stream()>>>(v, ue, s.up_w, de, s.dn_w, x, y, ord, L);
+  } else {
+    const size_t lds = ((size_t)s.du + s.up_nvals) * sizeof(double);
+    const bool fits = lds + 256 <= lds_budget();
+    const size_t sh = fits ? lds : s.up_nvals * sizeof(double);
+    if (s.du >= 4096) {
+      if (fits) launch_ell_step<1024, true>(s, v, grid, sh, x, y, L);
+      else launch_ell_step<1024, false>(s, v, grid, sh, x, y, L);
+    } else {
+      launch_ell_step<256, true>(s, v, grid, sh, x, y, L);
+    }
+  }
   QED_HIP(hipGetLastError());
-  return true;
+  return (int)grid;
 }
 
 // ---- batched launch with autotuned (block size, grid) ------------------------------------

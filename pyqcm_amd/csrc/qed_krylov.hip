@@ -116,65 +116,56 @@ __global__ __launch_bounds__(RB) void k_axpy_nrm(double a, const double* __restr
   if (threadIdx.x == 0) part[blockIdx.x] = s;
 }
 
-// ---- fused Lanczos step (device scalars) ---------------------------------------------
-// sc: [0] 1/beta_{k-1}, [1] -beta_{k-1}/beta_{k-2} (the product's scalars), [2] alpha_k,
-// [3] beta_k, [4] the axpy coefficient -alpha_k / beta_{k-1}, [5] beta_{k-1}
-// alpha_k = sc[0] * sum(part); the axpy coefficient follows
-__global__ void k_lzf_alpha(const double* __restrict__ part, int nb, double* __restrict__ sc) {
+// ---- Lanczos step (device scalars, LzStep) ----------------------------------------------
+// w_{k+1} = y - alpha_k v_k with alpha_k = <w_k, y> / beta_{k-1}; the parts of |w_{k+1}|^2.
+// Bound by its 24 bytes per element; each wave adds up the product's parts by itself, so
+// that a step is two launches and no scalar kernel (at most kLzParts parts).
+__global__ __launch_bounds__(RB) void k_lz_axpy_nrm(LzStep lz, int na, double* __restrict__ alpha, double* __restrict__ beta,
+                                                    const double* __restrict__ x, double* __restrict__ y, uint64_t n,
+                                                    double* __restrict__ part) {
   __shared__ double sh[RB / 64];
-  double s = 0.0;
-  for (int i = threadIdx.x; i < nb; i += RB) s += part[i];
-  s = block_sum(s, sh);
-  if (threadIdx.x == 0) {
-    const double a = s * sc[0];
-    sc[2] = a;
-    sc[4] = -a * sc[0];
+  const double b = lz.k == 0 ? 1.0 : sqrt(lz_sum(lz.pb, lz.nb));
+  const double inv = lz_inv(b);
+  const double al = lz_sum(lz.pa, na) * inv;
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    alpha[lz.k % lz.ring] = al;
+    if (lz.k > 0) beta[(lz.k - 1) % lz.ring] = b;
   }
-}
-
-// beta_k = sqrt(sum(part)); the next product's scalars
-__global__ void k_lzf_beta(const double* __restrict__ part, int nb, double* __restrict__ sc) {
-  __shared__ double sh[RB / 64];
-  double s = 0.0;
-  for (int i = threadIdx.x; i < nb; i += RB) s += part[i];
-  s = block_sum(s, sh);
-  if (threadIdx.x == 0) {
-    const double b = sqrt(s);
-    sc[3] = b;
-    sc[1] = -b * sc[0];  // -beta_k / beta_{k-1}
-    sc[0] = b != 0.0 ? 1.0 / b : 0.0;
-    sc[5] = b;
-  }
-}
-
-// y += sc[4] x, partial sums of y^2
-__global__ __launch_bounds__(RB) void k_lzf_axpy_nrm(const double* __restrict__ sc, const double* __restrict__ x,
-                                                     double* __restrict__ y, uint64_t n,
-                                                     double* __restrict__ part) {
-  __shared__ double sh[RB / 64];
-  const double a = sc[4];
+  const double a = -al * inv;
   double acc = 0.0;
-  for (uint64_t i = (uint64_t)blockIdx.x * RB + threadIdx.x; i < n; i += (uint64_t)gridDim.x * RB) {
-    double v = y[i] + a * x[i];
-    y[i] = v;
+  const uint64_t n2 = n / 2;
+  double2* __restrict__ y2 = reinterpret_cast<double2*>(y);
+  const double2* __restrict__ x2 = reinterpret_cast<const double2*>(x);
+  for (uint64_t i = (uint64_t)blockIdx.x * RB + threadIdx.x; i < n2; i += (uint64_t)gridDim.x * RB) {
+    const double2 u = x2[i];
+    double2 v = y2[i];
+    v.x += a * u.x;
+    v.y += a * u.y;
+    y2[i] = v;
+    acc += v.x * v.x + v.y * v.y;
+  }
+  if (n % 2 && blockIdx.x == 0 && threadIdx.x == 0) {
+    const double v = y[n - 1] + a * x[n - 1];
+    y[n - 1] = v;
     acc += v * v;
   }
-  double s = block_sum(acc, sh);
+  const double s = block_sum(acc, sh);
   if (threadIdx.x == 0) part[blockIdx.x] = s;
 }
 
-// eigenvector replay step: q -= a r; (r, q) <- (q / b, -b r); psi += c r_new
-__global__ void k_replay(double a, double b, double c, double* __restrict__ r,
-                         double* __restrict__ q, double* __restrict__ psi, uint64_t n) {
-  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (uint64_t)gridDim.x * blockDim.x) {
-    double rv = r[i];
-    double qv = q[i] - a * rv;
-    double rn = qv / b;
-    r[i] = rn;
-    q[i] = -b * rv;
-    psi[i] += c * rn;
-  }
+// p[0] = sum of n values (more than kLzParts)
+__global__ __launch_bounds__(1024) void k_lz_fold(double* __restrict__ p, int n) {
+  __shared__ double sh[16];
+  double s = 0.0;
+  for (int i = threadIdx.x; i < n; i += 1024) s += p[i];
+  s = block_sum(s, sh);
+  if (threadIdx.x == 0) p[0] = s;
+}
+
+// beta_k of the last step of a chunk
+__global__ __launch_bounds__(64) void k_lz_last(const double* __restrict__ pb, int nb, double* __restrict__ beta) {
+  const double b = sqrt(lz_sum(pb, nb));
+  if (threadIdx.x == 0) *beta = b;
 }
 
 // continued-fraction Lanczos step: (psi, q) <- (q / b, -b psi)
@@ -227,67 +218,172 @@ uint32_t stream_blocks(uint64_t n) {
 
 }  // namespace
 
-// lowest eigenvalue of the Lanczos tridiagonal and its normalized eigenvector
-// (QL eigenvalues, then inverse iteration for the vector)
-void tridiag_lowest(const std::vector<double>& a, const std::vector<double>& b, double* e0,
-                    std::vector<double>& vec) {
-  int n = (int)a.size();
+namespace {
+
+// Normalized eigenvector of the lowest eigenvalue lam of the Lanczos tridiagonal: three
+// steps of inverse iteration on (T - lam) with partial pivoting, one factorization
+void tridiag_vector(const std::vector<double>& a, const std::vector<double>& b, double lam, std::vector<double>& vec) {
+  const int n = (int)a.size();
   vec.assign(n, 1.0);
-  if (n == 1) {
-    *e0 = a[0];
-    return;
-  }
-  std::vector<double> d(a), e(b.begin(), b.begin() + (n - 1));
-  tridiag_eigen(n, d.data(), e.data(), nullptr);
-  double lam = d[0];
-  *e0 = lam;
-  // inverse iteration on (T - lam) with partial pivoting
   double scale = 0.0;
   for (int i = 0; i < n; ++i) scale = std::max(scale, std::fabs(a[i]) + (i < n - 1 ? std::fabs(b[i]) : 0.0));
-  double shift = lam - 1e-14 * std::max(scale, 1.0);
-  for (int it = 0; it < 3; ++it) {
-    // solve (T - shift I) x = vec; Gaussian elimination on the tridiagonal with pivoting
-    std::vector<double> dl(n - 1), dm(n), du(n - 1), du2(n, 0.0), rhs(vec);
-    for (int i = 0; i < n; ++i) dm[i] = a[i] - shift;
-    for (int i = 0; i < n - 1; ++i) dl[i] = du[i] = b[i];
-    std::vector<int> swapped(n, 0);
-    for (int i = 0; i < n - 1; ++i) {
-      if (std::fabs(dm[i]) >= std::fabs(dl[i])) {
-        if (dm[i] == 0.0) dm[i] = 1e-300;
-        double f = dl[i] / dm[i];
-        dm[i + 1] -= f * du[i];
-        rhs[i + 1] -= f * rhs[i];
-        if (i < n - 2) du2[i] = 0.0;
-      } else {
-        double f = dm[i] / dl[i];
-        dm[i] = dl[i];
-        double t = dm[i + 1];
-        dm[i + 1] = du[i] - f * t;
-        if (i < n - 2) {
-          du2[i] = du[i + 1];
-          du[i + 1] = -f * du2[i];
-        }
-        du[i] = t;
-        std::swap(rhs[i], rhs[i + 1]);
-        rhs[i + 1] -= f * rhs[i];
+  const double shift = lam - 1e-14 * std::max(scale, 1.0);
+  static thread_local std::vector<double> dm, du, du2, f;
+  static thread_local std::vector<char> swapped;
+  dm.resize(n);
+  du.assign(b.begin(), b.begin() + (n - 1));
+  du2.assign(n, 0.0);
+  f.resize(n);
+  swapped.assign(n, 0);
+  for (int i = 0; i < n; ++i) dm[i] = a[i] - shift;
+  for (int i = 0; i < n - 1; ++i) {
+    const double dl = b[i];
+    if (std::fabs(dm[i]) >= std::fabs(dl)) {
+      if (dm[i] == 0.0) dm[i] = 1e-300;
+      f[i] = dl / dm[i];
+      dm[i + 1] -= f[i] * du[i];
+    } else {
+      swapped[i] = 1;
+      f[i] = dm[i] / dl;
+      dm[i] = dl;
+      const double t = dm[i + 1];
+      dm[i + 1] = du[i] - f[i] * t;
+      if (i < n - 2) {
+        du2[i] = du[i + 1];
+        du[i + 1] = -f[i] * du2[i];
       }
+      du[i] = t;
     }
-    if (dm[n - 1] == 0.0) dm[n - 1] = 1e-300;
-    std::vector<double> x(n);
-    x[n - 1] = rhs[n - 1] / dm[n - 1];
-    if (n >= 2) x[n - 2] = (rhs[n - 2] - du[n - 2] * x[n - 1]) / dm[n - 2];
-    for (int i = n - 3; i >= 0; --i) x[i] = (rhs[i] - du[i] * x[i + 1] - du2[i] * x[i + 2]) / dm[i];
+  }
+  if (dm[n - 1] == 0.0) dm[n - 1] = 1e-300;
+  for (int it = 0; it < 3; ++it) {
+    for (int i = 0; i < n - 1; ++i) {
+      if (swapped[i]) std::swap(vec[i], vec[i + 1]);
+      vec[i + 1] -= f[i] * vec[i];
+    }
+    vec[n - 1] /= dm[n - 1];
+    if (n >= 2) vec[n - 2] = (vec[n - 2] - du[n - 2] * vec[n - 1]) / dm[n - 2];
+    for (int i = n - 3; i >= 0; --i) vec[i] = (vec[i] - du[i] * vec[i + 1] - du2[i] * vec[i + 2]) / dm[i];
     double nrm = 0.0;
-    for (double v : x) nrm += v * v;
+    for (double v : vec) nrm += v * v;
     nrm = std::sqrt(nrm);
-    for (int i = 0; i < n; ++i) vec[i] = x[i] / nrm;
+    for (double& v : vec) v /= nrm;
   }
   // sign convention: first component positive (sign does not affect the Ritz residual)
   if (vec[0] < 0)
     for (double& v : vec) v = -v;
 }
 
+}  // namespace
+
+// lowest eigenvalue of the Lanczos tridiagonal and its normalized eigenvector
+// (QL eigenvalues, then inverse iteration for the vector)
+void tridiag_lowest(const std::vector<double>& a, const std::vector<double>& b, double* e0,
+                    std::vector<double>& vec) {
+  const int n = (int)a.size();
+  if (n == 1) {
+    vec.assign(1, 1.0);
+    *e0 = a[0];
+    return;
+  }
+  std::vector<double> d(a), e(b.begin(), b.begin() + (n - 1));
+  tridiag_eigen(n, d.data(), e.data(), nullptr);
+  *e0 = d[0];
+  tridiag_vector(a, b, d[0], vec);
+}
+
 namespace {
+
+// The same for a matrix that grows by a row per call, started from the pair (lam, vec) of
+// the last call: Rayleigh quotient iteration, accepted when it is stationary and a Sturm
+// count finds no eigenvalue below. O(n) where the QL sweep is O(n^2), which took most of a
+// small ground state (177 steps: 40 of 60 ms).
+void tridiag_lowest_next(const std::vector<double>& a, const std::vector<double>& b, double* lam,
+                         std::vector<double>& vec) {
+  const int n = (int)a.size();
+  if (n <= 16 || (int)vec.size() != n - 1) {
+    tridiag_lowest(a, b, lam, vec);
+    return;
+  }
+  static thread_local std::vector<double> x;
+  x.assign(vec.begin(), vec.end());
+  x.push_back(0.0);
+  double scale = 1.0;
+  for (int i = 0; i < n; ++i) scale = std::max(scale, std::fabs(a[i]) + std::fabs(b[i]));
+  // the new row couples to the last component only: start from the first-order update
+  x[n - 1] = b[n - 2] * x[n - 2] / (*lam - a[n - 1] != 0.0 ? *lam - a[n - 1] : scale);
+  double rho = 0.0;
+  bool ok = false;
+  for (int it = 0; it < 6; ++it) {
+    double nn = 0.0, num = 0.0;
+    for (int i = 0; i < n; ++i) nn += x[i] * x[i];
+    for (int i = 0; i < n; ++i) num += x[i] * (a[i] * x[i] + (i + 1 < n ? 2.0 * b[i] * x[i + 1] : 0.0));
+    rho = num / nn;
+    double res = 0.0;
+    for (int i = 0; i < n; ++i) {
+      const double r = (a[i] - rho) * x[i] + (i > 0 ? b[i - 1] * x[i - 1] : 0.0) + (i + 1 < n ? b[i] * x[i + 1] : 0.0);
+      res += r * r;
+    }
+    // the quotient's error is of second order in the residual
+    if (!(res <= nn * scale * scale)) break;
+    if (res <= 1e-20 * nn * scale * scale) {
+      ok = true;
+      break;
+    }
+    static thread_local std::vector<double> next;
+    tridiag_vector(a, b, rho, next);
+    x = next;
+  }
+  if (ok) {  // negative pivots of T - (rho - delta): the eigenvalues below
+    const double shift = rho - 1e-12 * scale;
+    double q = a[0] - shift;
+    for (int i = 0; ok && i < n; ++i) {
+      if (i > 0) q = a[i] - shift - b[i - 1] * b[i - 1] / q;
+      if (!(q > 0.0)) ok = false;
+    }
+  }
+  if (!ok) {
+    tridiag_lowest(a, b, lam, vec);
+    return;
+  }
+  *lam = rho;
+  tridiag_vector(a, b, rho, vec);
+}
+
+// Pinned host memory for the scalars of a Lanczos run, taken from a small pool (one per
+// concurrent run) and given back.
+class PinnedScalars {
+ public:
+  static constexpr size_t kDoubles = 4 * kLzRing;
+  PinnedScalars() {
+    std::lock_guard<std::mutex> lk(mutex());
+    if (!idle().empty()) {
+      p_ = idle().back();
+      idle().pop_back();
+    } else {
+      QED_HIP(hipHostMalloc((void**)&p_, kDoubles * sizeof(double), hipHostMallocDefault));
+    }
+  }
+  PinnedScalars(const PinnedScalars&) = delete;
+  ~PinnedScalars() {
+    (void)hipStreamSynchronize(stream());
+    std::lock_guard<std::mutex> lk(mutex());
+    if (idle().size() < 8) idle().push_back(p_);
+    else (void)hipHostFree(p_);
+  }
+  double* get() { return p_; }
+
+ private:
+  static std::mutex& mutex() {
+    static std::mutex m;
+    return m;
+  }
+  static std::vector<double*>& idle() {  // never destroyed: the runtime may be gone by then
+    static auto* v = new std::vector<double*>();
+    return *v;
+  }
+  double* p_ = nullptr;
+};
 
 }  // namespace
 
@@ -296,7 +392,7 @@ std::recursive_mutex& lib_mutex() {
   return m;
 }
 
-void multi_dot(const double* x, const double* const* ys, int m, uint64_t n, double* out, double* work) {
+void multi_dot(const double* x, const double* const* ys, int m, uint64_t n, double* out) {
   if (m > kMaxMulti) fail("multi_dot: too many vectors");
   if (m == 0) return;
   if (n == 0) {
@@ -306,7 +402,7 @@ void multi_dot(const double* x, const double* const* ys, int m, uint64_t n, doub
   PtrList l{};
   for (int k = 0; k < m; ++k) l.p[k] = ys[k];
   uint32_t nb = red_blocks(n);
-  double* part = work ? work : red_scratch().as<double>();
+  double* part = red_scratch().as<double>();
   double* fin = part + (size_t)kMaxBlocks * kMaxMulti;
   k_multi_dot<<<nb, RB, 0, stream()>>>(x, l, m, n, part);
   k_finish<<<1, RB, 0, stream()>>>(part, nb, m, fin);
@@ -314,9 +410,9 @@ void multi_dot(const double* x, const double* const* ys, int m, uint64_t n, doub
   QED_HIP(hipStreamSynchronize(stream()));
 }
 
-double dot(const double* x, const double* y, uint64_t n, double* work) {
+double dot(const double* x, const double* y, uint64_t n) {
   double r;
-  multi_dot(x, &y, 1, n, &r, work);
+  multi_dot(x, &y, 1, n, &r);
   return r;
 }
 
@@ -332,9 +428,9 @@ void scal2(double ar, double* r, double aq, double* q, uint64_t n) {
   if (n) k_scal2<<<stream_blocks(n), 256, 0, stream()>>>(ar, r, aq, q, n);
 }
 
-double axpy_nrm2(double a, const double* x, double* y, uint64_t n, double* work) {
+double axpy_nrm2(double a, const double* x, double* y, uint64_t n) {
   uint32_t nb = red_blocks(n);
-  double* part = work ? work : red_scratch().as<double>();
+  double* part = red_scratch().as<double>();
   double* fin = part + (size_t)kMaxBlocks * kMaxMulti;
   k_axpy_nrm<<<nb, RB, 0, stream()>>>(a, x, y, n, part);
   k_finish<<<1, RB, 0, stream()>>>(part, nb, 1, fin);
@@ -366,119 +462,148 @@ void multi_axpy_rev(const double* c, const double* x, double* const* ys, int m, 
   QED_HIP(hipStreamSynchronize(stream()));
 }
 
-// The eigenvalue pass of the Lanczos ground state, one fused step per iteration where the
-// sector takes the fused product: with w_k = beta_{k-1} v_k kept unnormalized,
-//   y = H v_k - beta_{k-1} v_{k-1} = (H w_k) / beta_{k-1} - (beta_{k-1} / beta_{k-2}) w_{k-1}
-// is one pass of the product kernel (which also sums <w_k, y>), and
-//   w_{k+1} = y - (alpha_k / beta_{k-1}) w_k,  beta_k = |w_{k+1}|
-// one more streaming pass: 24 D bytes beyond the product instead of 72 D for the separate
-// scale, dot and axpy passes, and one scalar download per step.
-bool lanczos_eigen_fused(qed_sector& s, double accur, int max_iter, const double* psi, std::vector<double>& alpha,
-                         std::vector<double>& beta, std::vector<double>& evec, double& e0,
-                         const LanczosWork* ws) {
-  const uint64_t n = s.D;
-  if (ws && s.dd > kFusedPartDoubles) return false;
-  DevBuf rb, qb, sc, part;
-  double *r, *q, *scd, *pd;
-  if (ws) {
-    r = ws->r;
-    q = ws->q;
-    scd = ws->sc;
-    pd = ws->part;
-  } else {
-    rb.alloc(n * 8);
-    qb.alloc(n * 8);
-    sc.alloc(8 * sizeof(double));
-    part.alloc((size_t)std::max<uint32_t>(s.dd, kMaxBlocks) * 8);
-    r = rb.as<double>();
-    q = qb.as<double>();
-    scd = sc.as<double>();
-    pd = part.as<double>();
-  }
-  QED_HIP(hipMemcpyAsync(r, psi, n * 8, hipMemcpyDeviceToDevice, stream()));
-  if (ws) k_zero<<<stream_blocks(n), 256, 0, stream()>>>(q, n);
-  else QED_HIP(hipMemsetAsync(q, 0, n * 8, stream()));
-  const double init[8] = {1.0, 0.0, 0.0, 0.0, 0.0, 1.0, 0.0, 0.0};
-  QED_HIP(hipMemcpyAsync(scd, init, sizeof(init), hipMemcpyHostToDevice, stream()));
-  double ritz = 2.0 * accur;
-  double ab[2];
-  const uint32_t nb = red_blocks(n);
-  while (ritz > accur) {
-    if (!hv_lanczos(s, r, q, scd, pd)) {
-      if (alpha.empty()) return false;
-      fail("fused Lanczos product unavailable after the first step");
-    }
-    k_lzf_alpha<<<1, RB, 0, stream()>>>(pd, (int)s.dd, scd);
-    k_lzf_axpy_nrm<<<nb, RB, 0, stream()>>>(scd, r, q, n, pd);
-    k_lzf_beta<<<1, RB, 0, stream()>>>(pd, (int)nb, scd);
-    QED_HIP(hipMemcpyAsync(ab, scd + 2, 2 * sizeof(double), hipMemcpyDeviceToHost, stream()));
-    QED_HIP(hipStreamSynchronize(stream()));
-    std::swap(r, q);
-    alpha.push_back(ab[0]);
-    beta.push_back(ab[1]);
-    tridiag_lowest(alpha, beta, &e0, evec);
-    ritz = std::fabs(evec.back() * beta.back());
-    if ((int)alpha.size() > max_iter)
-      fail("Lanczos procedure exceeded " + std::to_string(max_iter) + " iterations");
-  }
-  return true;
-}
+namespace {
 
-void lanczos_gs(qed_sector& s, double accur, int max_iter, double* psi, double* E0, int* niter,
-                std::vector<double>* alpha_out, std::vector<double>* beta_out, const LanczosWork* ws) {
-  const uint64_t n = s.D;
-  // with a workspace: the two recurrence vectors and the reduction partials are the
-  // caller's, zero fills are kernels, and the product is one that allocates nothing (the
-  // split-halves form builds its tables on first use, so the default row kernel instead)
-  const int var = ws && s.hv_variant >= 20 ? 12 : -1;
-  std::vector<double> alpha, beta, evec;
-  double e0 = 0.0;
-  DevBuf rb, qb;
-  double *r = nullptr, *q = nullptr;
-  auto vectors = [&] {
+// The device side of a Lanczos run: the two vectors, the parts of the two reductions and
+// the last kLzRing alpha and beta, in the caller's memory where given.
+struct LanczosRun {
+  const qed_sector& s;
+  uint64_t n;
+  DevBuf rb, qb, wb;
+  double *r, *q, *pa, *pb[2], *alpha, *beta;
+  int nb = 0;  // parts of the last |w|^2
+  int k = 0;   // steps done
+
+  LanczosRun(const qed_sector& sec, const LanczosWork* ws) : s(sec), n(sec.D) {
     if (ws) {
       r = ws->r;
       q = ws->q;
-    } else if (!rb.p) {
+      pa = ws->red;
+    } else {
       rb.alloc(n * 8);
       qb.alloc(n * 8);
+      wb.alloc(kLzWork * 8);
       r = rb.as<double>();
       q = qb.as<double>();
+      pa = wb.as<double>();
     }
+    pb[0] = pa + kLzRows;
+    pb[1] = pb[0] + kLzParts;
+    alpha = pb[1] + kLzParts;
+    beta = alpha + kLzRing;
+  }
+  void start(const double* psi) {
+    if (n) {
+      QED_HIP(hipMemcpyAsync(r, psi, n * 8, hipMemcpyDeviceToDevice, stream()));
+      k_zero<<<stream_blocks(n), 256, 0, stream()>>>(q, n);
+    }
+    k = 0;
+  }
+  // one step: w in r, the next one in r afterwards
+  void step() {
+    LzStep L;
+    L.kind = 1;
+    L.k = k;
+    L.pb = pb[(k + 1) & 1];
+    L.nb = nb;
+    L.beta = beta;
+    L.ring = kLzRing;
+    L.pa = pa;
+    int na = hv_step(s, r, q, L);
+    if (na > kLzParts) {
+      k_lz_fold<<<1, 1024, 0, stream()>>>(pa, na);
+      na = 1;
+    }
+    const uint32_t grid = (uint32_t)std::min<uint64_t>(std::max<uint64_t>((n + RB * 8 - 1) / (RB * 8), 1), kLzParts);
+    k_lz_axpy_nrm<<<grid, RB, 0, stream()>>>(L, na, alpha, beta, r, q, n, pb[k & 1]);
+    nb = (int)grid;
+    std::swap(r, q);
+    ++k;
+  }
+  // the alpha and beta of the last kLzRing steps into host memory (asynchronous)
+  void fetch(double* h) {
+    k_lz_last<<<1, 64, 0, stream()>>>(pb[(k + 1) & 1], nb, beta + (k - 1) % kLzRing);
+    QED_HIP(hipMemcpyAsync(h, alpha, 2 * kLzRing * sizeof(double), hipMemcpyDeviceToHost, stream()));
+    QED_HIP(hipGetLastError());
+  }
+};
+
+}  // namespace
+
+// The ground state by Lanczos. The recurrence runs on the device in chunks of steps, the
+// scalars of a chunk come down with one copy, and the host applies the stopping test to
+// each of its steps while the next chunk runs; steps beyond the converged one are dropped.
+// The eigenvector is rebuilt by the same recurrence with the known scalars, one launch per
+// step. Chunks are short where a step costs more than the round trip it saves (about 20 us):
+// below 2^20 amplitudes a step takes 10 to 40 us, above 2^24 over 200 us.
+void lanczos_gs(qed_sector& s, double accur, int max_iter, double* psi, double* E0, int* niter,
+                std::vector<double>* alpha_out, std::vector<double>* beta_out, const LanczosWork* ws) {
+  const uint64_t n = s.D;
+  const int chunk = n <= (1u << 20) ? 8 : n <= (1u << 24) ? 2 : 1;
+  std::vector<double> alpha, beta, evec;
+  double e0 = 0.0;
+  PinnedScalars pin;
+  LanczosRun run(s, ws);
+  run.start(psi);
+  struct Event {
+    hipEvent_t e = nullptr;
+    Event() { QED_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming)); }
+    ~Event() { (void)hipEventDestroy(e); }
+  } done[2];
+  const bool ahead = chunk > 1;
+  int launched = 0, tested = 0;  // steps
+  int end[2] = {0, 0};           // steps done at the end of the two chunks in flight
+  int slot = 0;
+  bool converged = !(2.0 * accur > accur);  // as the loop of the scalar form: no step for such accur
+  auto launch = [&] {
+    const int c = std::max(1, std::min(chunk, max_iter + 1 - launched));
+    for (int i = 0; i < c; ++i) run.step();
+    launched += c;
+    run.fetch(pin.get() + slot * 2 * kLzRing);
+    QED_HIP(hipEventRecord(done[slot].e, stream()));
+    end[slot] = launched;
+    slot ^= 1;
   };
-  auto reset = [&] {
-    vectors();
-    QED_HIP(hipMemcpyAsync(r, psi, n * 8, hipMemcpyDeviceToDevice, stream()));
-    if (ws) k_zero<<<stream_blocks(n), 256, 0, stream()>>>(q, n);
-    else QED_HIP(hipMemsetAsync(q, 0, n * 8, stream()));
-  };
-  if (var >= 0 || !lanczos_eigen_fused(s, accur, max_iter, psi, alpha, beta, evec, e0, ws)) {
-    reset();
-    double ritz = 2.0 * accur;
-    while (ritz > accur) {
-      if (!beta.empty()) scal2(1.0 / beta.back(), r, -beta.back(), q, n);
-      hv(s, r, q, var);
-      std::swap(r, q);
-      double a = dot(q, r, n, ws ? ws->red : nullptr);
-      alpha.push_back(a);
-      beta.push_back(axpy_nrm2(-a, q, r, n, ws ? ws->red : nullptr));
-      tridiag_lowest(alpha, beta, &e0, evec);
-      ritz = std::fabs(evec.back() * beta.back());
+  while (!converged) {
+    if (launched == tested) launch();
+    if (ahead && launched <= max_iter && launched - tested <= chunk) launch();
+    // the older chunk in flight
+    const int o = launched > tested && end[slot] > tested ? slot : slot ^ 1;
+    QED_HIP(hipEventSynchronize(done[o].e));
+    const double* h = pin.get() + o * 2 * kLzRing;
+    for (int k = tested; k < end[o] && !converged; ++k) {
+      alpha.push_back(h[k % kLzRing]);
+      beta.push_back(h[kLzRing + k % kLzRing]);
+      tridiag_lowest_next(alpha, beta, &e0, evec);
       if ((int)alpha.size() > max_iter)
         fail("Lanczos procedure exceeded " + std::to_string(max_iter) + " iterations");
+      converged = !(std::fabs(evec.back() * beta.back()) > accur);
     }
+    tested = end[o];
   }
+  if (!alpha.empty()) tridiag_lowest(alpha, beta, &e0, evec);
   *E0 = e0;
   *niter = (int)beta.size();
   if (alpha_out) *alpha_out = alpha;
   if (beta_out) *beta_out = beta;
-  // eigenvector replay from the saved start vector
-  reset();
-  scal(evec[0], psi, n);
+  if (evec.empty()) return;
+  // eigenvector: the recurrence again from the start vector
+  run.start(psi);
+  if (n) k_scal<<<stream_blocks(n), 256, 0, stream()>>>(evec[0], psi, n);
   for (size_t j = 1; j < evec.size(); ++j) {
-    hv(s, r, q, var);
-    k_replay<<<stream_blocks(n), 256, 0, stream()>>>(alpha[j - 1], beta[j - 1], evec[j], r, q, psi, n);
+    // w_j = (H w_{j-1}) / b1 - (b1 / b2) w_{j-2} - (alpha_{j-1} / b1) w_{j-1}, v_j = w_j / beta_{j-1}
+    const double b1 = j >= 2 ? beta[j - 2] : 1.0, b2 = j >= 3 ? beta[j - 3] : 1.0;
+    LzStep L;
+    L.kind = 2;
+    L.s0 = 1.0 / b1;
+    L.s1 = j >= 2 ? -b1 * (1.0 / b2) : 0.0;
+    L.s2 = alpha[j - 1] * (1.0 / b1);
+    L.c = evec[j] / beta[j - 1];
+    L.psi = psi;
+    hv_step(s, run.r, run.q, L);
+    std::swap(run.r, run.q);
   }
+  QED_HIP(hipGetLastError());
   QED_HIP(hipStreamSynchronize(stream()));
 }
 
@@ -971,9 +1096,9 @@ namespace {
 
 // Device memory of qed_lanczos_gs_noalloc, one copy per GPU for the life of the process:
 // the two recurrence vectors of a sector of at most kNoAllocMaxDim amplitudes, the BLAS-1
-// block partials, the fused step's scalars and row partials (34.7 MB in all).
+// parts and scalars of the steps (34.1 MB in all).
 constexpr uint64_t kNoAllocMaxDim = 1ull << 21;
-constexpr size_t kNoAllocDoubles = 2 * kNoAllocMaxDim + kRedDoubles + 8 + kFusedPartDoubles;
+constexpr size_t kNoAllocDoubles = 2 * kNoAllocMaxDim + kLzWork;
 static __device__ __align__(256) double scratch[kNoAllocDoubles];
 
 constexpr int kMaxDevices = 64;
@@ -1018,8 +1143,7 @@ int qed_lanczos_gs_noalloc(qed_sector* s, double accur, int max_iter, double* ps
       fail("qed_lanczos_gs_noalloc: sector dimension " + std::to_string(s->D) + " exceeds the scratch limit of " +
            std::to_string(kNoAllocMaxDim));
     double* base = noalloc_scratch();
-    const LanczosWork ws{base, base + kNoAllocMaxDim, base + 2 * kNoAllocMaxDim,
-                         base + 2 * kNoAllocMaxDim + kRedDoubles, base + 2 * kNoAllocMaxDim + kRedDoubles + 8};
+    const LanczosWork ws{base, base + kNoAllocMaxDim, base + 2 * kNoAllocMaxDim};
     std::vector<double> a, b;
     lanczos_gs(*s, accur, max_iter, psi, E0, niter, &a, &b, &ws);
     if (alpha) std::copy(a.begin(), a.end(), alpha);
@@ -1029,43 +1153,33 @@ int qed_lanczos_gs_noalloc(qed_sector* s, double accur, int max_iter, double* ps
 
 // Measurement: average milliseconds per Lanczos step of the eigenvalue pass from psi
 // (normalized), `steps` steps each (no stopping test), HIP events on the library stream:
-// ms[0] the fused step (product with the scale and dot folded in, then axpy + norm),
-// ms[1] the separate passes (scale, product, dot, axpy + norm) with their host round
-// trips. ms[0] = -1 when the sector does not take the fused product.
+// ms[0] the step of lanczos_gs (product with the scale and dot folded in, then axpy + norm),
+// ms[1] the separate passes (scale, product, dot, axpy + norm), both with a host round trip
+// per step.
 int qed_lanczos_steps_timed(qed_sector* s, const double* psi, int steps, double* ms) {
   std::lock_guard<std::recursive_mutex> lk(lib_mutex());
   return guard([&] {
     const uint64_t n = s->D;
-    DevBuf rb(n * 8), qb(n * 8), sc(8 * sizeof(double)), part((size_t)std::max<uint32_t>(s->dd, kMaxBlocks) * 8);
-    double* r = rb.as<double>();
-    double* q = qb.as<double>();
-    double* scd = sc.as<double>();
-    double* pd = part.as<double>();
+    LanczosRun run(*s, nullptr);
+    double* r = run.r;
+    double* q = run.q;
     hipEvent_t e0, e1;
     QED_HIP(hipEventCreate(&e0));
     QED_HIP(hipEventCreate(&e1));
-    const uint32_t nb = red_blocks(n);
+    PinnedScalars pin;
     auto reset = [&] {
-      QED_HIP(hipMemcpyAsync(r, psi, n * 8, hipMemcpyDeviceToDevice, stream()));
-      QED_HIP(hipMemsetAsync(q, 0, n * 8, stream()));
-      const double init[8] = {1.0, 0.0, 0.0, 0.0, 0.0, 1.0, 0.0, 0.0};
-      QED_HIP(hipMemcpyAsync(scd, init, sizeof(init), hipMemcpyHostToDevice, stream()));
+      run.start(psi);
       QED_HIP(hipStreamSynchronize(stream()));
     };
-    ms[0] = -1.0;
     reset();
-    if (hv_lanczos(*s, r, q, scd, pd)) {
-      reset();
+    run.step();
+    reset();
+    {
       QED_HIP(hipEventRecord(e0, stream()));
-      double ab[2];
       for (int k = 0; k < steps; ++k) {
-        hv_lanczos(*s, r, q, scd, pd);
-        k_lzf_alpha<<<1, RB, 0, stream()>>>(pd, (int)s->dd, scd);
-        k_lzf_axpy_nrm<<<nb, RB, 0, stream()>>>(scd, r, q, n, pd);
-        k_lzf_beta<<<1, RB, 0, stream()>>>(pd, (int)nb, scd);
-        QED_HIP(hipMemcpyAsync(ab, scd + 2, 2 * sizeof(double), hipMemcpyDeviceToHost, stream()));
+        run.step();
+        run.fetch(pin.get());
         QED_HIP(hipStreamSynchronize(stream()));
-        std::swap(r, q);
       }
       QED_HIP(hipEventRecord(e1, stream()));
       QED_HIP(hipEventSynchronize(e1));

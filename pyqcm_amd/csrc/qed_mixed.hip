@@ -171,13 +171,17 @@ __device__ __forceinline__ uint32_t code_target(uint32_t c, const uint32_t* __re
 
 // y[I] += sum_J H[I, J] x[J], one thread per basis state: the diagonal of the factorized
 // state, and every factorized hop of it mapped to its representative
-template <bool PACKED>
+template <bool PACKED, int EP = 0>
 __global__ __launch_bounds__(256) void k_hv_mixed(HvView v, const uint32_t* __restrict__ up_ell, uint32_t Wu,
                                                   const uint32_t* __restrict__ dn_ell, uint32_t Wd,
                                                   const uint32_t* __restrict__ full_of, const uint32_t* __restrict__ len,
                                                   const uint32_t* __restrict__ code, uint32_t n,
-                                                  const double* __restrict__ x, double* __restrict__ y) {
+                                                  const double* __restrict__ x, double* __restrict__ y,
+                                                  LzStep lz = LzStep{}) {
   constexpr uint32_t mask = (1u << kEllTargetBits) - 1u;
+  double2 sc = make_double2(0.0, 0.0);
+  double dot = 0.0;
+  if constexpr (EP != 0) sc = lz_scalars(lz);
   for (uint32_t I = blockIdx.x * blockDim.x + threadIdx.x; I < n; I += gridDim.x * blockDim.x) {
     const uint32_t f = full_of[I];
     const uint32_t iu = f % v.du, id = f / v.du;
@@ -205,7 +209,12 @@ __global__ __launch_bounds__(256) void k_hv_mixed(HvView v, const uint32_t* __re
       const double t = a * sqrt(lin / (double)lj) * x[J];
       acc += (c >> 31) ? -t : t;
     }
-    y[I] += acc;
+    lz_update<EP>(lz, sc, acc, x[I], y + I, EP == 2 ? lz.psi + I : nullptr, dot);
+  }
+  if constexpr (EP == 1) {
+    __shared__ double red[4];
+    dot = block_sum(dot, red);
+    if (threadIdx.x == 0) lz.pa[blockIdx.x] = dot;
   }
 }
 
@@ -463,20 +472,23 @@ GroupTables group_tables(int N, int n_sites, const std::vector<std::vector<int>>
   return T;
 }
 
-void hv_mixed(const qed_sector& s, const double* x, double* y) {
+template <int EP>
+static int launch_mixed(const qed_sector& s, const double* x, double* y, const LzStep& L) {
   auto T = std::static_pointer_cast<MixedTables>(s.mixed);
   const qed_sector& b = *T->base;
-  const uint32_t n = (uint32_t)s.D;
-  if (n == 0) return;
-  if (T->packed)
-    k_hv_mixed<true><<<grid_for(n), 256, 0, stream()>>>(view(b), b.up_ell.as<uint32_t>(), b.up_w, b.dn_ell.as<uint32_t>(),
-                                                       b.dn_w, T->full_of.as<uint32_t>(), T->len.as<uint32_t>(),
-                                                       T->code.as<uint32_t>(), n, x, y);
-  else
-    k_hv_mixed<false><<<grid_for(n), 256, 0, stream()>>>(view(b), b.up_ell.as<uint32_t>(), b.up_w, b.dn_ell.as<uint32_t>(),
-                                                        b.dn_w, T->full_of.as<uint32_t>(), T->len.as<uint32_t>(),
-                                                        T->code.as<uint32_t>(), n, x, y);
+  const uint32_t n = (uint32_t)s.D, grid = grid_for(n);
+  if (n == 0) return 0;
+  auto k = T->packed ? k_hv_mixed<true, EP> : k_hv_mixed<false, EP>;
+  k<<<grid, 256, 0, stream()>>>(view(b), b.up_ell.as<uint32_t>(), b.up_w, b.dn_ell.as<uint32_t>(), b.dn_w,
+                                T->full_of.as<uint32_t>(), T->len.as<uint32_t>(), T->code.as<uint32_t>(), n, x, y, L);
   QED_HIP(hipGetLastError());
+  return (int)grid;
+}
+
+void hv_mixed(const qed_sector& s, const double* x, double* y) { launch_mixed<0>(s, x, y, LzStep{}); }
+
+int hv_step_mixed(const qed_sector& s, const double* x, double* y, const LzStep& L) {
+  return L.kind == 1 ? launch_mixed<1>(s, x, y, L) : launch_mixed<2>(s, x, y, L);
 }
 
 void sector_diagonal(const qed_sector& s, double* d) {

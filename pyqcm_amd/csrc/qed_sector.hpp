@@ -38,7 +38,6 @@ struct qed_sector {
   qed::DevBuf up_ell, dn_ell;
   uint32_t up_w = 0, dn_w = 0;
 
-  int hv_variant = -1;  // -1 = automatic
   // row visiting order of the tiled-order row kernel (built on its first use)
   mutable qed::DevBuf row_order;
 
@@ -177,10 +176,64 @@ void hv(const qed_sector& s, const double* x, double* y, int variant = -1);
 // sector's structure does not suit them (nothing launched)
 bool hv_split(const qed_sector& s, const double* x, double* y, int passes = 3);
 std::string split_status(const qed_sector& s);
-// one fused Lanczos product: y <- lz[0] (H x) + lz[1] y (device scalars) and, per row of
-// the vector, the partial sums of <x, y_new> in lz_part (dd doubles); false when the
-// sector does not take the fused kernel (nothing launched)
-bool hv_lanczos(const qed_sector& s, const double* x, double* y, const double* lz, double* lz_part);
+// One product of a Lanczos recurrence on unnormalized vectors w_k = beta_{k-1} v_k, with
+// the update of y folded into the product's epilogue:
+//   kind 1 (eigenvalue pass): y <- (H w_k) / beta_{k-1} - (beta_{k-1} / beta_{k-2}) y, the
+//     parts of <w_k, y> in pa[0 .. nparts); beta_{k-1} = sqrt(sum of pb) and beta_{k-2} are
+//     device values, so that no step waits for the host;
+//   kind 2 (eigenvector pass): y <- s0 (H w) + s1 y - s2 w and psi += c y.
+struct LzStep {
+  int kind = 0;
+  int k = 0;                   // step; 0: y <- H w
+  const double* pb = nullptr;  // parts of |w_k|^2, at most kLzParts
+  int nb = 0;
+  const double* beta = nullptr;  // beta_i at beta[i % ring]
+  int ring = 1;
+  double* pa = nullptr;  // kLzRows doubles
+  double s0 = 0, s1 = 0, s2 = 0, c = 0;
+  double* psi = nullptr;
+};
+constexpr int kLzParts = 1024;        // partial sums that every wave of a kernel adds up itself
+constexpr uint32_t kLzRows = 1 << 16;  // parts that a product may leave (folded when above kLzParts)
+// the product of one step; the number of parts it leaves in pa
+int hv_step(const qed_sector& s, const double* x, double* y, const LzStep& L);
+int hv_step_mixed(const qed_sector& s, const double* x, double* y, const LzStep& L);
+int hv_step_general(const qed_sector& s, const double* x, double* y, const LzStep& L);
+
+// Sum of n <= kLzParts values by each wave on its own (no barrier): the order depends on n
+// alone, so that every wave of every kernel gets the same bits.
+__device__ __forceinline__ double lz_sum(const double* __restrict__ p, int n) {
+  double s = 0.0;
+  for (int i = (int)(threadIdx.x & 63); i < n; i += 64) s += p[i];
+  return wave_sum(s);
+}
+__device__ __forceinline__ double lz_inv(double b) { return b != 0.0 ? 1.0 / b : 0.0; }
+// the scalars of step k: s0 = 1 / beta_{k-1}, s1 = -beta_{k-1} / beta_{k-2} (beta_{-1} = 1; a
+// vanishing beta, an exhausted Krylov space, leaves zero vectors instead of NaN)
+__device__ __forceinline__ double2 lz_scalars(const LzStep& L) {
+  if (L.kind == 2) return make_double2(L.s0, L.s1);
+  if (L.k == 0) return make_double2(1.0, 0.0);
+  const double b = sqrt(lz_sum(L.pb, L.nb));
+  const double inv2 = L.k >= 2 ? lz_inv(L.beta[(L.k - 2) % L.ring]) : 1.0;
+  return make_double2(lz_inv(b), -b * inv2);
+}
+// the update of one element; EP 0: y += h, 1 and 2 as LzStep::kind. dot collects <w, y>.
+template <int EP>
+__device__ __forceinline__ void lz_update(const LzStep& L, double2 sc, double h, double w, double* y, double* psi,
+                                          double& dot) {
+  if constexpr (EP == 0) {
+    *y += h;
+  } else if constexpr (EP == 1) {
+    const double v = sc.x * h + sc.y * *y;
+    *y = v;
+    dot += w * v;
+  } else {
+    const double v = (sc.x * h + sc.y * *y) - L.s2 * w;
+    *y = v;
+    *psi += L.c * v;
+  }
+}
+
 // y += H x on a symmetry-adapted sector (s.mixed set)
 void hv_mixed(const qed_sector& s, const double* x, double* y);
 // d += the diagonal of H on a symmetry-adapted or mixed-number sector (D doubles)
@@ -200,36 +253,31 @@ struct GroupTables {
 };
 GroupTables group_tables(int N, int n_sites, const std::vector<std::vector<int>>& gens, bool bath_irrep);
 
-// BLAS-1 on the library stream. dot/nrm2 return host scalars (synchronizing). `work`, where
-// given, is device memory for the block partials (kMaxBlocks * 65 doubles); the library's
-// own buffer otherwise.
-double dot(const double* x, const double* y, uint64_t n, double* work = nullptr);
+// BLAS-1 on the library stream. dot/nrm2 return host scalars (synchronizing).
+double dot(const double* x, const double* y, uint64_t n);
 double nrm2(const double* x, uint64_t n);
 void axpy(double a, const double* x, double* y, uint64_t n);
 void scal(double a, double* x, uint64_t n);
 // r *= ar; q *= aq (one pass)
 void scal2(double ar, double* r, double aq, double* q, uint64_t n);
 // y += a x and returns ||y|| (one pass, synchronizing)
-double axpy_nrm2(double a, const double* x, double* y, uint64_t n, double* work = nullptr);
+double axpy_nrm2(double a, const double* x, double* y, uint64_t n);
 // multi-dot: out[k] = <x, ys[k]> for k < m (one pass over x)
-void multi_dot(const double* x, const double* const* ys, int m, uint64_t n, double* out, double* work = nullptr);
+void multi_dot(const double* x, const double* const* ys, int m, uint64_t n, double* out);
 // y -= sum_k c[k] xs[k] (one pass)
 void multi_axpy(const double* c, const double* const* xs, int m, double* y, uint64_t n);
 // ys[k] -= c[k] x for each k (one pass over x)
 void multi_axpy_rev(const double* c, const double* x, double* const* ys, int m, uint64_t n);
 
 // device memory of a Lanczos run supplied by the caller: the two recurrence vectors (D
-// doubles each), the BLAS-1 block partials (kRedDoubles), the fused step's scalars (8) and
-// row partials (kFusedPartDoubles; the fused step needs max(dd, 2048))
+// doubles each) and the parts and scalars of its steps (kLzWork doubles)
 struct LanczosWork {
   double* r;
   double* q;
   double* red;
-  double* sc;
-  double* part;
 };
-constexpr size_t kRedDoubles = 2048 * 65 + 512;
-constexpr size_t kFusedPartDoubles = 2048;
+constexpr int kLzRing = 64;  // alpha and beta of the last steps on the device
+constexpr size_t kLzWork = kLzRows + 2 * kLzParts + 2 * kLzRing + 64;
 void lanczos_gs(qed_sector& s, double accur, int max_iter, double* psi, double* E0, int* niter,
                 std::vector<double>* alpha, std::vector<double>* beta, const LanczosWork* ws = nullptr);
 int band_lanczos(qed_sector& s, const double* phi, int p0, int M0, int max_iter_BL,

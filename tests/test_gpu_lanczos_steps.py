@@ -1,0 +1,83 @@
+"""The chunked Lanczos ground state on every kind of sector and kernel it takes: values,
+vector and step count against the plain recurrence in numpy, the iteration limit at and
+around a chunk's end, and Krylov spaces that are exhausted inside the first chunk."""
+import numpy as np
+import pytest
+
+from tests import models as TM
+
+pytestmark = pytest.mark.gpu
+
+
+def _plain(hv, x, accur, max_iter):
+    """alpha, beta of the textbook recurrence up to the first step with |beta e_last| <= accur"""
+    a, b = [], []
+    r, q = x.copy(), np.zeros_like(x)
+    while True:
+        if b:
+            r, q = r / b[-1], -b[-1] * q
+        q = q + hv(r)
+        r, q = q, r
+        a.append(q @ r)
+        r = r - a[-1] * q
+        b.append(np.linalg.norm(r))
+        T = np.diag(a) + np.diag(b[:-1], 1) + np.diag(b[:-1], -1)
+        e, u = np.linalg.eigh(T)
+        if abs(u[-1, 0] * b[-1]) <= accur or len(a) > max_iter:
+            return np.array(a), np.array(b), e[0]
+
+
+def _sectors():
+    from pyqcm_amd.sector import GeneralSector, MixedSector, Sector
+    m, v = TM.square(2, 3, tp=-0.3)
+    yield "factorized 6 sites", Sector(6, 3, 3, m.flat(v)), 1e-12
+    yield "factorized one state", Sector(6, 6, 0, m.flat(v)), 1e-12
+    yield "factorized six states", Sector(6, 1, 6, m.flat(v)), 1e-12
+    yield "mirror basis", MixedSector(6, 3, 3, m.flat(v), 6, [[1, 0, 3, 2, 5, 4]], 0), 1e-12
+    m, v = TM.chain(13, U=4.0, mu=2.0)
+    yield "odd rows", Sector(13, 6, 1, m.flat(v)), 1e-11
+    m, v = TM.square(4, 4, tp=-0.3)
+    yield "long rows", Sector(16, 8, 1, m.flat(v)), 1e-11
+    m, v = TM.square(2, 2, tp=-0.3)
+    m.add("hx", "one-body", [(i, i + 4, 1.0) for i in range(4)])
+    v["hx"] = 0.4
+    yield "spin flip", GeneralSector(4, [(nu, 4 - nu) for nu in range(5)], m.flat(v)), 1e-12
+
+
+def test_steps_values_and_vector(gpu_lib):
+    rng = np.random.default_rng(3)
+    for name, S, accur in _sectors():
+        x = rng.standard_normal(S.dim)
+        x /= np.linalg.norm(x)
+        E0, psi, n, a, b = S.lanczos_gs(start=x, accur=accur)
+        pa, pb, pe = _plain(S.hv, x, accur, 1000)
+        psi = psi.to_host()
+        print(name, S.dim, n, len(pa), E0, flush=True)
+        # the last steps of a small space follow a vanishing beta, where the stopping test
+        # sits at round-off: one step either way
+        assert abs(n - len(pa)) <= 1
+        assert abs(E0 - pe) <= 1e-11 * max(1.0, abs(pe))
+        k = max(1, min(n, len(pa)) // 2)  # before orthogonality is lost
+        np.testing.assert_allclose(a[:k], pa[:k], rtol=0, atol=1e-9 * max(1.0, np.abs(pa).max()))
+        # |H psi - E0 psi| = |beta e_last| <= accur and the rounding of psi
+        assert np.linalg.norm(S.hv(psi) - E0 * psi) <= 1e-9 * max(1.0, abs(E0))
+        assert abs(np.linalg.norm(psi) - 1.0) <= 1e-9
+        S.close()
+
+
+@pytest.mark.parametrize("size", [(2, 4), (3, 3)])
+def test_iteration_limit(gpu_lib, size):
+    from pyqcm_amd.sector import Sector
+    m, v = TM.square(*size, tp=-0.3)
+    L = m.L
+    S = Sector(L, L // 2, L // 2, m.flat(v))
+    x = np.random.default_rng(1).standard_normal(S.dim)
+    x /= np.linalg.norm(x)
+    E0, _, n, a, b = S.lanczos_gs(start=x)
+    E1, _, n1, a1, b1 = S.lanczos_gs(start=x, max_iter=n)  # just enough
+    assert (E0, n) == (E1, n1)
+    np.testing.assert_array_equal(a, a1)
+    for limit in (0, 1, 7, 8, 9, 15, 16, 17, n - 1):
+        with pytest.raises(gpu_lib.QEDError, match="exceeded %d iterations" % limit):
+            S.lanczos_gs(start=x, max_iter=limit)
+    S.close()
