@@ -40,7 +40,7 @@ namespace {
 
 constexpr int kBT = 256;               // threads per block
 constexpr uint64_t kChunk = kBT * 8;   // elements per block
-constexpr int kBM = 20;                // vectors per multi-operation
+constexpr int kBM = kBandVectors;      // vectors per multi-operation
 
 __host__ __device__ inline uint32_t nblocks(uint64_t n) { return (uint32_t)((n + kChunk - 1) / kChunk); }
 
@@ -120,13 +120,12 @@ __global__ void k_mdot_final(const MDot* __restrict__ d, int nj, const double* _
   if (lane == 0) D.out[q] = s;
 }
 
-// ---- multi-axpy: y += sgn * sum_q (*c[q]) x[q]; optionally y *= scale first -------------
+// ---- multi-axpy: y += sgn * sum_q (*c[q]) x[q] -------------------------------------------
 struct MAxpy {
   double* y;
   const double* x[kBM];
   const double* c[kBM];  // device scalars
   double sgn;
-  double scale;  // applied to y before the sum
   int m;
   uint64_t n;
   uint32_t blk0;
@@ -143,7 +142,7 @@ __global__ __launch_bounds__(kBT) void k_maxpy(const MAxpy* __restrict__ d, int 
 #pragma unroll
   for (int q = 0; q < kBM; ++q) c[q] = (q < m) ? D.sgn * *D.c[q] : 0.0;
   for (uint64_t i = i0 + threadIdx.x; i < i1; i += kBT) {
-    double v = D.y[i] * D.scale;
+    double v = D.y[i];
 #pragma unroll
     for (int q = 0; q < kBM; ++q)
       if (q < m) v += c[q] * D.x[q][i];
@@ -151,11 +150,14 @@ __global__ __launch_bounds__(kBT) void k_maxpy(const MAxpy* __restrict__ d, int 
   }
 }
 
-// ---- reverse multi-axpy: y[q] -= (*c[q]) x ----------------------------------------------
+// ---- band step, before the product: x *= scale, y[q] -= c[q] x, zero = 0 ---------------
+// (one pass over the vectors: x is read once, and the product's output is cleared here)
 struct MRev {
-  const double* x;
+  double* x;
+  double* zero;
   double* y[kBM];
-  const double* c[kBM];
+  double c[kBM];
+  double scale;
   int m;
   uint64_t n;
   uint32_t blk0;
@@ -168,15 +170,62 @@ __global__ __launch_bounds__(kBT) void k_mrev(const MRev* __restrict__ d, int nj
   const uint64_t i0 = (uint64_t)(b - D.blk0) * kChunk;
   const uint64_t i1 = min(i0 + kChunk, D.n);
   const int m = D.m;
-  double c[kBM];
-#pragma unroll
-  for (int q = 0; q < kBM; ++q) c[q] = (q < m) ? *D.c[q] : 0.0;
-  for (uint64_t i = i0 + threadIdx.x; i < i1; i += kBT) {  // x read once
-    const double xv = D.x[i];
+  const double sc = D.scale;
+  for (uint64_t i = i0 + threadIdx.x; i < i1; i += kBT) {
+    const double xv = D.x[i] * sc;
+    if (sc != 1.0) D.x[i] = xv;
+    if (D.zero) D.zero[i] = 0.0;
 #pragma unroll
     for (int q = 0; q < kBM; ++q)
-      if (q < m) D.y[q][i] -= c[q] * xv;
+      if (q < m) D.y[q][i] -= D.c[q] * xv;
   }
+}
+
+// ---- band step, after the product: y -= sum_q c[q] x[q], and the parts of <dx, y> -------
+struct MTail {
+  double* y;
+  const double* x[kBM];
+  double c[kBM];
+  const double* dx;  // null: no scalar product
+  double* out;
+  int m;
+  uint64_t n;
+  uint32_t blk0;
+};
+
+__global__ __launch_bounds__(kBT) void k_mtail(const MTail* __restrict__ d, int nj, double* __restrict__ part) {
+  __shared__ double red[kBT / 64];
+  const uint32_t b = blockIdx.x;
+  const int j = find_job(d, nj, b);
+  const MTail& D = d[j];
+  const uint64_t i0 = (uint64_t)(b - D.blk0) * kChunk;
+  const uint64_t i1 = min(i0 + kChunk, D.n);
+  const int m = D.m;
+  double acc = 0.0;
+  for (uint64_t i = i0 + threadIdx.x; i < i1; i += kBT) {
+    double v = D.y[i];
+#pragma unroll
+    for (int q = 0; q < kBM; ++q)
+      if (q < m) v -= D.c[q] * D.x[q][i];
+    D.y[i] = v;
+    if (D.dx) acc += D.dx[i] * v;
+  }
+  acc = block_sum(acc, red);
+  if (threadIdx.x == 0) part[b] = acc;
+}
+
+// one wavefront per job
+__global__ void k_mtail_final(const MTail* __restrict__ d, int nj, const double* __restrict__ part) {
+  const int j = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
+  const int lane = threadIdx.x & 63;
+  if (j >= nj) return;
+  const MTail& D = d[j];
+  if (!D.dx) return;
+  const uint32_t nb = nblocks(D.n);
+  double s = 0.0;
+  for (uint32_t b = lane; b < nb; b += 64) s += part[D.blk0 + b];
+  s = wave_sum(s);
+  if (lane == 0) *D.out = s;
 }
 
 // ---- fill: x = 0 ------------------------------------------------------------------------
@@ -569,12 +618,11 @@ void lanczos_gs_batch(const std::vector<qed_sector*>& S, const std::vector<doubl
   QED_HIP(hipMemcpyAsync(dk.p, &zero, sizeof(int), hipMemcpyHostToDevice, stream()));
   // autotune the batched H.v on scratch vectors (results discarded)
   HvBatchConfig cfg;
-  {
-    std::vector<std::unique_ptr<DevBuf>> sx(nj), sy(nj);
+  if (!hv_batch_tuned(HB, cfg)) {
+    std::vector<std::unique_ptr<DevBuf>> sy(nj);
     HvBatch tb;
     hv_batch_prepare(tb, cs);
     for (int j = 0; j < nj; ++j) {
-      sx[j].reset(new DevBuf(S[j]->D * 8));
       sy[j].reset(new DevBuf(S[j]->D * 8));
       tb.host[j].x[0] = tb.host[j].x[1] = A[j]->as<double>();
       tb.host[j].y[0] = tb.host[j].y[1] = sy[j]->as<double>();
@@ -737,15 +785,15 @@ struct BandJob {
   std::vector<double> evec;  // lowest eigenvector of the last test (warm start)
   std::vector<std::unique_ptr<DevBuf>> owned;
   std::vector<double*> free_list;
-  // device scalars of the step: [0..p0] multi-dot, [p0+1 .. p0+pc] pending-block overlaps,
-  // then the deflated-vector overlaps and T(j, j)
+  // device scalars of the step: [0..p0] norm and start-vector overlaps, [p0+1 .. p0+pc)
+  // pending-block overlaps, [2 kBM ..] the deflated-vector overlaps, [3 kBM] T(j, j)
   double* scd = nullptr;  // this job's kSc scalars in the batch's device array
   double* sch = nullptr;  // and their host copy
   // pending host reads from the previous step
-  int prev_j = -1, prev_nk = 0, prev_pc = 0, prev_nI = 0, nk = 0;
+  int prev_j = -1, prev_nI = 0, nk = 0;
   bool check_pending = false;
   double z = 0.0;
-  std::vector<double> hcoef;  // host coefficients uploaded for phase 4
+  std::vector<double> over;  // overlaps of v[j] with the pending block
   double& T(int a, int b) { return t[(size_t)b * M0 + a]; }
   double* get() {
     if (!free_list.empty()) {
@@ -805,7 +853,7 @@ void band_lanczos_batch(const std::vector<qed_sector*>& S, const std::vector<con
   }
   // the step scalars of all jobs in one device array (one download per step, into pinned
   // host memory); the descriptor tables of a step go up in two staged copies: phase 1's,
-  // and those of phases 2-6 together with the host-supplied phase-4 coefficients
+  // and those of phases 2-6
   DevBuf sc_all((size_t)std::max(1, nj) * kSc * sizeof(double));
   double* sch_all = nullptr;
   QED_HIP(hipHostMalloc((void**)&sch_all, (size_t)std::max(1, nj) * kSc * sizeof(double), hipHostMallocDefault));
@@ -815,13 +863,13 @@ void band_lanczos_batch(const std::vector<qed_sector*>& S, const std::vector<con
     J[i].scd = sc_all.as<double>() + (size_t)i * kSc;
     J[i].sch = sch_all + (size_t)i * kSc;
   }
-  // staging bounds: per step at most 8 + 2 kBM tables of nj descriptors, the H.v job table,
-  // the activity flags and the coefficients
-  const size_t per_table = (size_t)std::max(1, nj) * (sizeof(MAxpy) + sizeof(uint32_t)) + 256;
+  // staging bounds: per step at most 8 + 2 kBM tables of nj descriptors, the H.v job table
+  // and the activity flags
+  const size_t per_table =
+      (size_t)std::max(1, nj) * (std::max({sizeof(MAxpy), sizeof(MTail), sizeof(MRev), sizeof(MDot)}) + sizeof(uint32_t)) + 256;
   Stager stage1, stage2;
-  stage1.init(per_table + 256);
-  stage2.init((8 + 2 * (size_t)kBM) * per_table + (size_t)std::max(1, nj) * (sizeof(HvJob) + sizeof(int)) +
-              (size_t)std::max(1, nj) * kBM * sizeof(double) + 4096);
+  stage1.init(2 * per_table + 256);
+  stage2.init((8 + 2 * (size_t)kBM) * per_table + (size_t)std::max(1, nj) * (sizeof(HvJob) + sizeof(int)) + 4096);
   std::vector<std::function<void()>> launches;  // the staged group's kernels, in order
   HvBatch HB;
   if (!cs.empty()) hv_batch_prepare(HB, cs);
@@ -829,7 +877,7 @@ void band_lanczos_batch(const std::vector<qed_sector*>& S, const std::vector<con
   Table<MDot> TD;
   Table<MAxpy> TA;
   Table<MRev> TR;
-  Table<VFill> TF;
+  Table<MTail> TT;
   HvBatchConfig cfg;
   bool tuned = false;
   int steps = 0;
@@ -861,13 +909,27 @@ void band_lanczos_batch(const std::vector<qed_sector*>& S, const std::vector<con
     const int n = (int)TR.h.size();
     launches.push_back([d, total, n] { k_mrev<<<total, kBT, 0, stream()>>>(d, n); });
   };
+  DevBuf part_tail;
+  auto run_mtail = [&]() {
+    if (TT.h.empty()) return;
+    MTail* d = stage2.put(TT);
+    const uint32_t total = TT.total;
+    const int n = (int)TT.h.size();
+    ensure(part_tail, (size_t)total * sizeof(double));
+    launches.push_back([&part_tail, d, total, n] {
+      k_mtail<<<total, kBT, 0, stream()>>>(d, n, part_tail.as<double>());
+      k_mtail_final<<<(n + 3) / 4, 256, 0, stream()>>>(d, n, part_tail.as<double>());
+    });
+  };
   auto flush_launches = [&]() {
     stage2.flush();
     for (auto& f : launches) f();
     launches.clear();
   };
   while (true) {
-    // ---- phase 1: norm of v[j] and overlaps with the start vectors (all live jobs) ----
+    // ---- phase 1: norm of v[j], its overlaps with the start vectors and with the pending
+    //      block (all live jobs). v[j] is not normalized yet: the overlaps are those of the
+    //      normalized vector times its norm ----
     TD.clear();
     bool live = false;
     for (auto& b : J) {
@@ -882,7 +944,22 @@ void band_lanczos_batch(const std::vector<qed_sector*>& S, const std::vector<con
       d.m = b.p0 + 1;
       d.n = b.n;
       d.out = b.scd;
+      const int nk = b.pc - 1;
+      const bool one = d.m + nk <= kBM;  // one pass over v[j] serves both
+      if (one) {
+        for (int q = 0; q < nk; ++q) d.y[d.m + q] = b.v[b.j + 1 + q];
+        d.m += nk;
+      }
       TD.add(d, b.n);
+      if (!one) {
+        MDot e{};
+        e.x = b.v[b.j];
+        for (int q = 0; q < nk; ++q) e.y[q] = b.v[b.j + 1 + q];
+        e.m = nk;
+        e.n = b.n;
+        e.out = b.scd + b.p0 + 1;
+        TD.add(e, b.n);
+      }
     }
     if (!live) break;
     if (!TD.h.empty()) {  // (every live job may have reached M0: it retires below)
@@ -905,13 +982,9 @@ void band_lanczos_batch(const std::vector<qed_sector*>& S, const std::vector<con
       if (b.done) return;
       const double* s = b.sch;
       if (b.prev_j >= 0) {
-        // previous step: [kBM, kBM + nk) pending-block overlaps, [2 kBM, 2 kBM + nI)
-        // deflated-vector overlaps, [3 kBM] T(j, j); phase 1 wrote only [0, p0]
+        // previous step: [2 kBM, 2 kBM + nI) deflated-vector overlaps, [3 kBM] T(j, j);
+        // phase 1 wrote [0, p0] and the pending-block overlaps behind them
         const int pj = b.prev_j;
-        for (int q = 0; q < b.prev_nk; ++q) {
-          const int kk = pj + 1 + q;
-          if (kk >= b.prev_pc) b.T(pj, kk - b.prev_pc) = s[kBM + q];
-        }
         for (int q = 0; q < b.prev_nI; ++q) b.T(b.I[q], pj) = s[2 * kBM + q];
         b.T(pj, pj) = s[3 * kBM];
         for (int kk : b.I) b.T(pj, kk) = b.T(kk, pj);
@@ -991,6 +1064,13 @@ void band_lanczos_batch(const std::vector<qed_sector*>& S, const std::vector<con
       }
       if (b.j >= b.pc) b.T(b.j, b.j - b.pc) = z;
       for (int k = 0; k < b.p0; ++k) b.P[(size_t)b.j * b.p0 + k] = s[k + 1] / z;
+      b.nk = b.pc - 1;
+      b.over.assign(s + b.p0 + 1, s + b.p0 + 1 + b.nk);
+      for (int q = 0; q < b.nk; ++q) {
+        b.over[q] *= 1.0 / z;  // v[j] is scaled by the same factor
+        const int kk = b.j + 1 + q;
+        if (kk >= b.pc) b.T(b.j, kk - b.pc) = b.over[q];
+      }
       b.z = z;
       proceed[i] = 1;
     });
@@ -1001,64 +1081,27 @@ void band_lanczos_batch(const std::vector<qed_sector*>& S, const std::vector<con
       stats->band_checks += n_checks;
       stats->band_dense_checks += n_dense;
     }
-    // ---- phase 2: v[j] /= z; pending block orthogonalized against v[j] ----
-    // scale: y = y * (1/z) with no sum (MAxpy with m = 0)
-    TA.clear();
-    for (int i = 0; i < nj; ++i) {
-      if (!proceed[i]) continue;
-      BandJob& b = J[i];
-      MAxpy a{};
-      a.y = b.v[b.j];
-      a.m = 0;
-      a.sgn = 1.0;
-      a.scale = 1.0 / b.z;
-      a.n = b.n;
-      TA.add(a, b.n);
-    }
-    run_maxpy();
-    TD.clear();
+    // ---- phase 2: v[j] /= z; pending block orthogonalized against it; w = 0 ----
     TR.clear();
+    std::vector<double*> w(nj, nullptr);
     for (int i = 0; i < nj; ++i) {
       if (!proceed[i]) continue;
       BandJob& b = J[i];
-      const int nk = b.pc - 1;
-      b.nk = nk;
-      if (nk <= 0) continue;
-      MDot d{};
-      d.x = b.v[b.j];
-      for (int q = 0; q < nk; ++q) d.y[q] = b.v[b.j + 1 + q];
-      d.m = nk;
-      d.n = b.n;
-      d.out = b.scd + kBM;
-      TD.add(d, b.n);
+      w[i] = b.get();
       MRev r{};
       r.x = b.v[b.j];
-      for (int q = 0; q < nk; ++q) {
+      r.scale = 1.0 / b.z;
+      r.zero = w[i];
+      for (int q = 0; q < b.nk; ++q) {
         r.y[q] = b.v[b.j + 1 + q];
-        r.c[q] = b.scd + kBM + q;
+        r.c[q] = b.over[q];
       }
-      r.m = nk;
+      r.m = b.nk;
       r.n = b.n;
       TR.add(r, b.n);
     }
-    run_mdot();
     run_mrev();
     // ---- phase 3: w = H v[j] ----
-    TF.clear();
-    std::vector<double*> w(nj, nullptr);
-    for (int i = 0; i < nj; ++i) {
-      BandJob& b = J[i];
-      if (proceed[i]) {
-        w[i] = b.get();
-        TF.add(VFill{w[i], b.n, 0}, b.n);
-      }
-    }
-    if (!TF.h.empty()) {
-      VFill* d = stage2.put(TF);
-      const uint32_t total = TF.total;
-      const int n = (int)TF.h.size();
-      launches.push_back([d, total, n] { k_fill0<<<total, kBT, 0, stream()>>>(d, n); });
-    }
     for (size_t q = 0; q < cs.size(); ++q) act[q] = 0;
     for (int i = 0; i < nj; ++i) {
       if (!proceed[i]) continue;
@@ -1075,6 +1118,7 @@ void band_lanczos_batch(const std::vector<qed_sector*>& S, const std::vector<con
       HvJob* jobs_dev = reinterpret_cast<HvJob*>(jr.second);
       const int* act_dev = reinterpret_cast<const int*>(ar.second);
       launches.push_back([&, jobs_dev, act_dev] {
+        if (!tuned && hv_batch_tuned(HB, cfg)) tuned = true;
         if (!tuned) {
           // tune on scratch outputs (the trial products must not land in w)
           std::vector<std::unique_ptr<DevBuf>> sy(cs.size());
@@ -1089,17 +1133,15 @@ void band_lanczos_batch(const std::vector<qed_sector*>& S, const std::vector<con
           cfg = hv_batch_tune(tb, act_dev);
           QED_HIP(hipStreamSynchronize(stream()));
           tuned = true;
-          if (stats) stats->hv_config = cfg;
         }
+        if (stats) stats->hv_config = cfg;
         HB.jobs = jobs_dev;
         hv_batch(HB, cfg, 0, act_dev);
       });
     }
-    // ---- phase 4: w -= sum_k T(k, j) v[k] over the band; release the oldest vector ----
-    TA.clear();
-    auto hcr = stage2.reserve((size_t)std::max(1, nj) * kBM * sizeof(double));
-    double* hch = reinterpret_cast<double*>(hcr.first);
-    const double* hcd = reinterpret_cast<const double*>(hcr.second);
+    // ---- phase 4: w -= sum_k T(k, j) v[k] over the band, T(k, j) = T(j, k); <v_j, w> with
+    //      it where no deflated vector comes in between; release the oldest vector ----
+    TT.clear();
     for (int i = 0; i < nj; ++i) {
       if (!proceed[i]) continue;
       BandJob& b = J[i];
@@ -1111,39 +1153,22 @@ void band_lanczos_batch(const std::vector<qed_sector*>& S, const std::vector<con
           b.v[k0 - 1] = nullptr;
         }
       }
-      // T(k, j) = T(j, k): k = j - pc is z; k = j + 1 + q - pc (0 <= q < nk) is the q-th
-      // pending-block overlap of phase 2, still on the device; other entries are on the host
-      MAxpy a{};
+      MTail a{};
       a.y = w[i];
-      a.sgn = -1.0;
-      a.scale = 1.0;
       a.n = b.n;
-      int m = 0;
-      b.hcoef.clear();
-      std::vector<int> hslot;
       for (int k = k0; k < b.j; ++k) {
-        if (m >= kBM) fail("batched band Lanczos: band too wide");
-        a.x[m] = b.v[k];
-        const int q = k + b.pc - b.j - 1;
-        if (k == b.j - b.pc) {
-          hslot.push_back(m);
-          b.hcoef.push_back(b.z);
-        } else if (q >= 0 && q < b.nk) {
-          a.c[m] = b.scd + kBM + q;
-        } else {
-          hslot.push_back(m);
-          b.hcoef.push_back(b.T(b.j, k));
-        }
-        ++m;
+        if (a.m >= kBM) fail("batched band Lanczos: band too wide");
+        a.x[a.m] = b.v[k];
+        a.c[a.m] = b.T(b.j, k);
+        ++a.m;
       }
-      a.m = m;
-      if (!b.hcoef.empty()) {
-        std::copy(b.hcoef.begin(), b.hcoef.end(), hch + (size_t)i * kBM);
-        for (size_t u = 0; u < hslot.size(); ++u) a.c[hslot[u]] = hcd + (size_t)i * kBM + u;
+      if (b.I.empty()) {
+        a.dx = b.v[b.j];
+        a.out = b.scd + 3 * kBM;
       }
-      if (m > 0) TA.add(a, b.n);
+      if (a.m > 0 || a.dx) TT.add(a, b.n);
     }
-    run_maxpy();
+    run_mtail();
     // ---- phase 5: deflated vectors, one at a time (w -= <v_k, w> v_k) ----
     int maxI = 0;
     for (int i = 0; i < nj; ++i)
@@ -1166,7 +1191,6 @@ void band_lanczos_batch(const std::vector<qed_sector*>& S, const std::vector<con
         a.x[0] = b.v[b.I[u]];
         a.c[0] = b.scd + 2 * kBM + u;
         a.sgn = -1.0;
-        a.scale = 1.0;
         a.m = 1;
         a.n = b.n;
         TA.add(a, b.n);
@@ -1181,19 +1205,20 @@ void band_lanczos_batch(const std::vector<qed_sector*>& S, const std::vector<con
       if (!proceed[i]) continue;
       BandJob& b = J[i];
       if ((int)b.I.size() > kBM) fail("batched band Lanczos: too many deflations");
-      MDot d{};
-      d.x = b.v[b.j];
-      d.y[0] = w[i];
-      d.m = 1;
-      d.n = b.n;
-      d.out = b.scd + 3 * kBM;
-      TD.add(d, b.n);
+      if (!b.I.empty()) {
+        MDot d{};
+        d.x = b.v[b.j];
+        d.y[0] = w[i];
+        d.m = 1;
+        d.n = b.n;
+        d.out = b.scd + 3 * kBM;
+        TD.add(d, b.n);
+      }
       MAxpy a{};
       a.y = w[i];
       a.x[0] = b.v[b.j];
       a.c[0] = b.scd + 3 * kBM;
       a.sgn = -1.0;
-      a.scale = 1.0;
       a.m = 1;
       a.n = b.n;
       TA.add(a, b.n);
@@ -1206,8 +1231,6 @@ void band_lanczos_batch(const std::vector<qed_sector*>& S, const std::vector<con
       BandJob& b = J[i];
       b.v[b.j + b.pc] = w[i];
       b.prev_j = b.j;
-      b.prev_pc = b.pc;
-      b.prev_nk = b.nk;
       b.prev_nI = (int)b.I.size();
       b.check_pending = (b.j >= 4 * b.p0 && b.j % b.p0 == 0);
       ++b.j;

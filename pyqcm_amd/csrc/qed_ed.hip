@@ -628,6 +628,43 @@ QMat sector_qmatrix(qed_sector& T, const double* phi, int p) {
   return q;
 }
 
+// Sectors whose band Lanczos runs in the batched form, both parts of a Green function in
+// step: factorized, rows in LDS, few start vectors, and small enough that the host round
+// trips of the one-sector form cost more than its vectors (and that twice the vectors are
+// no burden).
+bool batched_band(const qed_sector& T, int p) {
+  return T.factorized() && p + 1 <= kBandVectors && T.D <= (1u << 22) && T.du <= 4096;
+}
+
+// Lehmann forms of several sectors, p start vectors each (null sectors give empty forms)
+std::vector<QMat> sector_qmatrices(const std::vector<qed_sector*>& T, const std::vector<const double*>& phi, int p) {
+  std::vector<QMat> out(T.size());
+  std::vector<qed_sector*> S;
+  std::vector<const double*> ph;
+  std::vector<size_t> which;
+  for (size_t k = 0; k < T.size(); ++k) {
+    if (!T[k]) continue;
+    if (T[k]->D < (uint64_t)gi("max_dim_full") || !batched_band(*T[k], p)) {
+      out[k] = sector_qmatrix(*T[k], phi[k], p);
+      continue;
+    }
+    S.push_back(T[k]);
+    ph.push_back(phi[k]);
+    which.push_back(k);
+  }
+  if (!S.empty()) {
+    std::vector<std::vector<double>> e, Q;
+    band_lanczos_batch(S, ph, std::vector<int>(S.size(), p), gi("max_iter_BL"), gd("accur_deflation"),
+                       gd("accur_band_lanczos"), e, Q, nullptr, degeneracy_gap());
+    for (size_t u = 0; u < which.size(); ++u) {
+      out[which[u]].L = p;
+      out[which[u]].e = std::move(e[u]);
+      out[which[u]].Q = std::move(Q[u]);
+    }
+  }
+  return out;
+}
+
 bool sector_valid(const Instance& I, int nup, int ndn) {
   const int L = I.model->L;
   return nup >= 0 && ndn >= 0 && nup <= L && ndn <= L;
@@ -838,25 +875,47 @@ void build_qmatrix(Instance& I, State& st, int spin) {
   }
   Model& M = *I.model;
   const int p = M.n_sites, L = M.L;
+  SectorPtr sec[2];
+  DevBuf phi[2];
+  std::vector<qed_sector*> T(2, nullptr);
+  std::vector<const double*> ph(2, nullptr);
   QMat parts[2];
+  bool done[2] = {false, false};
   for (int s = 0; s < 2; ++s) {
     const int pm = 2 * s - 1;
     const int tnup = st.nup + (spin == 0 ? pm : 0), tndn = st.ndn + (spin == 1 ? pm : 0);
     if (!sector_valid(I, tnup, tndn)) continue;
-    SectorPtr T = make_sector(I, tnup, tndn);
-    if (T->D == 0) continue;
-    DevBuf phi((size_t)p * T->D * 8);
-    QED_HIP(hipMemsetAsync(phi.p, 0, (size_t)p * T->D * 8, stream()));
+    sec[s] = make_sector(I, tnup, tndn);
+    if (sec[s]->D == 0) continue;
+    const uint64_t D = sec[s]->D;
+    phi[s].alloc((size_t)p * D * 8);
+    QED_HIP(hipMemsetAsync(phi[s].p, 0, (size_t)p * D * 8, stream()));
     for (int i = 0; i < p; ++i)
       if (qed_apply_c(L, st.nup, st.ndn, i + spin * L, pm, 1.0, st.psi.as<double>(),
-                      phi.as<double>() + (uint64_t)i * T->D) != 0)
+                      phi[s].as<double>() + (uint64_t)i * D) != 0)
         fail(qed_last_error());
-    QMat q = sector_qmatrix(*T, phi.as<double>(), p);
-    for (double& e : q.e) {
-      e -= st.energy;
-      if (pm == -1) e = -e;
+    T[s] = sec[s].get();
+    ph[s] = phi[s].as<double>();
+    // large: one part in memory at a time. A form to be rewritten as a matrix continued
+    // fraction also keeps the one-sector recurrence: the rewriting stops on a test at
+    // round-off level and amplifies the last bits of its poles
+    if (!batched_band(*T[s], p) || I.q_to_mcf) {
+      parts[s] = sector_qmatrix(*T[s], ph[s], p);
+      done[s] = true;
+      T[s] = nullptr;
+      phi[s].release();
+      sec[s].reset();
     }
-    parts[s] = streamline(q);
+  }
+  std::vector<QMat> q = sector_qmatrices(T, ph, p);
+  for (int s = 0; s < 2; ++s) {
+    if (T[s]) parts[s] = std::move(q[s]);
+    else if (!done[s]) continue;
+    for (double& e : parts[s].e) {
+      e -= st.energy;
+      if (s == 0) e = -e;
+    }
+    parts[s] = streamline(parts[s]);
   }
   QMat tot;
   tot.L = p;

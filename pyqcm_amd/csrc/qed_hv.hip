@@ -1081,6 +1081,13 @@ HvBatchConfig hv_batch_tune(const HvBatch& B, const int* active, bool force) {
   return best;
 }
 
+bool hv_batch_tuned(const HvBatch& B, HvBatchConfig& cfg) {
+  auto it = tune_cache().find(TuneKey{B.sig});
+  if (it == tune_cache().end()) return false;
+  cfg = it->second;
+  return true;
+}
+
 void hv_batch(const HvBatch& B, const HvBatchConfig& cfg, int parity, const int* active) {
   launch_batch(B, cfg, parity, active, stream());
   QED_HIP(hipGetLastError());

@@ -142,6 +142,8 @@ void hv_batch_upload(HvBatch& B);
 // times the candidate launch shapes on this batch (y[0] of every job receives the sums of
 // the trial products: pass scratch vectors) and caches the fastest by shape signature
 HvBatchConfig hv_batch_tune(const HvBatch& B, const int* active, bool force = false);
+// the tuned launch shape of such a batch, if there is one
+bool hv_batch_tuned(const HvBatch& B, HvBatchConfig& cfg);
 void hv_batch(const HvBatch& B, const HvBatchConfig& cfg, int parity, const int* active);
 
 struct BatchStats {
@@ -162,6 +164,7 @@ BatchStats& last_batch_stats();
 void lanczos_gs_batch(const std::vector<qed_sector*>& S, const std::vector<double*>& psi, double accur,
                       int max_iter, bool use_graph, int chunk, std::vector<double>& E0,
                       std::vector<int>& niter, BatchStats* stats);
+constexpr int kBandVectors = 20;  // vectors of one multi-vector operation of the batched band Lanczos
 // band Lanczos of many sectors (start vectors phi[j]: p[j] x D_j on the device)
 void band_lanczos_batch(const std::vector<qed_sector*>& S, const std::vector<const double*>& phi,
                         const std::vector<int>& p, int max_iter_BL, double accur_deflation,
