@@ -558,8 +558,8 @@ class HostPool {
 };
 
 template <class F>
-void parallel_for(int n, F f) {
-  if (n < 4 || HostPool::get().threads() <= 1) {
+void parallel_for(int n, F f, int at_least = 4) {
+  if (n < at_least || HostPool::get().threads() <= 1) {
     for (int i = 0; i < n; ++i) f(i);
     return;
   }
@@ -1246,17 +1246,11 @@ void band_lanczos_batch(const std::vector<qed_sector*>& S, const std::vector<con
     if (b.n == 0 || b.p0 == 0 || jj == 0) return;
     std::vector<double> H((size_t)jj * jj);
     for (int c = 0; c < jj; ++c)
-      for (int r = 0; r < jj; ++r) H[(size_t)c * jj + r] = b.T(r, c);
+      for (int r = c; r < jj; ++r) H[(size_t)r * jj + c] = b.T(r, c);  // (the band is stored below the diagonal)
     evals[i].assign(jj, 0.0);
-    sym_eigen(jj, H.data(), evals[i].data(), true);
-    Q[i].assign((size_t)b.p0 * jj, 0.0);
-    for (int c = 0; c < jj; ++c)
-      for (int m = 0; m < jj; ++m) {
-        const double u = H[(size_t)c * jj + m];
-        if (u == 0.0) continue;
-        for (int k = 0; k < b.p0; ++k) Q[i][(size_t)c * b.p0 + k] += b.P[(size_t)m * b.p0 + k] * u;
-      }
-  });
+    Q[i].assign(b.P.begin(), b.P.begin() + (size_t)b.p0 * jj);
+    sym_eigen_project(jj, H.data(), evals[i].data(), b.p0, Q[i].data());
+  }, 2);
 }
 
 BatchStats& last_batch_stats() {

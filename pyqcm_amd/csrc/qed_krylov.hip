@@ -743,17 +743,11 @@ int band_lanczos(qed_sector& s, const double* phi, int p0, int M0, int max_iter_
   if (j == 0) return 0;
   std::vector<double> Hpr((size_t)j * j);
   for (int c = 0; c < j; ++c)
-    for (int r = 0; r < j; ++r) Hpr[(size_t)c * j + r] = T(r, c);
+    for (int r = c; r < j; ++r) Hpr[(size_t)r * j + c] = T(r, c);
   evals.assign(j, 0.0);
-  sym_eigen(j, Hpr.data(), evals.data(), true);
   // Q = P U  (p0 x j)
-  Q.assign((size_t)p0 * j, 0.0);
-  for (int c = 0; c < j; ++c)
-    for (int m = 0; m < j; ++m) {
-      double u = Hpr[(size_t)c * j + m];
-      if (u == 0.0) continue;
-      for (int k = 0; k < p0; ++k) Q[(size_t)c * p0 + k] += P[(size_t)m * p0 + k] * u;
-    }
+  Q.assign(P.begin(), P.begin() + (size_t)p0 * j);
+  sym_eigen_project(j, Hpr.data(), evals.data(), p0, Q.data());
   return j;
 }
 

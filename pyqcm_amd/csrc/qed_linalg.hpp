@@ -21,6 +21,10 @@ void tridiag_eigen(int n, double* d, const double* e, double* z);
 // eigenvalues in w; eigenvectors (columns) in a if vectors.
 void sym_eigen(int n, double* a, double* w, bool vectors);
 
+// Ascending eigenvalues w of the symmetric a (n x n; its lower triangle a[i n + j], j <= i,
+// is read) and P U for its eigenvectors U, in place of P (p x n, column-major)
+void sym_eigen_project(int n, const double* a, double* w, int p, double* P);
+
 // Complex dense inverse in place (n x n column-major); returns false if singular.
 bool cinverse(int n, std::complex<double>* a);
 // log |det a| (a is overwritten by its LU factors).
