@@ -816,7 +816,7 @@ constexpr int kSc = 4 * kBM + 8;  // device scalars per job and step
 void band_lanczos_batch(const std::vector<qed_sector*>& S, const std::vector<const double*>& phi,
                         const std::vector<int>& p, int max_iter_BL, double accur_deflation,
                         double accur_band_lanczos, std::vector<std::vector<double>>& evals,
-                        std::vector<std::vector<double>>& Q, BatchStats* stats, double min_gap) {
+                        std::vector<std::vector<double>>& Q, BatchStats* stats, double min_gap, bool rows) {
   const int nj = (int)S.size();
   std::atomic<int> gap_fail{0};  // a degenerate pair found by a worker (no_degenerate_BL)
   evals.assign(nj, {});
@@ -1118,7 +1118,7 @@ void band_lanczos_batch(const std::vector<qed_sector*>& S, const std::vector<con
       HvJob* jobs_dev = reinterpret_cast<HvJob*>(jr.second);
       const int* act_dev = reinterpret_cast<const int*>(ar.second);
       launches.push_back([&, jobs_dev, act_dev] {
-        if (!tuned && hv_batch_tuned(HB, cfg)) tuned = true;
+        if (!tuned && hv_batch_tuned(HB, cfg, rows)) tuned = true;
         if (!tuned) {
           // tune on scratch outputs (the trial products must not land in w)
           std::vector<std::unique_ptr<DevBuf>> sy(cs.size());
@@ -1130,7 +1130,7 @@ void band_lanczos_batch(const std::vector<qed_sector*>& S, const std::vector<con
             tb.host[q].y[0] = tb.host[q].y[1] = sy[q]->as<double>();
           }
           hv_batch_upload(tb);
-          cfg = hv_batch_tune(tb, act_dev);
+          cfg = hv_batch_tune(tb, act_dev, rows);
           QED_HIP(hipStreamSynchronize(stream()));
           tuned = true;
         }

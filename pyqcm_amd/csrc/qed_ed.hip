@@ -631,7 +631,8 @@ QMat sector_qmatrix(qed_sector& T, const double* phi, int p) {
 // Sectors whose band Lanczos runs in the batched form, both parts of a Green function in
 // step: factorized, rows in LDS, few start vectors, and small enough that the host round
 // trips of the one-sector form cost more than its vectors (and that twice the vectors are
-// no burden).
+// no burden). The products take the row form, so that the result does not depend on the
+// launch shape that is timed to be the fastest.
 bool batched_band(const qed_sector& T, int p) {
   return T.factorized() && p + 1 <= kBandVectors && T.D <= (1u << 22) && T.du <= 4096;
 }
@@ -655,7 +656,7 @@ std::vector<QMat> sector_qmatrices(const std::vector<qed_sector*>& T, const std:
   if (!S.empty()) {
     std::vector<std::vector<double>> e, Q;
     band_lanczos_batch(S, ph, std::vector<int>(S.size(), p), gi("max_iter_BL"), gd("accur_deflation"),
-                       gd("accur_band_lanczos"), e, Q, nullptr, degeneracy_gap());
+                       gd("accur_band_lanczos"), e, Q, nullptr, degeneracy_gap(), true);
     for (size_t u = 0; u < which.size(); ++u) {
       out[which[u]].L = p;
       out[which[u]].e = std::move(e[u]);
@@ -896,10 +897,8 @@ void build_qmatrix(Instance& I, State& st, int spin) {
         fail(qed_last_error());
     T[s] = sec[s].get();
     ph[s] = phi[s].as<double>();
-    // large: one part in memory at a time. A form to be rewritten as a matrix continued
-    // fraction also keeps the one-sector recurrence: the rewriting stops on a test at
-    // round-off level and amplifies the last bits of its poles
-    if (!batched_band(*T[s], p) || I.q_to_mcf) {
+    // large: one part in memory at a time
+    if (!batched_band(*T[s], p)) {
       parts[s] = sector_qmatrix(*T[s], ph[s], p);
       done[s] = true;
       T[s] = nullptr;

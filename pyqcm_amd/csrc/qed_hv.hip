@@ -912,6 +912,11 @@ struct TuneKey {
   std::vector<uint64_t> sig;
   bool operator<(const TuneKey& o) const { return sig < o.sig; }
 };
+TuneKey tune_key(const HvBatch& B, bool rows) {
+  TuneKey k{B.sig};
+  k.sig.push_back(rows ? 1 : 0);
+  return k;
+}
 std::map<TuneKey, HvBatchConfig>& tune_cache() {
   static std::map<TuneKey, HvBatchConfig> c;
   return c;
@@ -1040,7 +1045,7 @@ void hv_batch_upload(HvBatch& B) {
                          stream()));
 }
 
-HvBatchConfig hv_batch_tune(const HvBatch& B, const int* active, bool force) {
+HvBatchConfig hv_batch_tune(const HvBatch& B, const int* active, bool rows) {
   static std::once_flag once;
   std::call_once(once, [] {
     const int bytes = (int)lds_budget();
@@ -1048,15 +1053,15 @@ HvBatchConfig hv_batch_tune(const HvBatch& B, const int* active, bool force) {
     (void)hipFuncSetAttribute((const void*)k_hv_ell_batch<512>, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
     (void)hipFuncSetAttribute((const void*)k_hv_ell_batch<1024>, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
   });
-  TuneKey key{B.sig};
+  const TuneKey key = tune_key(B, rows);
   auto it = tune_cache().find(key);
-  if (it != tune_cache().end() && !force) return it->second;
+  if (it != tune_cache().end()) return it->second;
   // candidates: block size x persistent grid (multiples of the CU count) or one tile per block
   const int cus = device_cu_count();
   std::vector<HvBatchConfig> cand;
   for (int bs : {256, 512, 1024})
     for (int mult : {0, 2, 4, 8}) cand.push_back({bs, mult ? (uint32_t)(cus * mult) : 0u, 0.0f, 0});
-  if (B.tiled)
+  if (B.tiled && !rows)
     for (int mult : {0, 4, 8}) cand.push_back({256, mult ? (uint32_t)(cus * mult) : 0u, 0.0f, 1});
   hipEvent_t e0, e1;
   QED_HIP(hipEventCreate(&e0));
@@ -1081,8 +1086,8 @@ HvBatchConfig hv_batch_tune(const HvBatch& B, const int* active, bool force) {
   return best;
 }
 
-bool hv_batch_tuned(const HvBatch& B, HvBatchConfig& cfg) {
-  auto it = tune_cache().find(TuneKey{B.sig});
+bool hv_batch_tuned(const HvBatch& B, HvBatchConfig& cfg, bool rows) {
+  auto it = tune_cache().find(tune_key(B, rows));
   if (it == tune_cache().end()) return false;
   cfg = it->second;
   return true;

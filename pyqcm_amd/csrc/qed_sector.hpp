@@ -141,9 +141,11 @@ void hv_batch_prepare(HvBatch& B, const std::vector<const qed_sector*>& S);
 void hv_batch_upload(HvBatch& B);
 // times the candidate launch shapes on this batch (y[0] of every job receives the sums of
 // the trial products: pass scratch vectors) and caches the fastest by shape signature
-HvBatchConfig hv_batch_tune(const HvBatch& B, const int* active, bool force = false);
+// rows: the row form only, whose sums run in the same order whatever the launch shape (the
+// tiled form's do not, and a choice by timing between the two changes last bits)
+HvBatchConfig hv_batch_tune(const HvBatch& B, const int* active, bool rows = false);
 // the tuned launch shape of such a batch, if there is one
-bool hv_batch_tuned(const HvBatch& B, HvBatchConfig& cfg);
+bool hv_batch_tuned(const HvBatch& B, HvBatchConfig& cfg, bool rows = false);
 void hv_batch(const HvBatch& B, const HvBatchConfig& cfg, int parity, const int* active);
 
 struct BatchStats {
@@ -169,7 +171,8 @@ constexpr int kBandVectors = 20;  // vectors of one multi-vector operation of th
 void band_lanczos_batch(const std::vector<qed_sector*>& S, const std::vector<const double*>& phi,
                         const std::vector<int>& p, int max_iter_BL, double accur_deflation,
                         double accur_band_lanczos, std::vector<std::vector<double>>& evals,
-                        std::vector<std::vector<double>>& Q, BatchStats* stats, double min_gap = -1.0);
+                        std::vector<std::vector<double>>& Q, BatchStats* stats, double min_gap = -1.0,
+                        bool rows = false);
 void tridiag_lowest(const std::vector<double>& a, const std::vector<double>& b, double* e0,
                     std::vector<double>& vec);
 
