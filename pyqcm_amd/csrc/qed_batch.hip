@@ -41,7 +41,24 @@ namespace {
 constexpr int kBT = 256;               // threads per block
 constexpr uint64_t kChunk = kBT * 8;   // elements per block
 constexpr int kBM = kBandVectors;      // vectors per multi-operation
+// Chunks of a launch that leave half of the chip idle: a pass is then bound by the latency of
+// each thread's chain of loads, and its work is spread over more threads with every sum in
+// its old order (8 sites, 2 chunks a part: multi-dot 25 -> 6.2 us, band subtraction 14 -> 6.7,
+// update before the product 13 -> 5.6). Above, the vectors' bytes bound a pass and one read
+// of x serves all of a block's vectors.
+constexpr uint32_t kFewBlocks = 128;
 
+// An elementwise pass (D::kElementwise) over a vector that would leave most of the chip idle
+// takes a quarter of that: 8 sites, 3920 amplitudes, are two blocks else. Sums keep one
+// partition, and so one order of their terms, at all sizes.
+template <class D>
+__host__ __device__ inline uint64_t chunk_of(uint64_t n) {
+  return D::kElementwise && n <= (1u << 17) ? kChunk / 4 : kChunk;
+}
+template <class D>
+__host__ __device__ inline uint32_t blocks_of(uint64_t n) {
+  return (uint32_t)((n + chunk_of<D>(n) - 1) / chunk_of<D>(n));
+}
 __host__ __device__ inline uint32_t nblocks(uint64_t n) { return (uint32_t)((n + kChunk - 1) / kChunk); }
 
 template <class D>
@@ -70,6 +87,7 @@ __device__ __forceinline__ double block_sum(double v, double* red) {
 
 // ---- multi-dot: out[q] = <x, y[q]> -------------------------------------------------------
 struct MDot {
+  static constexpr bool kElementwise = false;
   const double* x;
   const double* y[kBM];
   double* out;  // device, m values
@@ -78,30 +96,68 @@ struct MDot {
   uint32_t blk0;
 };
 
+// Block (b, g): the g-th NQ of the vectors y over one chunk. NQ = kBM reads x once; few
+// chunks (launch_mdot) split the vectors over blocks instead, with all loads of a chunk in
+// flight. Either way each sum is one thread's terms in order, then its wave, then the waves.
+template <int NQ>
 __global__ __launch_bounds__(kBT) void k_mdot_part(const MDot* __restrict__ d, int nj,
                                                    double* __restrict__ part) {
-  __shared__ double red[kBT / 64];
+  __shared__ double red[kBT / 64][NQ];
   const uint32_t b = blockIdx.x;
+  const int q0 = blockIdx.y * NQ;
   const int j = find_job(d, nj, b);
   const MDot& D = d[j];
+  const int m = min(D.m - q0, NQ);
+  if (m <= 0) return;
   const uint64_t i0 = (uint64_t)(b - D.blk0) * kChunk;
   const uint64_t i1 = min(i0 + kChunk, D.n);
-  const int m = D.m;
-  double acc[kBM];
+  double acc[NQ];
 #pragma unroll
-  for (int q = 0; q < kBM; ++q) acc[q] = 0.0;
-  for (uint64_t i = i0 + threadIdx.x; i < i1; i += kBT) {  // x read once
-    const double xv = D.x[i];
+  for (int q = 0; q < NQ; ++q) acc[q] = 0.0;
+  if constexpr (NQ == kBM) {
+    for (uint64_t i = i0 + threadIdx.x; i < i1; i += kBT) {
+      const double xv = D.x[i];
 #pragma unroll
-    for (int q = 0; q < kBM; ++q)
-      if (q < m) acc[q] += xv * D.y[q][i];
-  }
-#pragma unroll
-  for (int q = 0; q < kBM; ++q) {
-    if (q < m) {  // uniform across the block
-      const double s = block_sum(acc[q], red);
-      if (threadIdx.x == 0) part[(size_t)b * kBM + q] = s;
+      for (int q = 0; q < NQ; ++q)
+        if (q < m) acc[q] += xv * D.y[q][i];
     }
+  } else {
+    constexpr int K = (int)(kChunk / kBT);
+    double xv[K];
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const uint64_t i = i0 + threadIdx.x + (uint64_t)k * kBT;
+      xv[k] = i < i1 ? D.x[i] : 0.0;
+    }
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+      if (q < m) {
+        const double* __restrict__ y = D.y[q0 + q];
+        double yv[K];
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+          const uint64_t i = i0 + threadIdx.x + (uint64_t)k * kBT;
+          yv[k] = i < i1 ? y[i] : 0.0;
+        }
+#pragma unroll
+        for (int k = 0; k < K; ++k) acc[q] += xv[k] * yv[k];
+      }
+    }
+  }
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) {
+    if (q < m) {  // uniform across the block
+      const double s = wave_sum(acc[q]);
+      if (lane == 0) red[wave][q] = s;
+    }
+  }
+  __syncthreads();
+  if ((int)threadIdx.x < m) {
+    double s = 0.0;
+#pragma unroll
+    for (int i = 0; i < kBT / 64; ++i) s += red[i][threadIdx.x];
+    part[(size_t)b * kBM + q0 + threadIdx.x] = s;
   }
 }
 
@@ -120,8 +176,16 @@ __global__ void k_mdot_final(const MDot* __restrict__ d, int nj, const double* _
   if (lane == 0) D.out[q] = s;
 }
 
+void launch_mdot(const MDot* d, uint32_t total, int n, double* part) {
+  constexpr int NQ = 4;
+  if (total <= kFewBlocks) k_mdot_part<NQ><<<dim3(total, (kBM + NQ - 1) / NQ), kBT, 0, stream()>>>(d, n, part);
+  else k_mdot_part<kBM><<<total, kBT, 0, stream()>>>(d, n, part);
+  k_mdot_final<<<(n * kBM + 3) / 4, 256, 0, stream()>>>(d, n, part);
+}
+
 // ---- multi-axpy: y += sgn * sum_q (*c[q]) x[q] -------------------------------------------
 struct MAxpy {
+  static constexpr bool kElementwise = true;
   double* y;
   const double* x[kBM];
   const double* c[kBM];  // device scalars
@@ -135,8 +199,9 @@ __global__ __launch_bounds__(kBT) void k_maxpy(const MAxpy* __restrict__ d, int 
   const uint32_t b = blockIdx.x;
   const int j = find_job(d, nj, b);
   const MAxpy& D = d[j];
-  const uint64_t i0 = (uint64_t)(b - D.blk0) * kChunk;
-  const uint64_t i1 = min(i0 + kChunk, D.n);
+  const uint64_t ch = chunk_of<MAxpy>(D.n);
+  const uint64_t i0 = (uint64_t)(b - D.blk0) * ch;
+  const uint64_t i1 = min(i0 + ch, D.n);
   const int m = D.m;
   double c[kBM];
 #pragma unroll
@@ -153,6 +218,7 @@ __global__ __launch_bounds__(kBT) void k_maxpy(const MAxpy* __restrict__ d, int 
 // ---- band step, before the product: x *= scale, y[q] -= c[q] x, zero = 0 ---------------
 // (one pass over the vectors: x is read once, and the product's output is cleared here)
 struct MRev {
+  static constexpr bool kElementwise = true;
   double* x;
   double* zero;
   double* y[kBM];
@@ -167,8 +233,9 @@ __global__ __launch_bounds__(kBT) void k_mrev(const MRev* __restrict__ d, int nj
   const uint32_t b = blockIdx.x;
   const int j = find_job(d, nj, b);
   const MRev& D = d[j];
-  const uint64_t i0 = (uint64_t)(b - D.blk0) * kChunk;
-  const uint64_t i1 = min(i0 + kChunk, D.n);
+  const uint64_t ch = chunk_of<MRev>(D.n);
+  const uint64_t i0 = (uint64_t)(b - D.blk0) * ch;
+  const uint64_t i1 = min(i0 + ch, D.n);
   const int m = D.m;
   const double sc = D.scale;
   for (uint64_t i = i0 + threadIdx.x; i < i1; i += kBT) {
@@ -183,6 +250,7 @@ __global__ __launch_bounds__(kBT) void k_mrev(const MRev* __restrict__ d, int nj
 
 // ---- band step, after the product: y -= sum_q c[q] x[q], and the parts of <dx, y> -------
 struct MTail {
+  static constexpr bool kElementwise = false;
   double* y;
   const double* x[kBM];
   double c[kBM];
@@ -193,8 +261,12 @@ struct MTail {
   uint32_t blk0;
 };
 
-__global__ __launch_bounds__(kBT) void k_mtail(const MTail* __restrict__ d, int nj, double* __restrict__ part) {
+// BT = kBT, or four times that for few chunks: all its threads update the chunk, and kBT of
+// them add up <dx, y> from LDS in the order that kBT threads alone would
+template <int BT>
+__global__ __launch_bounds__(BT) void k_mtail(const MTail* __restrict__ d, int nj, double* __restrict__ part) {
   __shared__ double red[kBT / 64];
+  __shared__ double vs[BT > kBT ? kChunk : 1], ds[BT > kBT ? kChunk : 1];
   const uint32_t b = blockIdx.x;
   const int j = find_job(d, nj, b);
   const MTail& D = d[j];
@@ -202,15 +274,33 @@ __global__ __launch_bounds__(kBT) void k_mtail(const MTail* __restrict__ d, int 
   const uint64_t i1 = min(i0 + kChunk, D.n);
   const int m = D.m;
   double acc = 0.0;
-  for (uint64_t i = i0 + threadIdx.x; i < i1; i += kBT) {
+  for (uint64_t i = i0 + threadIdx.x; i < i1; i += BT) {
     double v = D.y[i];
 #pragma unroll
     for (int q = 0; q < kBM; ++q)
       if (q < m) v -= D.c[q] * D.x[q][i];
     D.y[i] = v;
-    if (D.dx) acc += D.dx[i] * v;
+    if constexpr (BT > kBT) {
+      vs[i - i0] = v;
+      ds[i - i0] = D.dx ? D.dx[i] : 0.0;
+    } else {
+      if (D.dx) acc += D.dx[i] * v;
+    }
   }
-  acc = block_sum(acc, red);
+  if constexpr (BT > kBT) {
+    __syncthreads();
+    if (threadIdx.x < kBT) {
+      const uint32_t c = (uint32_t)(i1 - i0);
+      for (uint32_t i = threadIdx.x; i < c; i += kBT) acc += ds[i] * vs[i];
+      acc = wave_sum(acc);
+      if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;
+    }
+    __syncthreads();
+    acc = 0.0;
+    for (int i = 0; i < kBT / 64; ++i) acc += red[i];
+  } else {
+    acc = block_sum(acc, red);
+  }
   if (threadIdx.x == 0) part[b] = acc;
 }
 
@@ -230,6 +320,7 @@ __global__ void k_mtail_final(const MTail* __restrict__ d, int nj, const double*
 
 // ---- fill: x = 0 ------------------------------------------------------------------------
 struct VFill {
+  static constexpr bool kElementwise = true;
   double* x;
   uint64_t n;
   uint32_t blk0;
@@ -239,14 +330,16 @@ __global__ __launch_bounds__(kBT) void k_fill0(const VFill* __restrict__ d, int 
   const uint32_t b = blockIdx.x;
   const int j = find_job(d, nj, b);
   const VFill& D = d[j];
-  const uint64_t i0 = (uint64_t)(b - D.blk0) * kChunk;
-  const uint64_t i1 = min(i0 + kChunk, D.n);
+  const uint64_t ch = chunk_of<VFill>(D.n);
+  const uint64_t i0 = (uint64_t)(b - D.blk0) * ch;
+  const uint64_t i1 = min(i0 + ch, D.n);
   for (uint64_t i = i0 + threadIdx.x; i < i1; i += kBT) D.x[i] = 0.0;
 }
 
 // ---- Lanczos (ground state) ------------------------------------------------------------
 // vectors A, B per sector; at iteration k (parity p = k & 1) r = p ? B : A, q = p ? A : B.
 struct LJob {
+  static constexpr bool kElementwise = false;
   double* v[2];
   double* alpha;  // per-iteration scalars (device)
   double* beta;
@@ -358,6 +451,7 @@ __global__ void k_lz_next(int* __restrict__ kdev) {
 
 // eigenvector replay: q -= a r; (r, q) <- (q / b, -b r); psi += c r_new, for step i < len
 struct RJob {
+  static constexpr bool kElementwise = false;
   double* r;
   double* q;
   double* psi;
@@ -388,6 +482,7 @@ __global__ __launch_bounds__(kBT) void k_replay_batch(const RJob* __restrict__ d
 }
 
 struct PsiScale {
+  static constexpr bool kElementwise = true;
   double* psi;
   double c;
   uint64_t n;
@@ -397,8 +492,9 @@ __global__ __launch_bounds__(kBT) void k_psi_scale(const PsiScale* __restrict__ 
   const uint32_t b = blockIdx.x;
   const int j = find_job(d, nj, b);
   const PsiScale& D = d[j];
-  const uint64_t i0 = (uint64_t)(b - D.blk0) * kChunk;
-  const uint64_t i1 = min(i0 + kChunk, D.n);
+  const uint64_t ch = chunk_of<PsiScale>(D.n);
+  const uint64_t i0 = (uint64_t)(b - D.blk0) * ch;
+  const uint64_t i1 = min(i0 + ch, D.n);
   for (uint64_t i = i0 + threadIdx.x; i < i1; i += kBT) D.psi[i] *= D.c;
 }
 
@@ -414,7 +510,7 @@ struct Table {
   }
   void add(D v, uint64_t n) {
     v.blk0 = total;
-    total += nblocks(n);
+    total += blocks_of<D>(n);
     h.push_back(v);
   }
   // uploads the descriptors followed by their first blocks as a compact uint32 array
@@ -891,8 +987,7 @@ void band_lanczos_batch(const std::vector<qed_sector*>& S, const std::vector<con
     const int n = (int)TD.h.size();
     ensure(part, (size_t)total * kBM * sizeof(double));
     launches.push_back([&part, d, total, n] {
-      k_mdot_part<<<total, kBT, 0, stream()>>>(d, n, part.as<double>());
-      k_mdot_final<<<(n * kBM + 3) / 4, 256, 0, stream()>>>(d, n, part.as<double>());
+      launch_mdot(d, total, n, part.as<double>());
     });
   };
   auto run_maxpy = [&]() {
@@ -917,7 +1012,8 @@ void band_lanczos_batch(const std::vector<qed_sector*>& S, const std::vector<con
     const int n = (int)TT.h.size();
     ensure(part_tail, (size_t)total * sizeof(double));
     launches.push_back([&part_tail, d, total, n] {
-      k_mtail<<<total, kBT, 0, stream()>>>(d, n, part_tail.as<double>());
+      if (total <= kFewBlocks) k_mtail<4 * kBT><<<total, 4 * kBT, 0, stream()>>>(d, n, part_tail.as<double>());
+      else k_mtail<kBT><<<total, kBT, 0, stream()>>>(d, n, part_tail.as<double>());
       k_mtail_final<<<(n + 3) / 4, 256, 0, stream()>>>(d, n, part_tail.as<double>());
     });
   };
@@ -966,8 +1062,7 @@ void band_lanczos_batch(const std::vector<qed_sector*>& S, const std::vector<con
       MDot* d = stage1.put(TD);
       ensure(part, (size_t)TD.total * kBM * sizeof(double));
       stage1.flush();
-      k_mdot_part<<<TD.total, kBT, 0, stream()>>>(d, (int)TD.h.size(), part.as<double>());
-      k_mdot_final<<<((int)TD.h.size() * kBM + 3) / 4, 256, 0, stream()>>>(d, (int)TD.h.size(), part.as<double>());
+      launch_mdot(d, TD.total, (int)TD.h.size(), part.as<double>());
     }
     QED_HIP(hipMemcpyAsync(sch_all, sc_all.p, (size_t)nj * kSc * sizeof(double), hipMemcpyDeviceToHost, stream()));
     QED_HIP(hipStreamSynchronize(stream()));

@@ -68,3 +68,10 @@ def test_start_vectors_that_deflate_and_many_of_them(gpu_lib):
     big = 1j * np.array([1e4])
     E0, G = _instance_green(m, vals, "R0:N2:S0", big, "band_many")
     np.testing.assert_allclose(G[0] * big[0], np.eye(12), rtol=0, atol=1e-3)
+
+
+@pytest.mark.parametrize("n,nup,ndn", [(9, 5, 4), (10, 5, 5), (11, 5, 5)])
+def test_few_and_many_chunks(gpu_lib, n, nup, ndn):
+    """Sums over few chunks (14 and 52 of 2048 amplitudes in the two parts: vectors split over
+    blocks) and over many (180: one block per chunk), against the one-sector form as above"""
+    test_instance_green_function_matches_one_sector_form(gpu_lib, n, nup, ndn)
