@@ -117,6 +117,26 @@ def test_trivial_group_is_the_factorized_sector(gpu_lib):
     np.testing.assert_allclose(S.hv(x, y), F.hv(x, y), rtol=0, atol=1e-12)
 
 
+@pytest.mark.parametrize("L,nup,ndn", [(17, 2, 2), (16, 2, 2), (5, 1, 0), (2, 1, 1)])
+def test_product_over_all_pairs(gpu_lib, L, nup, ndn):
+    """A different hop between every two orbitals: 546 amplitudes (read from memory), 482 and
+    fewer (from LDS), lists of hops that end within and at a group of 8."""
+    from pyqcm_amd.sector import MixedSector, Sector
+    rng = np.random.default_rng(11)
+    m = O.ClusterModel(L)
+    t = rng.standard_normal((L, L))
+    m.add("t", "one-body", [(a + s * L, b + s * L, t[a, b]) for s in (0, 1) for a in range(L) for b in range(a + 1, L)])
+    m.add("U", "interaction", [(i, i + L, 1.0) for i in range(L)])
+    f = m.flat({"t": 1.0, "U": 3.0})
+    S = MixedSector(L, nup, ndn, f, L, np.zeros((0, L), np.int32), 0, False)
+    F = Sector(L, nup, ndn, f)
+    x, y = rng.standard_normal((2, F.dim))
+    h = F.hv(x, np.zeros(F.dim))
+    # two sums of at most 62 terms of the size of the result, in different orders
+    tol = 62 * np.finfo(float).eps * (1.0 + np.abs(t).max() * 62 * np.abs(x).max())
+    np.testing.assert_allclose(S.hv(x, y), y + h, rtol=0, atol=tol)
+
+
 def test_plaquette_8bath_ground_state_in_irrep_0(gpu_lib, golden):
     """tests/test_diagonalization/S_format.ref: new_cluster_model('clus', 4, 8,
     generators=[[2,1,4,3,0,0,0,0,2,2,2,2],[3,4,1,2,0,0,2,2,0,0,2,2]], bath_irrep=True);
