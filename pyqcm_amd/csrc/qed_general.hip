@@ -14,7 +14,8 @@
 // operator stores for (c, r); with Jordan-Wigner operators that is 2 v (c_r c_c + h.c.).
 //
 // Device layout: the sorted states (8 B each); the product is a gather per basis state:
-// each term applied to the state's bits, the target located by binary search.
+// each term applied to the state's bits, the target located by rank tables, or by binary
+// search where a sector has none.
 #include <algorithm>
 #include <cmath>
 #include <memory>
@@ -28,13 +29,25 @@ namespace qed {
 namespace {
 
 constexpr int kMaxOrbGeneral = 24;  // orbitals per spin
+constexpr int kTermGroup = 8;       // terms whose loads are in flight together
+// orbitals per spin up to which the ranks are kept in LDS: 16 KB as 16-bit words, so that
+// eight workgroups still share a CU; the tables of more orbitals are read from memory
+constexpr int kLdsRank = 13;
 
-// one term of the product: kind 0 one-body hop or diagonal (c^+_r c_c, both directions
-// listed), 1 density-density n_r n_c, 2 pair w (c_r c_c + h.c.); r, c as 64-bit masks
-struct GTerm {
-  uint64_t mr, mc;
+// An off-diagonal term exchanges the occupation of two orbitals, m: it takes a state s to
+// s ^ m, with the sign of the bits between the two. A hop and its conjugate are one term (a
+// state takes part in one of them, where one of the two orbitals is filled), as are a pair
+// and its conjugate (where both or neither are).
+struct GHop {
+  uint64_t m, inside;
   double w;
-  int kind;
+  uint64_t one;  // 1: acts on states with one of the two filled, 0: on the others
+};
+
+// a diagonal term: w where all of m is filled
+struct GDiag {
+  uint64_t m;
+  double w;
 };
 
 // Index of a state without a search, when every down word's allowed up words are those of
@@ -53,8 +66,11 @@ struct LocateTables {
 
 struct GeneralTables {
   DevBuf states;  // uint64, ascending
-  DevBuf terms;   // GTerm
-  int nterms = 0;
+  // off-diagonal terms within the up word, within the down word and others, each part
+  // padded to kTermGroup with terms that act on no state; then the diagonal ones
+  DevBuf hops, diags;
+  int end_up = 0, end_dn = 0, end_hop = 0, ndiag = 0;
+  int L = 0;
   std::vector<uint64_t> host_states;
   DevBuf prefix, rank, allowed;
   bool tabled = false;
@@ -88,51 +104,86 @@ __device__ __forceinline__ uint32_t locate(const LocateTables& T, const uint64_t
   return T.prefix[dn] + T.rank[up];
 }
 
-// parity of the bits of s strictly between the single-bit masks a and b
-__device__ __forceinline__ int between_parity(uint64_t s, uint64_t a, uint64_t b) {
+// the bits strictly between the single-bit masks a and b
+uint64_t between(uint64_t a, uint64_t b) {
   const uint64_t lo = a < b ? a : b, hi = a < b ? b : a;
-  const uint64_t inside = (hi - 1ull) & ~((lo << 1) - 1ull);
-  return __popcll(s & inside) & 1;
+  return (hi - 1ull) & ~((lo << 1) - 1ull);
+}
+
+enum Look { kSearch, kTables, kTablesLds };  // how a target is located
+
+// kTermGroup terms: PART 0 the up word only, 1 the down word only, 2 any. base + rank[up]
+// and prefix[dn] + rk are the index of state (up, dn).
+template <int LOOK, int PART>
+__device__ __forceinline__ void term_group(const GHop* __restrict__ h, const uint64_t* __restrict__ st, uint32_t n,
+                                           const LocateTables& loc, const uint16_t* ranks, uint64_t s, uint32_t I,
+                                           uint32_t base, uint32_t rk, const double* __restrict__ x, double& acc) {
+  uint32_t J[kTermGroup];
+  double xv[kTermGroup];
+#pragma unroll
+  for (int q = 0; q < kTermGroup; ++q) {
+    const uint64_t m = h[q].m, s2 = s ^ m;
+    const bool acts = (uint64_t)(__popcll(s & m) & 1) == h[q].one;
+    uint32_t t = n;
+    if constexpr (LOOK == kSearch) {
+      if (acts) t = find_state(st, n, s2);
+    } else {
+      const uint32_t up = (uint32_t)s2, dn = (uint32_t)(s2 >> 32);
+      if constexpr (PART == 0) {
+        t = base + (LOOK == kTablesLds ? (uint32_t)ranks[up] : loc.rank[up]);
+      } else if constexpr (PART == 1) {
+        t = loc.prefix[dn] + rk;
+      } else {
+        const bool in = (loc.allowed[__popc(dn)] >> __popc(up)) & 1ull;
+        t = in ? loc.prefix[dn] + (LOOK == kTablesLds ? (uint32_t)ranks[up] : loc.rank[up]) : n;
+      }
+      if (!acts) t = n;
+    }
+    J[q] = t;
+  }
+#pragma unroll
+  for (int q = 0; q < kTermGroup; ++q) xv[q] = x[J[q] == n ? I : J[q]];
+#pragma unroll
+  for (int q = 0; q < kTermGroup; ++q) {
+    const double w = (__popcll(s & h[q].inside) & 1) ? -h[q].w : h[q].w;
+    const double t = fma(w, xv[q], acc);
+    acc = J[q] == n ? acc : t;
+  }
 }
 
 // y[I] += sum_J H[I, J] x[J]: every term applied to basis state I gives <J|T|I>, which is
-// H[I, J] since the term list is Hermitian and real
-template <int EP>
+// H[I, J] since the terms are Hermitian and real. Bound by the latency of a term's chain of
+// loads (rank, x) and by its integer work, not by bytes (24 per state): the loads of eight
+// terms are in flight together, a term within one word looks up that word only, and the
+// ranks are kept in LDS. 4 sites + 8 bath orbitals with pairing (2.7 million states): 615 us
+// with one term and one direction of it at a time, 226 us.
+template <int EP, int LOOK>
 __global__ __launch_bounds__(256) void k_hv_general(const uint64_t* __restrict__ st, uint32_t n, LocateTables loc,
-                                                    const GTerm* __restrict__ terms, int nterms,
+                                                    int L, const GHop* __restrict__ hops, int end_up, int end_dn,
+                                                    int end_hop, const GDiag* __restrict__ diags, int ndiag,
                                                     const double* __restrict__ x, double* __restrict__ y, LzStep lz) {
+  __shared__ uint16_t ranks[LOOK == kTablesLds ? 1 << kLdsRank : 1];
+  if constexpr (LOOK == kTablesLds) {
+    for (uint32_t i = threadIdx.x; i < (1u << L); i += 256) ranks[i] = (uint16_t)loc.rank[i];
+    __syncthreads();
+  }
   double2 sc = make_double2(0.0, 0.0);
   double dot = 0.0;
   if constexpr (EP != 0) sc = lz_scalars(lz);
   for (uint32_t I = blockIdx.x * blockDim.x + threadIdx.x; I < n; I += gridDim.x * blockDim.x) {
     const uint64_t s = st[I];
     double diag = 0.0, acc = 0.0;
-    for (int k = 0; k < nterms; ++k) {
-      const GTerm t = terms[k];
-      if (t.kind == 1) {
-        if ((s & t.mr) && (s & t.mc)) diag += t.w;
-      } else if (t.kind == 0) {
-        if (t.mr == t.mc) {
-          if (s & t.mr) diag += t.w;
-        } else if ((s & t.mc) && !(s & t.mr)) {
-          const uint64_t s2 = s - t.mc + t.mr;
-          const uint32_t J = locate(loc, st, n, s2);
-          if (J == n) continue;
-          const double v = t.w * x[J];
-          acc += between_parity(s, t.mr, t.mc) ? -v : v;
-        }
-      } else {
-        // <J| c_r c_c |I> = -(-1)^(bits between) when I holds both, and the same for the
-        // conjugate when I holds neither (the bits between are those of I in both cases)
-        const bool both = (s & t.mr) && (s & t.mc), none = !(s & t.mr) && !(s & t.mc);
-        if (!both && !none) continue;
-        const uint64_t s2 = both ? s - t.mr - t.mc : s + t.mr + t.mc;
-        const uint32_t J = locate(loc, st, n, s2);
-        if (J == n) continue;
-        const double v = t.w * x[J];
-        acc += between_parity(s, t.mr, t.mc) ? v : -v;
-      }
-    }
+    for (int k = 0; k < ndiag; ++k)
+      if ((s & diags[k].m) == diags[k].m) diag += diags[k].w;
+    uint32_t rk = 0;
+    if constexpr (LOOK == kTablesLds) rk = ranks[(uint32_t)s];
+    if constexpr (LOOK == kTables) rk = loc.rank[(uint32_t)s];
+    for (int k = 0; k < end_up; k += kTermGroup)
+      term_group<LOOK, 0>(hops + k, st, n, loc, ranks, s, I, I - rk, rk, x, acc);
+    for (int k = end_up; k < end_dn; k += kTermGroup)
+      term_group<LOOK, 1>(hops + k, st, n, loc, ranks, s, I, I - rk, rk, x, acc);
+    for (int k = end_dn; k < end_hop; k += kTermGroup)
+      term_group<LOOK, 2>(hops + k, st, n, loc, ranks, s, I, I - rk, rk, x, acc);
     const double xi = x[I];
     lz_update<EP>(lz, sc, diag * xi + acc, xi, y + I, EP == 2 ? lz.psi + I : nullptr, dot);
   }
@@ -167,19 +218,13 @@ __global__ __launch_bounds__(256) void k_general_apply(const uint64_t* __restric
 // d[I] += H[I, I]: the one-body diagonal and density-density terms (no hop or pair term
 // maps a state to itself)
 __global__ __launch_bounds__(256) void k_diag_general(const uint64_t* __restrict__ st, uint32_t n,
-                                                      const GTerm* __restrict__ terms, int nterms,
+                                                      const GDiag* __restrict__ diags, int ndiag,
                                                       double* __restrict__ d) {
   for (uint32_t I = blockIdx.x * blockDim.x + threadIdx.x; I < n; I += gridDim.x * blockDim.x) {
     const uint64_t s = st[I];
     double acc = 0.0;
-    for (int k = 0; k < nterms; ++k) {
-      const GTerm t = terms[k];
-      if (t.kind == 1) {
-        if ((s & t.mr) && (s & t.mc)) acc += t.w;
-      } else if (t.kind == 0 && t.mr == t.mc) {
-        if (s & t.mr) acc += t.w;
-      }
-    }
+    for (int k = 0; k < ndiag; ++k)
+      if ((s & diags[k].m) == diags[k].m) acc += diags[k].w;
     d[I] += acc;
   }
 }
@@ -191,11 +236,16 @@ uint32_t grid_of(uint64_t n) { return (uint32_t)std::min<uint64_t>(std::max<uint
 template <int EP>
 static int launch_general(const qed_sector& s, const double* x, double* y, int variant, const LzStep& L) {
   auto T = std::static_pointer_cast<GeneralTables>(s.general);
-  const uint32_t n = (uint32_t)s.D, grid = grid_of(n);
+  const uint32_t n = (uint32_t)s.D;
   if (n == 0) return 0;
-  LocateTables loc = T->loc();
-  if (variant == 0) loc.tabled = 0;  // the binary search (reference form of the lookup)
-  k_hv_general<EP><<<grid, 256, 0, stream()>>>(T->states.as<uint64_t>(), n, loc, T->terms.as<GTerm>(), T->nterms, x, y, L);
+  const LocateTables loc = T->loc();
+  // variant 0: the binary search (reference form of the lookup)
+  const bool tabled = loc.tabled && variant != 0, lds = tabled && T->L <= kLdsRank;
+  // ranks in LDS: eight workgroups per CU fill their tables once
+  const uint32_t grid = lds ? std::min(grid_of(n), (uint32_t)device_cu_count() * 8u) : grid_of(n);
+  auto k = !tabled ? k_hv_general<EP, kSearch> : lds ? k_hv_general<EP, kTablesLds> : k_hv_general<EP, kTables>;
+  k<<<grid, 256, 0, stream()>>>(T->states.as<uint64_t>(), n, loc, T->L, T->hops.as<GHop>(), T->end_up, T->end_dn,
+                                T->end_hop, T->diags.as<GDiag>(), T->ndiag, x, y, L);
   QED_HIP(hipGetLastError());
   return (int)grid;
 }
@@ -212,7 +262,7 @@ void diag_general(const qed_sector& s, double* d) {
   auto T = std::static_pointer_cast<GeneralTables>(s.general);
   const uint32_t n = (uint32_t)s.D;
   if (n == 0) return;
-  k_diag_general<<<grid_of(n), 256, 0, stream()>>>(T->states.as<uint64_t>(), n, T->terms.as<GTerm>(), T->nterms, d);
+  k_diag_general<<<grid_of(n), 256, 0, stream()>>>(T->states.as<uint64_t>(), n, T->diags.as<GDiag>(), T->ndiag, d);
   QED_HIP(hipGetLastError());
 }
 
@@ -291,7 +341,14 @@ int qed_general_sector_create(int L, int npairs, const int* pairs, int n_ops, co
       T->tabled = true;
     }
     // the terms
-    std::vector<GTerm> terms;
+    std::vector<GHop> part[3];
+    std::vector<GDiag> diags;
+    auto add_hop = [&](uint64_t mr, uint64_t mc, double w, uint64_t one) {
+      const uint64_t m = mr | mc;
+      const int p = !(m >> 32) ? 0 : !(m & 0xffffffffull) ? 1 : 2;
+      // (a pair within one word changes its particle number: the general lookup)
+      part[one ? p : 2].push_back({m, between(mr, mc), w, one});
+    };
     size_t off = 0;
     for (int o = 0; o < n_ops; ++o) {
       const double z = coefs[o];
@@ -303,27 +360,36 @@ int qed_general_sector_create(int L, int npairs, const int* pairs, int n_ops, co
         const uint64_t mr = orbital_mask(r, L), mc = orbital_mask(c, L);
         if (types[o] == 0) {
           // one_body_operator lists (r, c, v) and (c, r, v) for r < c (one_body_operator.hpp:70-76)
-          if (r == c) {
-            terms.push_back({mr, mr, v, 0});
-          } else if (r < c) {
-            terms.push_back({mr, mc, v, 0});
-            terms.push_back({mc, mr, v, 0});
-          }
+          if (r == c) diags.push_back({mr, v});
+          else if (r < c) add_hop(mr, mc, v, 1);
         } else if (types[o] == 1) {
-          terms.push_back({mr, mc, v, 1});
+          diags.push_back({mr | mc, v});
         } else if (types[o] == 2) {
-          if (r < c) terms.push_back({mr, mc, 2.0 * v, 2});
+          // <J| c_r c_c |I> = -(-1)^(bits between) when I holds both, and the same for the
+          // conjugate when I holds neither (the bits between are those of I in both cases)
+          if (r < c) add_hop(mr, mc, -2.0 * v, 0);
         } else {
           fail("unknown operator type");
         }
       }
     }
-    T->nterms = (int)terms.size();
+    std::vector<GHop> hops;
+    int* end[3] = {&T->end_up, &T->end_dn, &T->end_hop};
+    for (int p = 0; p < 3; ++p) {
+      hops.insert(hops.end(), part[p].begin(), part[p].end());
+      while (hops.size() % kTermGroup) hops.push_back({0, 0, 0.0, 1});
+      *end[p] = (int)hops.size();
+    }
+    T->ndiag = (int)diags.size();
+    T->L = L;
     T->states.alloc(std::max<uint64_t>(1, D) * 8);
-    T->terms.alloc(std::max<size_t>(1, terms.size()) * sizeof(GTerm));
+    T->hops.alloc(std::max<size_t>(1, hops.size()) * sizeof(GHop));
+    T->diags.alloc(std::max<size_t>(1, diags.size()) * sizeof(GDiag));
     if (D) QED_HIP(hipMemcpyAsync(T->states.p, T->host_states.data(), D * 8, hipMemcpyHostToDevice, stream()));
-    if (!terms.empty())
-      QED_HIP(hipMemcpyAsync(T->terms.p, terms.data(), terms.size() * sizeof(GTerm), hipMemcpyHostToDevice, stream()));
+    if (!hops.empty())
+      QED_HIP(hipMemcpyAsync(T->hops.p, hops.data(), hops.size() * sizeof(GHop), hipMemcpyHostToDevice, stream()));
+    if (!diags.empty())
+      QED_HIP(hipMemcpyAsync(T->diags.p, diags.data(), diags.size() * sizeof(GDiag), hipMemcpyHostToDevice, stream()));
     QED_HIP(hipStreamSynchronize(stream()));
     auto s = std::make_unique<qed_sector>();
     s->L = L;

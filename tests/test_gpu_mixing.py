@@ -213,6 +213,63 @@ def test_general_sector_diagonal_and_davidson(gpu_lib, case):
     S.close()
 
 
+def _apply(s, ops):
+    """ops = (orbital, creates) right to left on the Fock label s: (label, sign) or None"""
+    sign = 1.0
+    for o, creates in reversed(ops):
+        if ((s >> o) & 1) == creates:
+            return None
+        sign *= (-1.0) ** bin(s & ((1 << o) - 1)).count("1")
+        s ^= 1 << o
+    return s, sign
+
+
+def _hamiltonian(m, vals, states):
+    """H on the given labels by Jordan-Wigner strings (the dense oracle holds all 4^L)"""
+    idx = {s: i for i, s in enumerate(states)}
+    H = np.zeros((len(states), len(states)))
+    for name, op in m.operators.items():
+        for r, c, v in op.elements:
+            v = v * vals[name]
+            if op.kind == "interaction":
+                terms = [[(r, 1), (r, 0), (c, 1), (c, 0)]]
+            elif op.kind == "one-body":
+                terms = [[(r, 1), (c, 0)]] + ([[(c, 1), (r, 0)]] if r != c else [])
+            else:
+                terms = [[(r, 0), (c, 0)], [(c, 1), (r, 1)]]
+            for ops in terms:
+                for s, i in idx.items():
+                    t = _apply(s, ops)
+                    if t and t[0] in idx:
+                        H[idx[t[0]], i] += v * t[1]
+    return H
+
+
+@pytest.mark.parametrize("L,nsites", [(2, 2), (13, 4), (14, 4), (21, 3)])
+def test_general_lookups_by_size(gpu_lib, L, nsites):
+    """Ranks in LDS (up to 13 orbitals per spin), in memory (14 to 20), and the search (more),
+    with hops over every pair of nsites orbitals at both ends of the words, pairing across
+    and within the words: against the matrix of the Jordan-Wigner operators."""
+    from pyqcm_amd.sector import GeneralSector
+    rng = np.random.default_rng(5)
+    o = sorted({0, L - 1, L // 2, 1}) if nsites == 4 else list(range(L))[-nsites:]
+    m = O.ClusterModel(L)
+    t = rng.standard_normal((L, L))
+    m.add("t", "one-body", [(a + s * L, b + s * L, t[a, b]) for s in (0, 1) for a in o for b in o if a <= b])
+    m.add("U", "interaction", [(a, a + L, 1.0) for a in o])
+    m.add("D", "anomalous", [(a, b + L, t[b, a]) for a in o for b in o])
+    m.add("P", "anomalous", [(o[0], o[-1], 0.4), (o[0] + L, o[-1] + L, 0.7)])
+    vals = {"t": 1.0, "U": 2.0, "D": 0.5, "P": 1.0}
+    pairs = [(0, 0), (1, 1)] if L > 2 else [(0, 0), (2, 0), (0, 2), (1, 1), (2, 2)]
+    S = GeneralSector(L, pairs, _device_flat(m, vals))
+    H = _hamiltonian(m, vals, [int(v) for v in O.block_states(L, pairs)])
+    x, y = rng.standard_normal((2, S.dim))
+    # a row has at most 2 * 4 * 4 terms on either side; each product and sum rounds once
+    tol = 64 * np.finfo(float).eps * (np.abs(H) @ np.abs(x) + np.abs(y) + 1.0)
+    assert np.all(np.abs(S.hv(x, y) - (y + H @ x)) <= tol)
+    S.close()
+
+
 def test_general_nambu_plaquette_8bath_sector(gpu_lib):
     """The 2x2 plaquette + 8 bath orbitals with d-wave pairing, Nambu sector S = 0
     (D = C(24, 12) = 2,704,156): the rank-table product is bit-identical to the binary
