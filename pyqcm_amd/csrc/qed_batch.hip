@@ -3,7 +3,7 @@
 // them instead of one per sector.
 //
 //  * Ground state: Lanczos for all sectors in lockstep. Each iteration is a fixed kernel
-//    sequence (batched H.v, fused dot, fused axpy+norm) driven by a device-side
+//    sequence (batched H.v with the step's update and dot in it, axpy+norm) driven by a device-side
 //    iteration counter; two iterations (both parities of the vector rotation) are
 //    captured once in a hipGraph and replayed chunk by chunk. The recurrence scalars stay
 //    on the device; after each chunk the host reads them, applies the stopping test of
@@ -337,148 +337,88 @@ __global__ __launch_bounds__(kBT) void k_fill0(const VFill* __restrict__ d, int 
 }
 
 // ---- Lanczos (ground state) ------------------------------------------------------------
-// vectors A, B per sector; at iteration k (parity p = k & 1) r = p ? B : A, q = p ? A : B.
+// Unnormalized vectors w_k = beta_{k-1} v_k in A, B per sector, at iteration k (parity
+// p = k & 1) w_k in v[p]. The product's epilogue (HvBatchStep) makes
+// y = (H w_k) / beta_{k-1} - (beta_{k-1} / beta_{k-2}) w_{k-1} in v[p ^ 1] and the parts of
+// <w_k, y>; alpha and beta are one wavefront per sector, w_{k+1} = y - (alpha_k /
+// beta_{k-1}) w_k one pass. (The normalized recurrence took a scaling and a dot pass more,
+// 124 of 700 us for the sectors of 16 plaquettes with 8 bath orbitals, and its replay a
+// pass of 116 us; the 16 problems in all 1.514 -> 1.479 s.) The row form of the product at
+// all sizes: the tiled one, in two passes, has no place for the update.
 struct LJob {
   static constexpr bool kElementwise = false;
   double* v[2];
   double* alpha;  // per-iteration scalars (device)
   double* beta;
+  uint32_t row0, rows;  // this sector's rows (tiles) in the batched product
   uint64_t n;
   uint32_t blk0;
 };
 
-// k > 0: r /= beta[k-1]; q *= -beta[k-1]
-__global__ __launch_bounds__(kBT) void k_lz_scal(const LJob* __restrict__ d, int nj, int parity,
-                                                 const int* __restrict__ kdev,
-                                                 const int* __restrict__ active) {
-  const int k = *kdev;
-  if (k == 0) return;
-  const uint32_t b = blockIdx.x;
-  const int j = find_job(d, nj, b);
-  if (!active[j]) return;
-  const LJob& D = d[j];
-  double* r = D.v[parity];
-  double* q = D.v[parity ^ 1];
-  const double bt = D.beta[k - 1];
-  // a breakdown (beta = 0: the Krylov space is exhausted) leaves zero vectors, not NaN
-  const double inv = bt != 0.0 ? 1.0 / bt : 0.0;
-  const uint64_t i0 = (uint64_t)(b - D.blk0) * kChunk;
-  const uint64_t i1 = min(i0 + kChunk, D.n);
-  for (uint64_t i = i0 + threadIdx.x; i < i1; i += kBT) {
-    r[i] *= inv;
-    q[i] *= -bt;
-  }
-}
-
-// partials of <r, q> (r = v_k, q = H v_k - beta v_{k-1})
-__global__ __launch_bounds__(kBT) void k_lz_dot(const LJob* __restrict__ d, int nj, int parity,
-                                                const int* __restrict__ active, double* __restrict__ part) {
-  __shared__ double red[kBT / 64];
-  const uint32_t b = blockIdx.x;
-  const int j = find_job(d, nj, b);
-  const LJob& D = d[j];
-  double s = 0.0;
-  if (active[j]) {
-    const double* r = D.v[parity];
-    const double* q = D.v[parity ^ 1];
-    const uint64_t i0 = (uint64_t)(b - D.blk0) * kChunk;
-    const uint64_t i1 = min(i0 + kChunk, D.n);
-    for (uint64_t i = i0 + threadIdx.x; i < i1; i += kBT) s += r[i] * q[i];
-  }
-  s = block_sum(s, red);
-  if (threadIdx.x == 0) part[b] = s;
-}
-
-// sum of one job's block partials: one wavefront per job, lane-strided, fixed-order wave sum
-__device__ __forceinline__ double job_partial_sum(const LJob& D, const double* __restrict__ part, int lane) {
-  const uint32_t nb = nblocks(D.n);
-  double s = 0.0;
-  for (uint32_t b = lane; b < nb; b += 64) s += part[D.blk0 + b];
-  return wave_sum(s);
-}
-
-// alpha[k] = sum of the partials
+// alpha[k] from the product's parts; ca = -alpha / beta_{k-1}
 __global__ void k_lz_alpha(const LJob* __restrict__ d, int nj, const int* __restrict__ kdev,
-                           const int* __restrict__ active, const double* __restrict__ part) {
+                           const int* __restrict__ active, const double* __restrict__ part,
+                           const double2* __restrict__ sc, double* __restrict__ ca) {
   const int j = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
   const int lane = threadIdx.x & 63;
   if (j >= nj || !active[j]) return;
   const LJob& D = d[j];
-  const double s = job_partial_sum(D, part, lane);
-  if (lane == 0) D.alpha[*kdev] = s;
+  double s = 0.0;
+  for (uint32_t r = lane; r < D.rows; r += 64) s += part[D.row0 + r];
+  s = wave_sum(s);
+  if (lane == 0) {
+    const double a = s * sc[j].x;
+    D.alpha[*kdev] = a;
+    ca[j] = -a * sc[j].x;
+  }
 }
 
-// q -= alpha[k] r, partials of |q|^2
+// y += ca w, parts of |y|^2
 __global__ __launch_bounds__(kBT) void k_lz_axpy(const LJob* __restrict__ d, int nj, int parity,
-                                                 const int* __restrict__ kdev,
-                                                 const int* __restrict__ active,
+                                                 const int* __restrict__ active, const double* __restrict__ ca,
                                                  double* __restrict__ part) {
   __shared__ double red[kBT / 64];
   const uint32_t b = blockIdx.x;
   const int j = find_job(d, nj, b);
   const LJob& D = d[j];
+  if (!active[j]) return;
   double s = 0.0;
-  if (active[j]) {
-    const double a = D.alpha[*kdev];
-    const double* r = D.v[parity];
-    double* q = D.v[parity ^ 1];
-    const uint64_t i0 = (uint64_t)(b - D.blk0) * kChunk;
-    const uint64_t i1 = min(i0 + kChunk, D.n);
-    for (uint64_t i = i0 + threadIdx.x; i < i1; i += kBT) {
-      const double v = q[i] - a * r[i];
-      q[i] = v;
-      s += v * v;
-    }
+  const double a = ca[j];
+  const double* r = D.v[parity];
+  double* q = D.v[parity ^ 1];
+  const uint64_t i0 = (uint64_t)(b - D.blk0) * kChunk;
+  const uint64_t i1 = min(i0 + kChunk, D.n);
+  for (uint64_t i = i0 + threadIdx.x; i < i1; i += kBT) {
+    const double v = q[i] + a * r[i];
+    q[i] = v;
+    s += v * v;
   }
   s = block_sum(s, red);
   if (threadIdx.x == 0) part[b] = s;
 }
 
-// beta[k] = sqrt(sum of partials)
+// beta[k] = sqrt(sum of the parts), and the next product's scalars (a vanishing beta, an
+// exhausted Krylov space, leaves zero vectors)
 __global__ void k_lz_beta(const LJob* __restrict__ d, int nj, const int* __restrict__ kdev,
-                          const int* __restrict__ active, const double* __restrict__ part) {
+                          const int* __restrict__ active, const double* __restrict__ part,
+                          double2* __restrict__ sc) {
   const int j = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
   const int lane = threadIdx.x & 63;
   if (j >= nj || !active[j]) return;
   const LJob& D = d[j];
-  const double s = job_partial_sum(D, part, lane);
-  if (lane == 0) D.beta[*kdev] = std::sqrt(s);
+  const uint32_t nb = nblocks(D.n);
+  double s = 0.0;
+  for (uint32_t b = lane; b < nb; b += 64) s += part[D.blk0 + b];
+  s = wave_sum(s);
+  if (lane == 0) {
+    const double b = std::sqrt(s);
+    D.beta[*kdev] = b;
+    sc[j] = make_double2(lz_inv(b), -b * sc[j].x);
+  }
 }
 
 __global__ void k_lz_next(int* __restrict__ kdev) {
   if (threadIdx.x == 0) *kdev = *kdev + 1;
-}
-
-// eigenvector replay: q -= a r; (r, q) <- (q / b, -b r); psi += c r_new, for step i < len
-struct RJob {
-  static constexpr bool kElementwise = false;
-  double* r;
-  double* q;
-  double* psi;
-  const double* alpha;  // device, len
-  const double* beta;
-  const double* evec;
-  int len;
-  uint64_t n;
-  uint32_t blk0;
-};
-
-__global__ __launch_bounds__(kBT) void k_replay_batch(const RJob* __restrict__ d, int nj, int i) {
-  const uint32_t b = blockIdx.x;
-  const int j = find_job(d, nj, b);
-  const RJob& D = d[j];
-  if (i >= D.len) return;
-  const double a = D.alpha[i - 1], bt = D.beta[i - 1], c = D.evec[i];
-  const uint64_t i0 = (uint64_t)(b - D.blk0) * kChunk;
-  const uint64_t i1 = min(i0 + kChunk, D.n);
-  for (uint64_t t = i0 + threadIdx.x; t < i1; t += kBT) {
-    const double rv = D.r[t];
-    const double qv = D.q[t] - a * rv;
-    const double rn = qv / bt;
-    D.r[t] = rn;
-    D.q[t] = -bt * rv;
-    D.psi[t] += c * rn;
-  }
 }
 
 struct PsiScale {
@@ -685,12 +625,15 @@ void lanczos_gs_batch(const std::vector<qed_sector*>& S, const std::vector<doubl
   double* beta = alpha + (size_t)nj * ld;
   Table<LJob> T;
   Table<VFill> F;
+  uint32_t rows = 0;  // as hv_batch_prepare numbers them
   for (int j = 0; j < nj; ++j) {
     const uint64_t n = S[j]->D;
     A[j].reset(new DevBuf(n * 8));
     Bv[j].reset(new DevBuf(n * 8));
     QED_HIP(hipMemcpyAsync(A[j]->p, psi[j], n * 8, hipMemcpyDeviceToDevice, stream()));
-    T.add(LJob{{A[j]->as<double>(), Bv[j]->as<double>()}, alpha + (size_t)j * ld, beta + (size_t)j * ld, n, 0}, n);
+    T.add(LJob{{A[j]->as<double>(), Bv[j]->as<double>()}, alpha + (size_t)j * ld, beta + (size_t)j * ld, rows, S[j]->dd, n, 0},
+          n);
+    rows += S[j]->dd;
     F.add(VFill{Bv[j]->as<double>(), n, 0}, n);
   }
   LJob* dT = T.upload();
@@ -709,12 +652,15 @@ void lanczos_gs_batch(const std::vector<qed_sector*>& S, const std::vector<doubl
   hv_batch_upload(HB);
   std::vector<int> active(nj, 1);
   DevBuf dact((size_t)nj * sizeof(int)), dk(sizeof(int)), part((size_t)T.total * sizeof(double));
+  DevBuf rpart((size_t)std::max<uint32_t>(1, rows) * sizeof(double)), dca((size_t)nj * sizeof(double));
+  const std::vector<double2> sc0(nj, double2{1.0, 0.0});
+  DevBuf dsc = upload(sc0);
   QED_HIP(hipMemcpyAsync(dact.p, active.data(), nj * sizeof(int), hipMemcpyHostToDevice, stream()));
   const int zero = 0;
   QED_HIP(hipMemcpyAsync(dk.p, &zero, sizeof(int), hipMemcpyHostToDevice, stream()));
   // autotune the batched H.v on scratch vectors (results discarded)
   HvBatchConfig cfg;
-  if (!hv_batch_tuned(HB, cfg)) {
+  if (!hv_batch_tuned(HB, cfg, true)) {
     std::vector<std::unique_ptr<DevBuf>> sy(nj);
     HvBatch tb;
     hv_batch_prepare(tb, cs);
@@ -724,7 +670,7 @@ void lanczos_gs_batch(const std::vector<qed_sector*>& S, const std::vector<doubl
       tb.host[j].y[0] = tb.host[j].y[1] = sy[j]->as<double>();
     }
     hv_batch_upload(tb);
-    cfg = hv_batch_tune(tb, dact.as<int>());
+    cfg = hv_batch_tune(tb, dact.as<int>(), true);
     QED_HIP(hipStreamSynchronize(stream()));
   }
   if (stats) stats->hv_config = cfg;
@@ -732,13 +678,15 @@ void lanczos_gs_batch(const std::vector<qed_sector*>& S, const std::vector<doubl
   int* kd = dk.as<int>();
   double* pd = part.as<double>();
   const int nb1 = (nj + 3) / 4;  // one wavefront per job
+  HvBatchStep L;
+  L.kind = 1;
+  L.sc = dsc.as<double2>();
+  L.part = rpart.as<double>();
   auto iteration = [&](int parity) {
-    k_lz_scal<<<T.total, kBT, 0, stream()>>>(dT, nj, parity, kd, act);
-    hv_batch(HB, cfg, parity, act);
-    k_lz_dot<<<T.total, kBT, 0, stream()>>>(dT, nj, parity, act, pd);
-    k_lz_alpha<<<nb1, 256, 0, stream()>>>(dT, nj, kd, act, pd);
-    k_lz_axpy<<<T.total, kBT, 0, stream()>>>(dT, nj, parity, kd, act, pd);
-    k_lz_beta<<<nb1, 256, 0, stream()>>>(dT, nj, kd, act, pd);
+    hv_batch_step(HB, cfg, parity, act, L);
+    k_lz_alpha<<<nb1, 256, 0, stream()>>>(dT, nj, kd, act, rpart.as<double>(), dsc.as<double2>(), dca.as<double>());
+    k_lz_axpy<<<T.total, kBT, 0, stream()>>>(dT, nj, parity, act, dca.as<double>(), pd);
+    k_lz_beta<<<nb1, 256, 0, stream()>>>(dT, nj, kd, act, pd, dsc.as<double2>());
     k_lz_next<<<1, 64, 0, stream()>>>(kd);
   };
   hipGraphExec_t exec = nullptr;
@@ -828,38 +776,41 @@ void lanczos_gs_batch(const std::vector<qed_sector*>& S, const std::vector<doubl
   if (stats) {
     stats->lanczos_iterations = k;
   }
-  // ground-state vectors: replay the recurrence with the stored scalars
+  // ground-state vectors: the recurrence again with the stored scalars, one launch per step
   int maxlen = 0;
   std::vector<DevBuf> ev_dev;
-  Table<RJob> R;
   Table<PsiScale> PS;
-  std::vector<int> ones(nj, 1);
+  std::vector<const double*> evp(nj);
+  std::vector<double*> psip(nj);
+  std::vector<int> len(nj), ones(nj, 1);
   for (int j = 0; j < nj; ++j) {
     niter[j] = done_at[j];
     const uint64_t n = S[j]->D;
     ev_dev.emplace_back(std::max<size_t>(1, evec[j].size()) * 8);
     if (!evec[j].empty())
       QED_HIP(hipMemcpyAsync(ev_dev.back().p, evec[j].data(), evec[j].size() * 8, hipMemcpyHostToDevice, stream()));
-    // r = start vector (copy kept in psi), q = 0, psi *= evec[0]
+    // A = start vector (copy kept in psi), B = 0, psi *= evec[0]
     QED_HIP(hipMemcpyAsync(A[j]->p, psi[j], n * 8, hipMemcpyDeviceToDevice, stream()));
-    R.add(RJob{A[j]->as<double>(), Bv[j]->as<double>(), psi[j], alpha + (size_t)j * ld, beta + (size_t)j * ld,
-               ev_dev.back().as<double>(), (int)evec[j].size(), n, 0},
-          n);
+    evp[j] = ev_dev.back().as<double>();
+    psip[j] = psi[j];
+    len[j] = (int)evec[j].size();
     PS.add(PsiScale{psi[j], evec[j].empty() ? 0.0 : evec[j][0], n, 0}, n);
-    maxlen = std::max(maxlen, (int)evec[j].size());
+    maxlen = std::max(maxlen, len[j]);
   }
   k_fill0<<<F.total, kBT, 0, stream()>>>(dF, nj);
   PsiScale* dPS = PS.upload();
   k_psi_scale<<<PS.total, kBT, 0, stream()>>>(dPS, nj);
-  RJob* dR = R.upload();
+  DevBuf devp = upload(evp), dpsi = upload(psip), dlen = upload(len);
   QED_HIP(hipMemcpyAsync(dact.p, ones.data(), nj * sizeof(int), hipMemcpyHostToDevice, stream()));
-  // replay H.v: x = r (A), y = q (B): parity 0 of HB
-  for (int i = 1; i < maxlen; ++i) {
-    for (int j = 0; j < nj; ++j) active[j] = i < (int)evec[j].size() ? 1 : 0;
-    QED_HIP(hipMemcpyAsync(dact.p, active.data(), nj * sizeof(int), hipMemcpyHostToDevice, stream()));
-    hv_batch(HB, cfg, 0, act);
-    k_replay_batch<<<R.total, kBT, 0, stream()>>>(dR, nj, i);
-  }
+  HvBatchStep P;
+  P.kind = 2;
+  P.alpha = alpha;
+  P.beta = beta;
+  P.ld = ld;
+  P.evec = devp.as<const double*>();
+  P.len = dlen.as<int>();
+  P.psi = dpsi.as<double*>();
+  for (P.i = 1; P.i < maxlen; ++P.i) hv_batch_step(HB, cfg, (P.i - 1) & 1, act, P);
   QED_HIP(hipGetLastError());
   QED_HIP(hipStreamSynchronize(stream()));
 }

@@ -17,6 +17,7 @@
 #include <mutex>
 #include <random>
 #include <thread>
+#include <type_traits>
 #include <atomic>
 
 #include "../../include/qed.h"
@@ -278,18 +279,42 @@ __global__ __launch_bounds__(BS) void k_hv_ell(HvView v, const uint32_t* __restr
 // it with a stride. Jobs whose active flag is 0 are skipped. Parity selects which of the
 // job's two vector pairs is (x, y), so that an alternating recurrence needs only two job
 // tables.
-template <int BS>
+template <int BS, int EP = 0>
 __global__ __launch_bounds__(BS) void k_hv_ell_batch(const HvJob* __restrict__ jobs, int njobs,
                                                      uint32_t ntiles, int parity,
                                                      const int* __restrict__ active,
-                                                     const uint32_t* __restrict__ tile_job) {
+                                                     const uint32_t* __restrict__ tile_job,
+                                                     HvBatchStep L = HvBatchStep{}) {
   extern __shared__ double smem[];
+  __shared__ double red[EP == 1 ? BS / 64 : 1];
   for (uint32_t t = blockIdx.x; t < ntiles; t += gridDim.x) {
     const int lo = (int)tile_job[t];  // job owning tile t (row0[lo] <= t < row0[lo + 1])
     const HvJob& J = jobs[lo];
-    if (active[lo]) {
-      ell_row<BS, true>(J.v, J.up_ell, J.Wu, J.dn_ell, J.Wd, J.x[parity], J.y[parity], t - J.row0,
-                        smem);
+    if (active[lo] && (EP != 2 || L.i < L.len[lo])) {
+      if constexpr (EP == 0) {
+        ell_row<BS, true>(J.v, J.up_ell, J.Wu, J.dn_ell, J.Wd, J.x[parity], J.y[parity], t - J.row0, smem);
+      } else {
+        LzStep lz;
+        double2 sc;
+        if constexpr (EP == 1) {
+          sc = L.sc[lo];
+        } else {
+          const double* al = L.alpha + (size_t)lo * L.ld;
+          const double* be = L.beta + (size_t)lo * L.ld;
+          const double b1 = L.i >= 2 ? be[L.i - 2] : 1.0, b2 = L.i >= 3 ? be[L.i - 3] : 1.0;
+          sc = make_double2(1.0 / b1, L.i >= 2 ? -b1 * (1.0 / b2) : 0.0);
+          lz.s2 = al[L.i - 1] * (1.0 / b1);
+          lz.c = L.evec[lo][L.i] / be[L.i - 1];
+          lz.psi = L.psi[lo];
+        }
+        double dot = 0.0;
+        ell_row<BS, true, EP>(J.v, J.up_ell, J.Wu, J.dn_ell, J.Wd, J.x[parity], J.y[parity], t - J.row0, smem, &lz, sc,
+                              &dot);
+        if constexpr (EP == 1) {
+          dot = block_sum(dot, red);
+          if (threadIdx.x == 0) L.part[t] = dot;
+        }
+      }
     }
     __syncthreads();
   }
@@ -1049,9 +1074,11 @@ HvBatchConfig hv_batch_tune(const HvBatch& B, const int* active, bool rows) {
   static std::once_flag once;
   std::call_once(once, [] {
     const int bytes = (int)lds_budget();
-    (void)hipFuncSetAttribute((const void*)k_hv_ell_batch<256>, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-    (void)hipFuncSetAttribute((const void*)k_hv_ell_batch<512>, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-    (void)hipFuncSetAttribute((const void*)k_hv_ell_batch<1024>, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+    for (const void* f : {(const void*)k_hv_ell_batch<256>, (const void*)k_hv_ell_batch<512>, (const void*)k_hv_ell_batch<1024>,
+                          (const void*)k_hv_ell_batch<256, 1>, (const void*)k_hv_ell_batch<512, 1>,
+                          (const void*)k_hv_ell_batch<1024, 1>, (const void*)k_hv_ell_batch<256, 2>,
+                          (const void*)k_hv_ell_batch<512, 2>, (const void*)k_hv_ell_batch<1024, 2>})
+      (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
   });
   const TuneKey key = tune_key(B, rows);
   auto it = tune_cache().find(key);
@@ -1091,6 +1118,20 @@ bool hv_batch_tuned(const HvBatch& B, HvBatchConfig& cfg, bool rows) {
   if (it == tune_cache().end()) return false;
   cfg = it->second;
   return true;
+}
+
+void hv_batch_step(const HvBatch& B, const HvBatchConfig& cfg, int parity, const int* active, const HvBatchStep& L) {
+  const uint32_t grid = cfg.grid ? std::min<uint32_t>(cfg.grid, B.ntiles) : B.ntiles;
+  const uint32_t* tj = B.tile_job.as<uint32_t>();
+  auto go = [&](auto bs) {
+    constexpr int BS = decltype(bs)::value;
+    if (L.kind == 1) k_hv_ell_batch<BS, 1><<<grid, BS, B.lds, stream()>>>(B.jobs, B.njobs, B.ntiles, parity, active, tj, L);
+    else k_hv_ell_batch<BS, 2><<<grid, BS, B.lds, stream()>>>(B.jobs, B.njobs, B.ntiles, parity, active, tj, L);
+  };
+  if (cfg.block == 1024) go(std::integral_constant<int, 1024>{});
+  else if (cfg.block == 512) go(std::integral_constant<int, 512>{});
+  else go(std::integral_constant<int, 256>{});
+  QED_HIP(hipGetLastError());
 }
 
 void hv_batch(const HvBatch& B, const HvBatchConfig& cfg, int parity, const int* active) {

@@ -114,6 +114,22 @@ struct HvJob {
   double* y[2];
 };
 
+// the Lanczos epilogue of a batched product (row form), per job
+struct HvBatchStep {
+  int kind = 0;               // as LzStep: 1 eigenvalue pass, 2 eigenvector pass
+  const double2* sc = nullptr;  // kind 1: s0, s1 of each job
+  double* part = nullptr;     //         parts of <x, y>, one per row (tile) of the batch
+  // kind 2: the recurrence's scalars of each job (ld per job), its Ritz vector and length;
+  // step i makes w_i
+  const double* alpha = nullptr;
+  const double* beta = nullptr;
+  int ld = 0;
+  const double* const* evec = nullptr;
+  const int* len = nullptr;
+  double* const* psi = nullptr;
+  int i = 0;
+};
+
 struct HvBatch {
   std::vector<HvJob> host;  // fill x / y, then hv_batch_upload
   DevBuf dev;
@@ -147,6 +163,8 @@ HvBatchConfig hv_batch_tune(const HvBatch& B, const int* active, bool rows = fal
 // the tuned launch shape of such a batch, if there is one
 bool hv_batch_tuned(const HvBatch& B, HvBatchConfig& cfg, bool rows = false);
 void hv_batch(const HvBatch& B, const HvBatchConfig& cfg, int parity, const int* active);
+// one Lanczos step of every active job (row form)
+void hv_batch_step(const HvBatch& B, const HvBatchConfig& cfg, int parity, const int* active, const HvBatchStep& L);
 
 struct BatchStats {
   HvBatchConfig hv_config;

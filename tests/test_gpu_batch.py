@@ -252,3 +252,35 @@ def test_batch_solve_matches_oracle(gpu_lib):
             if inst == 0 and z.imag < 1.0:
                 continue  # band Lanczos G not converged there (see above)
             assert err <= 1e-8 * max(1.0, np.abs(ref).max())
+
+
+@pytest.mark.parametrize("graph", [True, False])
+def test_batch_lanczos_steps_of_uneven_jobs(gpu_lib, graph):
+    """Sectors of 400 to 4900 states in one batch (rows of 20 to 70 amplitudes, fewer than
+    a workgroup's threads; runs that end at different steps; chunks of 3 steps), against the
+    same instances one at a time and the dense spectrum of the smallest. The ground states
+    converge to 1e-12 of beta, their energies to its square: 1e-10 covers the sums."""
+    from oracle import oracle as O
+    from pyqcm_amd import qcm
+    from tests import models as TM
+    from tests.test_gpu_mcf import register, with_sites
+    qcm.set_global_parameter("max_dim_full", 64)
+    try:
+        cases = [(6, 0), (8, 0), (7, 1), (6, 2)]
+        pair = []
+        for n, S in cases:
+            m, vals = TM.chain(n, tp=-0.3, U=4.0, mu=1.7)
+            sec = "R0:N%d:S%d" % (n, S)
+            pair.append([register(with_sites(m, n), vals, sec) for _ in range(2)])
+        E = [qcm.ground_state_solve(a)[0] for a, _ in pair]
+        qcm.batch_solve([b for _, b in pair], graph=graph, chunk=3)
+        for (a, b), e in zip(pair, E):
+            assert abs(qcm.ground_state_solve(b)[0] - e) <= 1e-10 * abs(e)
+            z = np.array([0.5j, 2.0j])
+            np.testing.assert_allclose(qcm.Green_function(z, 0, b), qcm.Green_function(z, 0, a), rtol=0, atol=1e-7)
+        m, vals = TM.chain(6, tp=-0.3, U=4.0, mu=1.7)
+        H, _ = O.dense_hamiltonian(m, vals, 3, 3)
+        ref = np.linalg.eigvalsh(H)[0]
+        assert abs(E[0] - ref) <= 1e-10 * abs(ref)
+    finally:
+        qcm.set_global_parameter("max_dim_full", 256)
