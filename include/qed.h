@@ -140,12 +140,11 @@ int qed_lanczos_gs(qed_sector* s, double accur, int max_iter, double* psi_dev, d
 /* qed_lanczos_gs without device allocation. No counterpart in the reference: for callers
  * that cannot allocate device memory (tight solver loops, harnesses that forbid hipMalloc
  * after start-up). Same arguments and results as qed_lanczos_gs; the two recurrence
- * vectors and the reduction partials live in a fixed device array of the library (one
+ * vectors and the parts and scalars of its steps live in a fixed device array of the library (one
  * per GPU, 34.1 MB, held until the process ends), so the sector dimension is limited to
  * 2^21 = 2,097,152: a larger sector fails with an error and nothing is launched. All calls
  * on one GPU share that array, which keeps the last call's contents; the library lock
- * serializes the calls of one process, and calls that overlap on one GPU otherwise race.
- * A sector set to a split-halves H.v variant takes the default row kernel here. */
+ * serializes the calls of one process, and calls that overlap on one GPU otherwise race. */
 int qed_lanczos_gs_noalloc(qed_sector* s, double accur, int max_iter, double* psi_dev, double* E0,
                            int* niter, double* alpha, double* beta);
 

@@ -174,8 +174,8 @@ __device__ __forceinline__ uint32_t code_target(uint32_t c, const uint32_t* __re
 // three loads (table, code, x), and their latency and the vector units' address rate bound
 // the kernel: kHops chains are in flight at a time, and the amplitudes are read from LDS.
 // Packed orbit lengths are powers of two, so that sqrt(length(I) / length(J)) is one of 16
-// values and not a division and a square root per hop. 2x7 sites, half filled, one mirror
-// (5.9 million states): 329 us one hop at a time, 217 us by groups, 174 us with the
+// values and not a division and a square root per hop. 2x7 sites, half filled, two mirrors
+// (2,945,056 states): 329 us one hop at a time, 217 us by groups, 174 us with the
 // amplitudes in LDS.
 constexpr int kHops = 8;  // the tables' widths are multiples of it
 // amplitudes (both spins) held in LDS, 4 KB: up to 127 bonds per spin, all pairs of 16
