@@ -18,7 +18,7 @@ Prints one JSON line (rank 0, N=1):
   ground_state the workload's Lanczos ground state (E0, iterations, seconds) on the
                factorized sector and on irrep 0 of the cluster's two-mirror basis
   cpt          the CPT k-sum of the 3x4 cluster (128^2 k-points x 512 frequencies), device
-               time and FP64 rate on 41.5 kflop per (k, w)
+               time and FP64 rate on 13.8 kflop per (k, w)
   cdmft        the second half of the metric: converged CDMFT solves per second on the
                2x2 plaquette + 8 bath orbitals (16 bath parameters), n seeded points
                (U ~ U[0.5, 12], mu ~ U[0, U], t' ~ U[-0.5, 0.5]), solved by the batched
@@ -313,14 +313,14 @@ def traffic_from_profile():
 
 
 PEAK_FP64_TFLOPS = 78.6
-CPT_FLOP_PER_POINT = 41.5e3  # two complex 12 x 12 products and one LU inverse per (k, w)
+CPT_FLOP_PER_POINT = 8 * 12 ** 3  # one complex 12 x 12 inverse, (Gc^-1 - V)^-1, per (k, w)
 
 
 def cpt_leg(side=128, nw=512, reps=3, cpu=True):
     """CPT spectral trace on the 3x4 Hubbard cluster (t=1, U=8, mu=4, sector N=12 S=0,
     D = 853,776): G_cpt = G_c (1 - V(k) G_c)^-1 over a side^2 k-grid (k_i = (i+0.5)/side
     in the superdual basis) and nw frequencies w = linspace(-10, 10) + 0.1i, one device
-    launch; device time from HIP events, algorithmic flops 41.5 kflop per (k, w).
+    launch; device time from HIP events, algorithmic flops 13.8 kflop per (k, w), one inverse.
     With cpu: the same cluster's Lanczos ground state from the seed-0 start vector on the
     device and through the oracle's recurrence (one core), and the oracle's dense
     G_c (1 - V G_c)^-1 on a sample of 16 k-points x nw frequencies."""
