@@ -157,11 +157,12 @@ __device__ __forceinline__ void term_group(const GHop* __restrict__ h, const uin
 // terms are in flight together, a term within one word looks up that word only, and the
 // ranks are kept in LDS. 4 sites + 8 bath orbitals with pairing (2.7 million states): 615 us
 // with one term and one direction of it at a time, 226 us.
-template <int EP, int LOOK>
+template <int EP, int LOOK, class... Step>
 __global__ __launch_bounds__(256) void k_hv_general(const uint64_t* __restrict__ st, uint32_t n, LocateTables loc,
                                                     int L, const GHop* __restrict__ hops, int end_up, int end_dn,
                                                     int end_hop, const GDiag* __restrict__ diags, int ndiag,
-                                                    const double* __restrict__ x, double* __restrict__ y, LzStep lz) {
+                                                    const double* __restrict__ x, double* __restrict__ y, Step... step) {
+  const LzStep& lz = step_of<LzStep>(step...);
   __shared__ uint16_t ranks[LOOK == kTablesLds ? 1 << kLdsRank : 1];
   if constexpr (LOOK == kTablesLds) {
     for (uint32_t i = threadIdx.x; i < (1u << L); i += 256) ranks[i] = (uint16_t)loc.rank[i];
@@ -233,8 +234,8 @@ uint32_t grid_of(uint64_t n) { return (uint32_t)std::min<uint64_t>(std::max<uint
 
 }  // namespace
 
-template <int EP>
-static int launch_general(const qed_sector& s, const double* x, double* y, int variant, const LzStep& L) {
+template <int EP, class... Step>
+static int launch_general(const qed_sector& s, const double* x, double* y, int variant, const Step&... step) {
   auto T = std::static_pointer_cast<GeneralTables>(s.general);
   const uint32_t n = (uint32_t)s.D;
   if (n == 0) return 0;
@@ -243,15 +244,16 @@ static int launch_general(const qed_sector& s, const double* x, double* y, int v
   const bool tabled = loc.tabled && variant != 0, lds = tabled && T->L <= kLdsRank;
   // ranks in LDS: eight workgroups per CU fill their tables once
   const uint32_t grid = lds ? std::min(grid_of(n), (uint32_t)device_cu_count() * 8u) : grid_of(n);
-  auto k = !tabled ? k_hv_general<EP, kSearch> : lds ? k_hv_general<EP, kTablesLds> : k_hv_general<EP, kTables>;
+  auto k = !tabled ? k_hv_general<EP, kSearch, Step...>
+                   : lds ? k_hv_general<EP, kTablesLds, Step...> : k_hv_general<EP, kTables, Step...>;
   k<<<grid, 256, 0, stream()>>>(T->states.as<uint64_t>(), n, loc, T->L, T->hops.as<GHop>(), T->end_up, T->end_dn,
-                                T->end_hop, T->diags.as<GDiag>(), T->ndiag, x, y, L);
+                                T->end_hop, T->diags.as<GDiag>(), T->ndiag, x, y, step...);
   QED_HIP(hipGetLastError());
   return (int)grid;
 }
 
 void hv_general(const qed_sector& s, const double* x, double* y, int variant) {
-  launch_general<0>(s, x, y, variant, LzStep{});
+  launch_general<0>(s, x, y, variant);
 }
 
 int hv_step_general(const qed_sector& s, const double* x, double* y, const LzStep& L) {

@@ -251,12 +251,13 @@ __device__ __forceinline__ void ell_row(const HvView& v, const uint32_t* __restr
 // from the row staged in LDS. Down-spin hops: the row's neighbour list is uniform across
 // the workgroup; 8 neighbour rows are requested before any of them is consumed so that
 // each wave keeps 8 row loads in flight.
-template <int BS, bool LDSX, int EP = 0>
+template <int BS, bool LDSX, int EP = 0, class... Step>
 __global__ __launch_bounds__(BS) void k_hv_ell(HvView v, const uint32_t* __restrict__ up_ell,
                                                uint32_t Wu, const uint32_t* __restrict__ dn_ell,
                                                uint32_t Wd, const double* __restrict__ x,
-                                               double* __restrict__ y, LzStep lz = LzStep{}) {
+                                               double* __restrict__ y, Step... step) {
   extern __shared__ double smem[];
+  const LzStep& lz = step_of<LzStep>(step...);
   if constexpr (EP == 0) {
     ell_row<BS, LDSX>(v, up_ell, Wu, dn_ell, Wd, x, y, blockIdx.x, smem);
   } else {
@@ -279,13 +280,13 @@ __global__ __launch_bounds__(BS) void k_hv_ell(HvView v, const uint32_t* __restr
 // it with a stride. Jobs whose active flag is 0 are skipped. Parity selects which of the
 // job's two vector pairs is (x, y), so that an alternating recurrence needs only two job
 // tables.
-template <int BS, int EP = 0>
+template <int BS, int EP = 0, class... Step>
 __global__ __launch_bounds__(BS) void k_hv_ell_batch(const HvJob* __restrict__ jobs, int njobs,
                                                      uint32_t ntiles, int parity,
                                                      const int* __restrict__ active,
-                                                     const uint32_t* __restrict__ tile_job,
-                                                     HvBatchStep L = HvBatchStep{}) {
+                                                     const uint32_t* __restrict__ tile_job, Step... step) {
   extern __shared__ double smem[];
+  const HvBatchStep& L = step_of<HvBatchStep>(step...);
   __shared__ double red[EP == 1 ? BS / 64 : 1];
   for (uint32_t t = blockIdx.x; t < ntiles; t += gridDim.x) {
     const int lo = (int)tile_job[t];  // job owning tile t (row0[lo] <= t < row0[lo + 1])
@@ -457,14 +458,14 @@ __global__ __launch_bounds__(256) void k_hv_tileB_batch(const HvJob* __restrict_
 // Same product, two adjacent columns per thread: 16-byte loads of the down-spin neighbour
 // rows and of the ELL entry pairs (needs an even up dimension).
 // EP: the epilogue of one Lanczos step (LzStep), 0 for y += H x.
-template <int BS, int EP = 0>
+template <int BS, int EP = 0, class... Step>
 __global__ __launch_bounds__(BS) void k_hv_ell2(HvView v, const uint32_t* __restrict__ up_ell,
                                                 uint32_t Wu, const uint32_t* __restrict__ dn_ell,
                                                 uint32_t Wd, const double* __restrict__ x,
                                                 double* __restrict__ y,
-                                                const uint32_t* __restrict__ order = nullptr,
-                                                LzStep lz = LzStep{}) {
+                                                const uint32_t* __restrict__ order, Step... step) {
   extern __shared__ double smem[];
+  const LzStep& lz = step_of<LzStep>(step...);
   const uint32_t du = v.du;
   const uint32_t nvu = v.up_nvals;
   double* vals_s = smem;
@@ -740,10 +741,11 @@ static void set_lds_attributes() {
                               hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
     (void)hipFuncSetAttribute((const void*)k_hv_rows<256, false, true>,
                               hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-    for (const void* f : {(const void*)k_hv_ell<1024, true>, (const void*)k_hv_ell<1024, true, 1>,
-                          (const void*)k_hv_ell<1024, true, 2>, (const void*)k_hv_ell<256, true>,
-                          (const void*)k_hv_ell<256, true, 1>, (const void*)k_hv_ell<256, true, 2>,
-                          (const void*)k_hv_ell2<512>, (const void*)k_hv_ell2<512, 1>, (const void*)k_hv_ell2<512, 2>})
+    for (const void* f : {(const void*)k_hv_ell<1024, true>, (const void*)k_hv_ell<1024, true, 1, LzStep>,
+                          (const void*)k_hv_ell<1024, true, 2, LzStep>, (const void*)k_hv_ell<256, true>,
+                          (const void*)k_hv_ell<256, true, 1, LzStep>, (const void*)k_hv_ell<256, true, 2, LzStep>,
+                          (const void*)k_hv_ell2<512>, (const void*)k_hv_ell2<512, 1, LzStep>,
+                          (const void*)k_hv_ell2<512, 2, LzStep>})
       (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
   });
 }
@@ -843,7 +845,7 @@ void hv(const qed_sector& s, const double* x, double* y, int variant) {
   if (variant == 5) {
     const size_t lds2 = ((size_t)s.du + s.up_nvals + 1) * sizeof(double);
     if (s.du % 2 == 0 && s.du >= 4096 && lds2 <= lds_budget()) {
-      k_hv_ell2<512><<<s.dd, 512, lds2, st>>>(v, ue, s.up_w, de, s.dn_w, x, y);
+      k_hv_ell2<512><<<s.dd, 512, lds2, st>>>(v, ue, s.up_w, de, s.dn_w, x, y, (const uint32_t*)nullptr);
       QED_HIP(hipGetLastError());
       return;
     }
@@ -1074,10 +1076,12 @@ HvBatchConfig hv_batch_tune(const HvBatch& B, const int* active, bool rows) {
   static std::once_flag once;
   std::call_once(once, [] {
     const int bytes = (int)lds_budget();
-    for (const void* f : {(const void*)k_hv_ell_batch<256>, (const void*)k_hv_ell_batch<512>, (const void*)k_hv_ell_batch<1024>,
-                          (const void*)k_hv_ell_batch<256, 1>, (const void*)k_hv_ell_batch<512, 1>,
-                          (const void*)k_hv_ell_batch<1024, 1>, (const void*)k_hv_ell_batch<256, 2>,
-                          (const void*)k_hv_ell_batch<512, 2>, (const void*)k_hv_ell_batch<1024, 2>})
+    using S = HvBatchStep;
+    for (const void* f : {(const void*)k_hv_ell_batch<256>, (const void*)k_hv_ell_batch<512>,
+                          (const void*)k_hv_ell_batch<1024>, (const void*)k_hv_ell_batch<256, 1, S>,
+                          (const void*)k_hv_ell_batch<512, 1, S>, (const void*)k_hv_ell_batch<1024, 1, S>,
+                          (const void*)k_hv_ell_batch<256, 2, S>, (const void*)k_hv_ell_batch<512, 2, S>,
+                          (const void*)k_hv_ell_batch<1024, 2, S>})
       (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
   });
   const TuneKey key = tune_key(B, rows);

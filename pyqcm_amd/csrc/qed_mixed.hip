@@ -208,13 +208,13 @@ __device__ __forceinline__ void hop_group(const uint32_t* e, const uint32_t* c, 
   }
 }
 
-template <bool PACKED, bool VLDS, int EP = 0>
+template <bool PACKED, bool VLDS, int EP, class... Step>
 __global__ __launch_bounds__(256) void k_hv_mixed(HvView v, const uint32_t* __restrict__ up_ell, uint32_t Wu,
                                                   const uint32_t* __restrict__ dn_ell, uint32_t Wd,
                                                   const uint32_t* __restrict__ full_of, const uint32_t* __restrict__ len,
                                                   const uint32_t* __restrict__ code, uint32_t n, uint32_t dn_nvals,
-                                                  const double* __restrict__ x, double* __restrict__ y,
-                                                  LzStep lz = LzStep{}) {
+                                                  const double* __restrict__ x, double* __restrict__ y, Step... step) {
+  const LzStep& lz = step_of<LzStep>(step...);
   constexpr uint32_t mask = (1u << kEllTargetBits) - 1u;
   __shared__ double fac[PACKED ? 16 : 1];  // fac[t] = sqrt(2^(t - 7))
   __shared__ double vals[VLDS ? kLdsVals : 1];
@@ -517,22 +517,22 @@ GroupTables group_tables(int N, int n_sites, const std::vector<std::vector<int>>
   return T;
 }
 
-template <int EP>
-static int launch_mixed(const qed_sector& s, const double* x, double* y, const LzStep& L) {
+template <int EP, class... Step>
+static int launch_mixed(const qed_sector& s, const double* x, double* y, const Step&... step) {
   auto T = std::static_pointer_cast<MixedTables>(s.mixed);
   const qed_sector& b = *T->base;
   const uint32_t n = (uint32_t)s.D, grid = grid_for(n);
   if (n == 0) return 0;
   const bool vl = b.up_nvals + b.dn_nvals <= kLdsVals;
-  auto k = T->packed ? (vl ? k_hv_mixed<true, true, EP> : k_hv_mixed<true, false, EP>)
-                     : (vl ? k_hv_mixed<false, true, EP> : k_hv_mixed<false, false, EP>);
+  auto k = T->packed ? (vl ? k_hv_mixed<true, true, EP, Step...> : k_hv_mixed<true, false, EP, Step...>)
+                     : (vl ? k_hv_mixed<false, true, EP, Step...> : k_hv_mixed<false, false, EP, Step...>);
   k<<<grid, 256, 0, stream()>>>(view(b), b.up_ell.as<uint32_t>(), b.up_w, b.dn_ell.as<uint32_t>(), b.dn_w,
-                                T->full_of.as<uint32_t>(), T->len.as<uint32_t>(), T->code.as<uint32_t>(), n, b.dn_nvals, x, y, L);
+                                T->full_of.as<uint32_t>(), T->len.as<uint32_t>(), T->code.as<uint32_t>(), n, b.dn_nvals, x, y, step...);
   QED_HIP(hipGetLastError());
   return (int)grid;
 }
 
-void hv_mixed(const qed_sector& s, const double* x, double* y) { launch_mixed<0>(s, x, y, LzStep{}); }
+void hv_mixed(const qed_sector& s, const double* x, double* y) { launch_mixed<0>(s, x, y); }
 
 int hv_step_mixed(const qed_sector& s, const double* x, double* y, const LzStep& L) {
   return L.kind == 1 ? launch_mixed<1>(s, x, y, L) : launch_mixed<2>(s, x, y, L);

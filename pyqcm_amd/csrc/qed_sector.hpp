@@ -114,6 +114,18 @@ struct HvJob {
   double* y[2];
 };
 
+// The Lanczos step of a product kernel is passed as a trailing argument pack, so that the
+// plain products (no step) take no argument for it: at 4 us (9 sites) a product is its
+// launch, and 88 unused bytes of arguments are part of that.
+template <class Step>
+__device__ __forceinline__ Step step_of() {
+  return Step{};
+}
+template <class Step>
+__device__ __forceinline__ const Step& step_of(const Step& s) {
+  return s;
+}
+
 // the Lanczos epilogue of a batched product (row form), per job
 struct HvBatchStep {
   int kind = 0;               // as LzStep: 1 eigenvalue pass, 2 eigenvector pass
