@@ -99,8 +99,15 @@ __global__ void k_cf_eval(int n, const int* __restrict__ off, const int* __restr
 // An n x n complex matrix (n <= 16, padded to N with an identity block) is held by LN
 // lanes, R = N / LN rows in the registers of each: row i = q + LN s lives in lane q, slot s.
 // Gauss-Jordan with partial pivoting, rows never moved: at step k the unused row with the
-// largest |re| or |im| in column k is the pivot; its lane writes it to LDS, every lane of
-// the group reads it back and eliminates its own rows.
+// largest |.|^2 in column k is the pivot; its lane writes it to LDS, every lane of the group
+// reads it back and eliminates its own rows.
+//
+// An update is a product rounded once and then subtracted, six operations per element. Both
+// terms of the product added to the accumulator in turn take four, but round twice at the
+// accumulator's size: the error of an inverse is 1.09 to 1.10 times as large (n = 2 to 16,
+// against long double; 4.6 ms instead of 6.0 for the map below). Scaling the pivot row
+// or the row's factor by the pivot's inverse is the same for wide matrices; below 9 the
+// scaled factor is 0.2 to 0.8% worse in an inverse, and costs no less (ROW).
 //
 // What bounds it: the 4 n^3 FP64 multiply-adds of the inversion (1.5 ms for the 8.4 million
 // 12 x 12 matrices of a 128^2 k x 512 w map at 78.6 TFLOP/s) and the LDS broadcast of the
@@ -108,8 +115,8 @@ __global__ void k_cf_eval(int n, const int* __restrict__ off, const int* __restr
 // broadcast among more matrices: 4 lanes x 3 rows put 16 matrices in a wave, against 5 when
 // every lane held one column and exchanged it by lane shuffles (n complex shuffles per step
 // and 8 n selects per row exchange; that form took 23.8 ms for the map above, this one
-// 4.6 ms, 25 TFLOP/s). Small sums (4 x 4, 32^2 k x 20 w) are bound by their four launches:
-// 98 us with 16 matrices in turn per group and 80 waves, 4.6 us with one per group.
+// 6.0 ms, 19 TFLOP/s of 8 n^3 flops each). Small sums (4 x 4, 32^2 k x 20 w) are bound by their
+// four launches: 98 us with 16 matrices in turn per group and 80 waves, 5.1 us with one.
 
 struct KsumArgs {
   int n, nw, nk;        // nk: k points of this launch (k0: their first index of nk_all)
@@ -137,10 +144,13 @@ __device__ __forceinline__ uint32_t group_max(uint32_t v) {
   return v;
 }
 
-__device__ __forceinline__ uint32_t mag_bits(cplx v) {  // monotone in max(|re|, |im|)
-  const uint32_t r = (uint32_t)((uint64_t)__double_as_longlong(v.re) >> 32) << 1;
-  const uint32_t i = (uint32_t)((uint64_t)__double_as_longlong(v.im) >> 32) << 1;
-  return r > i ? r : i;
+__device__ __forceinline__ uint32_t mag_bits(cplx v) {  // monotone in |v|^2
+  return (uint32_t)((uint64_t)__double_as_longlong(cabs2(v)) >> 32);
+}
+
+// a b with the product of the second terms rounded first
+__device__ __forceinline__ cplx cmul_fma(cplx a, cplx b) {
+  return {fma(a.re, b.re, -(a.im * b.im)), fma(a.re, b.im, a.im * b.re)};
 }
 
 // log|det| as a product of |pivot|^2 kept in (0, 1) and a power of two
@@ -163,6 +173,7 @@ template <int N, int LN, bool INV>
 __device__ __forceinline__ void eliminate(cplx (&a)[N / LN][N], int q, double2* buf, uint64_t& perm,
                                           int (&step)[N / LN], LogDet& ld, bool& zero) {
   constexpr int R = N / LN;
+  constexpr bool ROW = N <= (INV ? 8 : 2);
   perm = 0;
 #pragma unroll
   for (int s = 0; s < R; ++s) step[s] = -1;
@@ -205,23 +216,24 @@ __device__ __forceinline__ void eliminate(cplx (&a)[N / LN][N], int q, double2* 
     const double c2 = cabs2(rp[k]);
     if (!INV) ld.mul(c2);
     else zero |= rp[k].re == 0.0 && rp[k].im == 0.0;
-    const double ic2 = 1.0 / c2;
-    const cplx dinv{rp[k].re * ic2, -rp[k].im * ic2};
+    const cplx dinv{rp[k].re / c2, -rp[k].im / c2};
+    if constexpr (ROW) {
+#pragma unroll
+      for (int j = 0; j < N; ++j)
+        if (j != k && (INV || j > k)) rp[j] = cmul_fma(rp[j], dinv);
+    }
 #pragma unroll
     for (int s = 0; s < R; ++s) {
-      cplx f = cmul(a[s][k], dinv);
-      if (INV) {
-        if (p == q + LN * s) f = {-dinv.re, -dinv.im};
-        a[s][k] = {-f.re, -f.im};
+      cplx f = ROW ? a[s][k] : cmul_fma(a[s][k], dinv);
+      if constexpr (INV) {  // the pivot row (cleared above) becomes the scaled row
+        const cplx own = ROW ? cplx{-1.0, 0.0} : cplx{-dinv.re, -dinv.im};
+        if (p == q + LN * s) f = own;
+        const cplx c = ROW ? cmul_fma(f, dinv) : f;
+        a[s][k] = {-c.re, -c.im};
       }
 #pragma unroll
-      for (int j = 0; j < N; ++j) {
-        if (j == k || (!INV && j < k)) continue;
-        a[s][j].re = fma(-f.re, rp[j].re, a[s][j].re);
-        a[s][j].re = fma(f.im, rp[j].im, a[s][j].re);
-        a[s][j].im = fma(-f.re, rp[j].im, a[s][j].im);
-        a[s][j].im = fma(-f.im, rp[j].re, a[s][j].im);
-      }
+      for (int j = 0; j < N; ++j)
+        if (j != k && (INV || j > k)) a[s][j] = csub(a[s][j], cmul_fma(f, rp[j]));
     }
   }
 }
@@ -329,8 +341,8 @@ __global__ __launch_bounds__(64) void k_gc_inverse(int n, int nw, const double* 
 // M(w, k) = Gc(w)^-1 - V(k) for the (w, k) of a launch. MODE 0: the inverses; 1: their
 // traces; 2: their sum over k; 3: the sum over k of log|det|. A group takes `chunk`
 // matrices in turn: one k point and a run of frequencies (modes 0, 1), or one frequency and
-// a run of k blocks (modes 2, 3). Two waves per SIMD, which the 12-wide form just fits
-// (250 registers); the sum over k of wide matrices takes 40 KB of LDS and one wave.
+// a run of k blocks (modes 2, 3). Two waves per SIMD, for which the 12- and 16-wide forms
+// spill 24 to 96 bytes per lane; the sum over k of wide matrices takes 40 KB of LDS and one wave.
 template <int N, int MODE>
 __global__ __launch_bounds__(64, MODE == 2 && N >= 12 ? 1 : 2) void k_ksum(KsumArgs A) {
   constexpr int LN = lanes_of<N>(), R = N / LN, G = 64 / LN;

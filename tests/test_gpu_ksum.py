@@ -68,3 +68,51 @@ def test_singular_cluster_green_function_is_refused(gpu_lib, n):
     for call in (lambda: LT.cpt_batch(G, V0, nv, mats, k, mode="trace"), lambda: LT.sef_batch(G, V0, nv, mats, k)):
         with pytest.raises(gpu_lib.QEDError, match="singular at a requested frequency"):
             call()
+
+
+def _gauss_jordan(M, real):
+    """Inverses of a batch of matrices by Gauss-Jordan with partial pivoting, in real
+    arithmetic of type `real` without fused multiply-adds."""
+    B, n = M.shape[:2]
+    re = np.concatenate([M.real.astype(real), np.broadcast_to(np.eye(n, dtype=real), M.shape)], 2)
+    im = np.concatenate([M.imag.astype(real), np.zeros(M.shape, real)], 2)
+    r = np.arange(B)
+    for k in range(n):
+        p = k + (re[:, k:, k] ** 2 + im[:, k:, k] ** 2).argmax(1)
+        for a in (re, im):
+            a[r, k], a[r, p] = a[r, p].copy(), a[r, k].copy()
+        c, s = re[:, k, k][:, None], im[:, k, k][:, None]
+        d = c * c + s * s
+        c, s = c / d, -s / d
+        re[:, k], im[:, k] = re[:, k] * c - im[:, k] * s, re[:, k] * s + im[:, k] * c
+        fr, fi = re[:, :, k].copy()[:, :, None], im[:, :, k].copy()[:, :, None]
+        fr[:, k] = fi[:, k] = 0.0
+        pr, pi = re[:, None, k], im[:, None, k]
+        re, im = re - (fr * pr - fi * pi), im - (fr * pi + fi * pr)
+    return re[:, :, n:] + 1j * im[:, :, n:]
+
+
+@pytest.mark.parametrize("n", [2, 4, 8, 12, 16])
+def test_rounding_error_of_the_inverse(gpu_lib, n):
+    """Geometric mean over 4096 matrices, known exactly, of the relative error of their
+    inverses. In 64 bits the same elimination without fused multiply-adds rounds each product
+    once more than the device, whose error is 0.91 to 0.93 of that one's; with two products
+    added to the accumulator in turn, two roundings of its size, it is 1.02 to 1.04 of it.
+    (The mean of 4096 logarithms is good to 1%.)"""
+    rng = np.random.default_rng(n)
+    k = np.stack(np.meshgrid(*[np.arange(4) / 4.0] * 3), -1).reshape(64, 3)  # phases 1, i, -1, -i
+    nv = np.concatenate([np.eye(3), np.eye(3)[[1, 2, 0]] + np.eye(3)])
+    exact = lambda *s: (rng.integers(-2**22, 2**22, s) + 1j * rng.integers(-2**22, 2**22, s)) / 2.0**20
+    log_dev, log_ref = [], []
+    for _ in range(64):
+        V0, mats = exact(n, n), exact(6, n, n)
+        ph = np.round(np.exp(2j * np.pi * (k @ nv.T)))
+        M = np.eye(n) - (V0 + np.einsum("kt,tab->kab", ph, mats))
+        dev = LT.cpt_batch(np.eye(n, dtype=complex)[None], V0, nv, mats, k, mode="full")[0]
+        inv = _gauss_jordan(M, np.longdouble)
+        norm = lambda a: np.sqrt((np.abs(a) ** 2).sum((1, 2)))
+        log_dev.append(np.log(norm(dev - inv) / norm(inv)))
+        log_ref.append(np.log(norm(_gauss_jordan(M, np.float64) - inv) / norm(inv)))
+    ratio = float(np.exp(np.mean(log_dev) - np.mean(log_ref)))
+    print("n = %d: error %.3e, %.3f of the unfused form's" % (n, np.exp(np.mean(log_dev)), ratio), flush=True)
+    assert ratio <= 0.98
