@@ -148,6 +148,15 @@ __device__ __forceinline__ uint32_t mag_bits(cplx v) {  // monotone in |v|^2
   return (uint32_t)((uint64_t)__double_as_longlong(cabs2(v)) >> 32);
 }
 
+// The same for |v|^2 beyond the range of a double: its exponent in 13 bits, 14 of its mantissa
+__device__ __forceinline__ uint32_t mag_bits_wide(cplx v) {
+  const int e = __builtin_amdgcn_frexp_exp(fmax(fabs(v.re), fabs(v.im)));
+  const double c2 = cabs2(cplx{ldexp(v.re, -e), ldexp(v.im, -e)});
+  if (c2 == 0.0) return 0;
+  const uint32_t mant = (uint32_t)((uint64_t)__double_as_longlong(__builtin_amdgcn_frexp_mant(c2)) >> 32) & 0xfffffu;
+  return (uint32_t)(2 * e + __builtin_amdgcn_frexp_exp(c2) + 4096) << 19 | mant >> 6 << 5;
+}
+
 // a b with the product of the second terms rounded first
 __device__ __forceinline__ cplx cmul_fma(cplx a, cplx b) {
   return {fma(a.re, b.re, -(a.im * b.im)), fma(a.re, b.im, a.im * b.re)};
@@ -169,7 +178,9 @@ struct LogDet {
 // row that was the pivot of step k holding C[k][:], so that A^-1[k][p_j] = C[k][j]; the
 // pivot rows p_j are the nibbles of perm and step[s] is the k of this lane's row s.
 // Otherwise the rows below only (the determinant). buf: N double2 of LDS for the group.
-template <int N, int LN, bool INV>
+// WIDE: pivots whose square leaves the range of a double (one inversion per frequency takes
+// it, as an inverse on the host would; the sums over k do not).
+template <int N, int LN, bool INV, bool WIDE = false>
 __device__ __forceinline__ void eliminate(cplx (&a)[N / LN][N], int q, double2* buf, uint64_t& perm,
                                           int (&step)[N / LN], LogDet& ld, bool& zero) {
   constexpr int R = N / LN;
@@ -182,7 +193,8 @@ __device__ __forceinline__ void eliminate(cplx (&a)[N / LN][N], int q, double2* 
     uint32_t key = 0;
 #pragma unroll
     for (int s = 0; s < R; ++s) {
-      const uint32_t m = (mag_bits(a[s][k]) & ~31u) | 16u | (uint32_t)(q + LN * s);
+      const uint32_t mag = WIDE ? mag_bits_wide(a[s][k]) : mag_bits(a[s][k]);
+      const uint32_t m = (mag & ~31u) | 16u | (uint32_t)(q + LN * s);
       key = dpp_max(key, step[s] < 0 ? m : 0u);
     }
     key = group_max<LN>(key);
@@ -213,10 +225,17 @@ __device__ __forceinline__ void eliminate(cplx (&a)[N / LN][N], int q, double2* 
     }
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
-    const double c2 = cabs2(rp[k]);
-    if (!INV) ld.mul(c2);
-    else zero |= rp[k].re == 0.0 && rp[k].im == 0.0;
-    const cplx dinv{rp[k].re / c2, -rp[k].im / c2};
+    cplx pv = rp[k];
+    int pe = 0;
+    if constexpr (WIDE) {
+      pe = __builtin_amdgcn_frexp_exp(fmax(fabs(pv.re), fabs(pv.im)));
+      pv = {ldexp(pv.re, -pe), ldexp(pv.im, -pe)};
+    }
+    const double c2 = cabs2(pv);
+    if (!INV) ld.mul(c2), ld.e += 2 * pe;
+    else zero |= pv.re == 0.0 && pv.im == 0.0;
+    cplx dinv{pv.re / c2, -pv.im / c2};
+    if constexpr (WIDE) dinv = {ldexp(dinv.re, -pe), ldexp(dinv.im, -pe)};
     if constexpr (ROW) {
 #pragma unroll
       for (int j = 0; j < N; ++j)
@@ -323,11 +342,11 @@ __global__ __launch_bounds__(64) void k_gc_inverse(int n, int nw, const double* 
     bool zero = false;
     if (pass == 0) {
       if (!logdet) continue;
-      eliminate<N, LN, false>(a, q, buf[g], perm, step, ld, zero);
+      eliminate<N, LN, false, true>(a, q, buf[g], perm, step, ld, zero);
       if (q == 0) logdet[w] = ld.value();
       continue;
     }
-    eliminate<N, LN, true>(a, q, buf[g], perm, step, ld, zero);
+    eliminate<N, LN, true, true>(a, q, buf[g], perm, step, ld, zero);
     if (zero) *singular = 1;
     double2* o = reinterpret_cast<double2*>(ginv) + (size_t)w * N * N;
 #pragma unroll

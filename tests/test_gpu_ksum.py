@@ -116,3 +116,23 @@ def test_rounding_error_of_the_inverse(gpu_lib, n):
     ratio = float(np.exp(np.mean(log_dev) - np.mean(log_ref)))
     print("n = %d: error %.3e, %.3f of the unfused form's" % (n, np.exp(np.mean(log_dev)), ratio), flush=True)
     assert ratio <= 0.98
+
+
+@pytest.mark.parametrize("n", [3, 8, 13])
+def test_cluster_green_function_beyond_the_range_of_a_square(gpu_lib, n):
+    """One orbital of Gc so small or so large that the square of its pivot leaves the range of
+    a double: it drops out of the lattice Green function, and its logarithm stays finite."""
+    _, V0, nv, mats, k = _inputs(n, 2, 3, 2, 11)
+    rng = np.random.default_rng(n)
+    G = rng.standard_normal((2, n, n)) + 1j * rng.standard_normal((2, n, n))
+    V = V0 + np.einsum("kt,tab->kab", np.exp(2j * np.pi * (k @ nv.T)), mats)
+    Gc = G.copy()
+    Gc[:, 0] = Gc[:, :, 0] = 0.0
+    Gc[:, 0, 0] = 1e-160 * (1 + 1j)
+    inv = np.linalg.inv(np.linalg.inv(Gc[:, 1:, 1:])[:, None] - V[:, 1:, 1:])
+    dev = LT.cpt_batch(Gc, V0, nv, mats, k, mode="full")
+    np.testing.assert_allclose(dev[:, :, 1:, 1:], inv, rtol=0, atol=1e-10 * np.abs(inv).max())
+    assert np.abs(dev[:, :, 0]).max() < 1e-100 and np.abs(dev[:, :, :, 0]).max() < 1e-100
+    Gc[:, 0, 0] = 1e160 * (1 + 1j)
+    ref = np.linalg.slogdet(V[None] @ Gc[:, None] - np.eye(n))[1].mean(1)
+    np.testing.assert_allclose(LT.sef_batch(Gc, V0, nv, mats, k), ref, rtol=1e-12)
