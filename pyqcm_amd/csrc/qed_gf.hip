@@ -12,12 +12,12 @@
 #include <cstring>
 #include <memory>
 #include <mutex>
-#include <thread>
 #include <type_traits>
 #include <vector>
 
 #include "../../include/qed.h"
 #include "qed_common.hpp"
+#include "qed_hostcopy.hpp"
 #include "qed_linalg.hpp"
 
 namespace qed {
@@ -598,7 +598,7 @@ class KsumLease {
 // often touched for the first time here, which is what a single thread is slow at).
 void copy_out(unsigned char* dst, const unsigned char* src_dev, size_t bytes, unsigned char* pin, size_t pin_bytes) {
   const size_t piece = pin_bytes / 2;
-  const int nt = bytes >= (size_t(8) << 20) ? 8 : 1;
+  const int nt = copy_threads(bytes);
   auto send = [&](size_t i) {
     const size_t o = i * piece;
     if (o < bytes)
@@ -610,12 +610,7 @@ void copy_out(unsigned char* dst, const unsigned char* src_dev, size_t bytes, un
     send(i + 1);
     const size_t o = i * piece, len = std::min(piece, bytes - o);
     const unsigned char* from = pin + (i & 1) * piece;
-    const size_t per = ((len + nt - 1) / nt + 4095) & ~size_t(4095);
-    std::vector<std::thread> th;
-    for (int t = 1; t < nt && t * per < len; ++t)
-      th.emplace_back([=] { std::memcpy(dst + o + t * per, from + t * per, std::min(per, len - t * per)); });
-    std::memcpy(dst + o, from, std::min(per, len));
-    for (auto& t : th) t.join();
+    copy_parallel(dst + o, from, len, nt);
   }
 }
 
