@@ -137,11 +137,12 @@ int qed_start_vector(qed_sector* s, int seed, double* x_dev);
 int qed_lanczos_gs(qed_sector* s, double accur, int max_iter, double* psi_dev, double* E0,
                    int* niter, double* alpha, double* beta);
 
-/* qed_lanczos_gs without device allocation. No counterpart in the reference: for callers
- * that cannot allocate device memory (tight solver loops, harnesses that forbid hipMalloc
- * after start-up). Same arguments and results as qed_lanczos_gs; the two recurrence
- * vectors and the parts and scalars of its steps live in a fixed device array of the library (one
- * per GPU, 34.1 MB, held until the process ends), so the sector dimension is limited to
+/* qed_lanczos_gs without allocation of device or pinned host memory, streams or events. No
+ * counterpart in the reference: for callers that cannot allocate (tight solver loops,
+ * harnesses that forbid hipMalloc after start-up). Same arguments and results as
+ * qed_lanczos_gs; the two recurrence vectors and the parts and scalars of its steps live in
+ * a fixed device array of the library (one per GPU, 34.1 MB, held until the process ends) and
+ * its pinned memory and events are made by qed_init. So the sector dimension is limited to
  * 2^21 = 2,097,152: a larger sector fails with an error and nothing is launched. All calls
  * on one GPU share that array, which keeps the last call's contents; the library lock
  * serializes the calls of one process, and calls that overlap on one GPU otherwise race. */

@@ -26,6 +26,7 @@ struct Error : std::runtime_error {
   } while (0)
 
 void ensure_init();
+void lanczos_host_init();  // once, with the library: the host side of qed_lanczos_gs_noalloc
 hipStream_t stream();
 void set_error(const std::string& msg);
 int device_cu_count();

@@ -350,42 +350,80 @@ void tridiag_lowest_next(const std::vector<double>& a, const std::vector<double>
   tridiag_vector(a, b, rho, vec);
 }
 
-// Pinned host memory for the scalars of a Lanczos run, taken from a small pool (one per
-// concurrent run) and given back.
-class PinnedScalars {
- public:
+// The host side of a Lanczos run: pinned memory for the scalars of two chunks of steps, and
+// an event for each.
+struct LanczosHost {
   static constexpr size_t kDoubles = 4 * kLzRing;
-  PinnedScalars() {
-    std::lock_guard<std::mutex> lk(mutex());
-    if (!idle().empty()) {
-      p_ = idle().back();
-      idle().pop_back();
-    } else {
-      QED_HIP(hipHostMalloc((void**)&p_, kDoubles * sizeof(double), hipHostMallocDefault));
+  double* pin = nullptr;
+  hipEvent_t done[2] = {nullptr, nullptr};
+  LanczosHost() {
+    try {
+      QED_HIP(hipHostMalloc((void**)&pin, kDoubles * sizeof(double), hipHostMallocDefault));
+      for (hipEvent_t& e : done) QED_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    } catch (...) {
+      release();
+      throw;
     }
   }
-  PinnedScalars(const PinnedScalars&) = delete;
-  ~PinnedScalars() {
-    (void)hipStreamSynchronize(stream());
-    std::lock_guard<std::mutex> lk(mutex());
-    if (idle().size() < 8) idle().push_back(p_);
-    else (void)hipHostFree(p_);
+  LanczosHost(const LanczosHost&) = delete;
+  ~LanczosHost() { release(); }
+
+ private:
+  void release() {
+    if (pin) (void)hipHostFree(pin);
+    for (hipEvent_t e : done)
+      if (e) (void)hipEventDestroy(e);
   }
-  double* get() { return p_; }
+};
+
+// made with the library for qed_lanczos_gs_noalloc, whose calls one lock serializes
+LanczosHost* g_fixed_host = nullptr;
+
+// One of them for the length of a run, from a small pool (one per concurrent run) and given
+// back; or the fixed one.
+class LanczosLease {
+ public:
+  explicit LanczosLease(bool fixed) : fixed_(fixed) {
+    if (fixed_) {
+      h_ = g_fixed_host;
+      return;
+    }
+    std::lock_guard<std::mutex> lk(mutex());
+    if (!idle().empty()) {
+      h_ = idle().back();
+      idle().pop_back();
+    } else {
+      h_ = new LanczosHost();
+    }
+  }
+  LanczosLease(const LanczosLease&) = delete;
+  ~LanczosLease() {
+    (void)hipStreamSynchronize(stream());
+    if (fixed_) return;
+    std::lock_guard<std::mutex> lk(mutex());
+    if (idle().size() < 8) idle().push_back(h_);
+    else delete h_;
+  }
+  LanczosHost* operator->() { return h_; }
 
  private:
   static std::mutex& mutex() {
     static std::mutex m;
     return m;
   }
-  static std::vector<double*>& idle() {  // never destroyed: the runtime may be gone by then
-    static auto* v = new std::vector<double*>();
+  static std::vector<LanczosHost*>& idle() {  // never destroyed: the runtime may be gone by then
+    static auto* v = new std::vector<LanczosHost*>();
     return *v;
   }
-  double* p_ = nullptr;
+  bool fixed_;
+  LanczosHost* h_ = nullptr;
 };
 
 }  // namespace
+
+void lanczos_host_init() {
+  if (!g_fixed_host) g_fixed_host = new LanczosHost();
+}
 
 std::recursive_mutex& lib_mutex() {
   static std::recursive_mutex m;
@@ -542,14 +580,9 @@ void lanczos_gs(qed_sector& s, double accur, int max_iter, double* psi, double* 
   const int chunk = n <= (1u << 20) ? 8 : n <= (1u << 24) ? 2 : 1;
   std::vector<double> alpha, beta, evec;
   double e0 = 0.0;
-  PinnedScalars pin;
+  LanczosLease host(ws != nullptr);
   LanczosRun run(s, ws);
   run.start(psi);
-  struct Event {
-    hipEvent_t e = nullptr;
-    Event() { QED_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming)); }
-    ~Event() { (void)hipEventDestroy(e); }
-  } done[2];
   const bool ahead = chunk > 1;
   int launched = 0, tested = 0;  // steps
   int end[2] = {0, 0};           // steps done at the end of the two chunks in flight
@@ -559,8 +592,8 @@ void lanczos_gs(qed_sector& s, double accur, int max_iter, double* psi, double* 
     const int c = std::max(1, std::min(chunk, max_iter + 1 - launched));
     for (int i = 0; i < c; ++i) run.step();
     launched += c;
-    run.fetch(pin.get() + slot * 2 * kLzRing);
-    QED_HIP(hipEventRecord(done[slot].e, stream()));
+    run.fetch(host->pin + slot * 2 * kLzRing);
+    QED_HIP(hipEventRecord(host->done[slot], stream()));
     end[slot] = launched;
     slot ^= 1;
   };
@@ -569,8 +602,8 @@ void lanczos_gs(qed_sector& s, double accur, int max_iter, double* psi, double* 
     if (ahead && launched <= max_iter && launched - tested <= chunk) launch();
     // the older chunk in flight
     const int o = launched > tested && end[slot] > tested ? slot : slot ^ 1;
-    QED_HIP(hipEventSynchronize(done[o].e));
-    const double* h = pin.get() + o * 2 * kLzRing;
+    QED_HIP(hipEventSynchronize(host->done[o]));
+    const double* h = host->pin + o * 2 * kLzRing;
     for (int k = tested; k < end[o] && !converged; ++k) {
       alpha.push_back(h[k % kLzRing]);
       beta.push_back(h[kLzRing + k % kLzRing]);
@@ -1160,7 +1193,7 @@ int qed_lanczos_steps_timed(qed_sector* s, const double* psi, int steps, double*
     hipEvent_t e0, e1;
     QED_HIP(hipEventCreate(&e0));
     QED_HIP(hipEventCreate(&e1));
-    PinnedScalars pin;
+    LanczosLease host(false);
     auto reset = [&] {
       run.start(psi);
       QED_HIP(hipStreamSynchronize(stream()));
@@ -1172,7 +1205,7 @@ int qed_lanczos_steps_timed(qed_sector* s, const double* psi, int steps, double*
       QED_HIP(hipEventRecord(e0, stream()));
       for (int k = 0; k < steps; ++k) {
         run.step();
-        run.fetch(pin.get());
+        run.fetch(host->pin);
         QED_HIP(hipStreamSynchronize(stream()));
       }
       QED_HIP(hipEventRecord(e1, stream()));

@@ -55,6 +55,12 @@ static void do_init(int device) {
     g_init_err = std::string("hipStreamCreate: ") + hipGetErrorString(e);
     return;
   }
+  try {
+    lanczos_host_init();
+  } catch (const std::exception& e) {
+    g_init_err = e.what();
+    return;
+  }
   g_ready = true;
 }
 

@@ -2,7 +2,12 @@
 vectors and partial sums live in a fixed device array of the library), against
 qed_lanczos_gs on the same sectors and start vectors: three calls in a row on sectors of
 decreasing size (the array keeps the previous call's contents), one of them on the fused
-Lanczos product; and the error for a sector beyond the array's limit."""
+Lanczos product; the error for a sector beyond the array's limit; and the runtime's allocating
+calls, counted."""
+import os
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 
@@ -71,3 +76,66 @@ def test_noalloc_lanczos_rejects_large_sector(gpu_lib):
         _lib.call("qed_lanczos_gs_noalloc", S.h, 1e-12, 10, psi.ptr, _lib.dp(E0), _lib.ip(nit), None, None)
     psi.free()
     S.close()
+
+
+COUNTER = r"""
+#include <dlfcn.h>
+#include <cstddef>
+#include <cstdio>
+#include <cstdlib>
+static int count = 0;
+static void* real(const char* name) {
+  static void* lib = dlopen("libamdhip64.so.7", RTLD_LAZY | RTLD_LOCAL);
+  void* f = lib ? dlsym(lib, name) : nullptr;
+  if (!f) { fprintf(stderr, "no %s\n", name); exit(3); }
+  return f;
+}
+#define COUNT(name, params, args) \
+  extern "C" int name params { ++count; return ((int(*) params)real(#name)) args; }
+COUNT(hipMalloc, (void** p, size_t n), (p, n))
+COUNT(hipMallocAsync, (void** p, size_t n, void* s), (p, n, s))
+COUNT(hipHostMalloc, (void** p, size_t n, unsigned f), (p, n, f))
+COUNT(hipFree, (void* p), (p))
+COUNT(hipHostFree, (void* p), (p))
+COUNT(hipEventCreate, (void** e), (e))
+COUNT(hipEventCreateWithFlags, (void** e, unsigned f), (e, f))
+COUNT(hipEventDestroy, (void* e), (e))
+COUNT(hipStreamCreateWithFlags, (void** s, unsigned f), (s, f))
+extern "C" int counted() { return count; }
+"""
+
+CALLS = r"""
+import ctypes, sys
+stub = ctypes.CDLL(sys.argv[1], ctypes.RTLD_GLOBAL)
+import numpy as np
+from pyqcm_amd import _lib
+from tests import models as TM
+from tests.test_zz_no_alloc import _run
+from pyqcm_amd.sector import Sector
+from pyqcm_amd._lib import DeviceArray
+_lib.call("qed_init", 0)
+made = 0
+for (m, vals), nup, ndn in [(TM.square(2, 3, U=4.0, mu=2.0), 3, 3), (TM.square(4, 4, tp=-0.3, U=8.0, mu=4.0), 8, 1)]:
+    S = Sector(m.L, nup, ndn, m.flat(vals))
+    x0 = np.random.default_rng(1).standard_normal(S.dim)
+    psi = DeviceArray.from_host(x0 / np.linalg.norm(x0))
+    E0, nit = np.zeros(1), np.zeros(1, np.int32)
+    before = stub.counted()
+    _lib.call("qed_lanczos_gs_noalloc", S.h, 1e-12, 400, psi.ptr, _lib.dp(E0), _lib.ip(nit), None, None)
+    made += stub.counted() - before
+print("outside", before, "inside", made, flush=True)
+"""
+
+
+def test_noalloc_lanczos_makes_no_runtime_objects(gpu_lib, tmp_path):
+    """In a process of its own the runtime's allocating calls are counted (their names are
+    resolved to a counting library first): none from the first call on, where pinned memory or
+    events made on demand would show."""
+    src, so = tmp_path / "count.cpp", tmp_path / "libcount.so"
+    src.write_text(COUNTER)
+    subprocess.check_call(["g++", "-O1", "-shared", "-fPIC", str(src), "-o", str(so), "-ldl"])
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    r = subprocess.run([sys.executable, "-c", CALLS, str(so)], cwd=root, capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0, (r.stdout, r.stderr)
+    _, outside, _, inside = r.stdout.split()[-4:]
+    assert int(outside) > 0 and int(inside) == 0, r.stdout
