@@ -518,12 +518,11 @@ __global__ __launch_bounds__(BS) void k_hv_ell2(HvView v, const uint32_t* __rest
       }
     }
     double2 yo = yr[c2];
-    double2 po = make_double2(0.0, 0.0);
-    if constexpr (EP == 2) po = reinterpret_cast<double2*>(lz.psi + (uint64_t)r * du)[c2];
-    lz_update<EP>(lz, sc, a0 + b0, xs[c], &yo.x, &po.x, dotp);
-    lz_update<EP>(lz, sc, a1 + b1, xs[c + 1], &yo.y, &po.y, dotp);
+    double* pr = nullptr;  // by single doubles: the caller's vector may be aligned to 8 bytes only
+    if constexpr (EP == 2) pr = lz.psi + (uint64_t)r * du + c;
+    lz_update<EP>(lz, sc, a0 + b0, xs[c], &yo.x, pr, dotp);
+    lz_update<EP>(lz, sc, a1 + b1, xs[c + 1], &yo.y, pr + 1, dotp);
     yr[c2] = yo;
-    if constexpr (EP == 2) reinterpret_cast<double2*>(lz.psi + (uint64_t)r * du)[c2] = po;
   }
   if constexpr (EP == 1) {
     const double t = block_sum(dotp, smem + ((nvu + 1u) & ~1u) + du);

@@ -81,3 +81,24 @@ def test_iteration_limit(gpu_lib, size):
         with pytest.raises(gpu_lib.QEDError, match="exceeded %d iterations" % limit):
             S.lanczos_gs(start=x, max_iter=limit)
     S.close()
+
+
+def test_vector_aligned_to_eight_bytes(gpu_lib):
+    """A start vector behind one double of another buffer, on the two-column kernel of long
+    rows: the same numbers as from an aligned one, and nothing written around it."""
+    from pyqcm_amd._lib import DeviceArray
+    from pyqcm_amd.sector import Sector
+    m, v = TM.square(4, 4, tp=-0.3)
+    S = Sector(16, 8, 1, m.flat(v))
+    x = np.random.default_rng(6).standard_normal(S.dim)
+    x /= np.linalg.norm(x)
+    out = []
+    for shift in (0, 1):
+        buf = DeviceArray.from_host(np.concatenate([np.full(shift, 7.0), x, [9.0]]))
+        E0, nit = np.zeros(1), np.zeros(1, np.int32)
+        gpu_lib.call("qed_lanczos_gs", S.h, 1e-12, 400, buf.offset(shift), gpu_lib.dp(E0), gpu_lib.ip(nit), None, None)
+        h = buf.to_host()
+        assert h[-1] == 9.0 and (shift == 0 or h[0] == 7.0)
+        out.append((float(E0[0]), int(nit[0]), h[shift:-1]))
+    assert out[0][:2] == out[1][:2]
+    np.testing.assert_array_equal(out[0][2], out[1][2])
