@@ -909,8 +909,9 @@ int hv_step(const qed_sector& s, const double* x, double* y, const LzStep& L) {
   const HvView v = view(s);
   // the kernels of hv(); the reduction needs eight more doubles of LDS
   const size_t lds2 = ((size_t)s.du + s.up_nvals + 1 + 16) * sizeof(double);
-  const uint32_t grid = std::min(s.dd, kLzRows);
-  if (s.du % 2 == 0 && s.du >= 4096 && lds2 <= lds_budget() && grid == s.dd) {
+  uint32_t grid = std::min(s.dd, kLzRows);
+  if (s.du % 2 == 0 && s.du >= 4096 && lds2 <= lds_budget()) {
+    grid = s.dd;
     ensure_row_order(s);
     const uint32_t* ue = s.up_ell.as<uint32_t>();
     const uint32_t* de = s.dn_ell.as<uint32_t>();

@@ -520,12 +520,12 @@ struct LanczosRun {
     } else {
       rb.alloc(n * 8);
       qb.alloc(n * 8);
-      wb.alloc(kLzWork * 8);
+      wb.alloc((kLzWork - kLzRows + lz_parts(s)) * 8);
       r = rb.as<double>();
       q = qb.as<double>();
       pa = wb.as<double>();
     }
-    pb[0] = pa + kLzRows;
+    pb[0] = pa + lz_parts(s);
     pb[1] = pb[0] + kLzParts;
     alpha = pb[1] + kLzParts;
     beta = alpha + kLzRing;

@@ -1,6 +1,7 @@
 // One factorized sector (N_up, N_dn) of a cluster Hamiltonian resident on the device.
 #pragma once
 
+#include <algorithm>
 #include <cstdint>
 #include <functional>
 #include <memory>
@@ -225,12 +226,15 @@ struct LzStep {
   int nb = 0;
   const double* beta = nullptr;  // beta_i at beta[i % ring]
   int ring = 1;
-  double* pa = nullptr;  // kLzRows doubles
+  double* pa = nullptr;  // lz_parts() doubles
   double s0 = 0, s1 = 0, s2 = 0, c = 0;
   double* psi = nullptr;
 };
 constexpr int kLzParts = 1024;        // partial sums that every wave of a kernel adds up itself
-constexpr uint32_t kLzRows = 1 << 16;  // parts that a product may leave (folded when above kLzParts)
+constexpr uint32_t kLzRows = 1 << 16;
+// parts that a product may leave (folded when above kLzParts): one per row where rows are
+// long (the two-column kernel), at most kLzRows otherwise
+inline size_t lz_parts(const qed_sector& s) { return s.du >= 4096 ? std::max(s.dd, kLzRows) : kLzRows; }
 // the product of one step; the number of parts it leaves in pa
 int hv_step(const qed_sector& s, const double* x, double* y, const LzStep& L);
 int hv_step_mixed(const qed_sector& s, const double* x, double* y, const LzStep& L);
@@ -313,6 +317,7 @@ struct LanczosWork {
   double* red;
 };
 constexpr int kLzRing = 64;  // alpha and beta of the last steps on the device
+// (of a sector with at most 2^28 amplitudes, whose long rows are no more than kLzRows)
 constexpr size_t kLzWork = kLzRows + 2 * kLzParts + 2 * kLzRing + 64;
 void lanczos_gs(qed_sector& s, double accur, int max_iter, double* psi, double* E0, int* niter,
                 std::vector<double>* alpha, std::vector<double>* beta, const LanczosWork* ws = nullptr);

@@ -102,3 +102,32 @@ def test_vector_aligned_to_eight_bytes(gpu_lib):
         out.append((float(E0[0]), int(nit[0]), h[shift:-1]))
     assert out[0][:2] == out[1][:2]
     np.testing.assert_array_equal(out[0][2], out[1][2])
+
+
+def test_more_long_rows_than_folded_parts(gpu_lib):
+    """19 sites, 5 up and 8 down: 75,582 rows of 11,628 (more than 2^16 parts of a scalar
+    product) take the kernel of long rows. A step's alpha and beta against the product and dot
+    products of the plain recurrence, and less time than that of its separate passes."""
+    from pyqcm_amd._lib import DeviceArray
+    from pyqcm_amd.sector import Sector
+    m, v = TM.chain(19, U=4.0, mu=2.0)
+    S = Sector(19, 5, 8, m.flat(v))
+    assert S.dd > 1 << 16 and S.du >= 4096 and S.du % 2 == 0
+    x = DeviceArray(S.dim)
+    gpu_lib.call("qed_start_vector", S.h, 1, x.ptr)
+    ms = np.zeros(2)
+    gpu_lib.call("qed_lanczos_steps_timed", S.h, x.ptr, 3, gpu_lib.dp(ms))
+    assert ms[0] < ms[1]
+    h = x.to_host()
+    w = S.hv(h)
+    a0 = float(h @ w)
+    w -= a0 * h
+    b0 = float(np.linalg.norm(w))
+    E0, nit = np.zeros(1), np.zeros(1, np.int32)
+    alpha, beta = np.zeros(2), np.zeros(2)
+    # any first Ritz value passes this limit: one step
+    gpu_lib.call("qed_lanczos_gs", S.h, 1e6, 1, x.ptr, gpu_lib.dp(E0), gpu_lib.ip(nit), gpu_lib.dp(alpha), gpu_lib.dp(beta))
+    assert nit[0] == 1
+    np.testing.assert_allclose([alpha[0], beta[0]], [a0, b0], rtol=1e-11)
+    x.free()
+    S.close()
