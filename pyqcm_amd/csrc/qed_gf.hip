@@ -594,11 +594,10 @@ class KsumLease {
 };
 
 // Copies bytes from the device to caller memory through the pinned buffer, in pieces: while
-// one piece is on its way the threads copy the previous one out (the caller's pages are
-// often touched for the first time here, which is what a single thread is slow at).
+// one piece is on its way the previous one is copied out, by several threads (128 MB: 2.8 ms,
+// about 10 by one).
 void copy_out(unsigned char* dst, const unsigned char* src_dev, size_t bytes, unsigned char* pin, size_t pin_bytes) {
   const size_t piece = pin_bytes / 2;
-  const int nt = copy_threads(bytes);
   auto send = [&](size_t i) {
     const size_t o = i * piece;
     if (o < bytes)
@@ -610,7 +609,7 @@ void copy_out(unsigned char* dst, const unsigned char* src_dev, size_t bytes, un
     send(i + 1);
     const size_t o = i * piece, len = std::min(piece, bytes - o);
     const unsigned char* from = pin + (i & 1) * piece;
-    copy_parallel(dst + o, from, len, nt);
+    CopyHelpers::get().copy(dst + o, from, len);
   }
 }
 
@@ -694,6 +693,7 @@ void ksum(int n, int nw, const double* Gc, const double* V0, int nterm, const do
   if (mode == 3) k_ksum_reduce<<<nw, 64, 0, st>>>(parts, 0, 0, d + o_part, 1.0 / nk, d + o_out);
   QED_HIP(hipGetLastError());
   QED_HIP(hipEventRecord(L->ev[1], st));
+  if (!small) touch_pages(reinterpret_cast<unsigned char*>(out), out_len * 8);  // while the kernels run
   QED_HIP(hipMemcpyAsync(h, ld, (small ? n_down : (size_t)nw + 1) * 8, hipMemcpyDeviceToHost, st));
   QED_HIP(hipStreamSynchronize(st));
   int bad = 0;
