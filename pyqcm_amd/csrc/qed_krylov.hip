@@ -589,7 +589,8 @@ void lanczos_gs(qed_sector& s, double accur, int max_iter, double* psi, double* 
   int slot = 0;
   bool converged = !(2.0 * accur > accur);  // as the loop of the scalar form: no step for such accur
   auto launch = [&] {
-    const int c = std::max(1, std::min(chunk, max_iter + 1 - launched));
+    // as many as there may be and one more, at which the limit is seen (the limit may be INT_MAX)
+    const int left = max_iter - launched, c = left >= chunk ? chunk : std::max(1, left + 1);
     for (int i = 0; i < c; ++i) run.step();
     launched += c;
     run.fetch(host->pin + slot * 2 * kLzRing);

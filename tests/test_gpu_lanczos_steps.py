@@ -83,6 +83,21 @@ def test_iteration_limit(gpu_lib, size):
     S.close()
 
 
+def test_largest_iteration_limit(gpu_lib):
+    """No limit to speak of (INT_MAX): the same run as with the default one."""
+    from pyqcm_amd._lib import DeviceArray
+    from pyqcm_amd.sector import Sector
+    m, v = TM.square(2, 4, tp=-0.3)
+    S = Sector(8, 4, 4, m.flat(v))
+    x = np.random.default_rng(2).standard_normal(S.dim)
+    x /= np.linalg.norm(x)
+    E0, psi, n, _, _ = S.lanczos_gs(start=x)
+    y, E1, n1 = DeviceArray.from_host(x), np.zeros(1), np.zeros(1, np.int32)
+    gpu_lib.call("qed_lanczos_gs", S.h, 1e-12, 2**31 - 1, y.ptr, gpu_lib.dp(E1), gpu_lib.ip(n1), None, None)
+    assert (E1[0], n1[0]) == (E0, n)
+    np.testing.assert_array_equal(y.to_host(), psi.to_host())
+
+
 def test_vector_aligned_to_eight_bytes(gpu_lib):
     """A start vector behind one double of another buffer, on the two-column kernel of long
     rows: the same numbers as from an aligned one, and nothing written around it."""
