@@ -44,13 +44,17 @@ constexpr int kBM = kBandVectors;      // vectors per multi-operation
 // Chunks of a launch that leave half of the chip idle: a pass is then bound by the latency of
 // each thread's chain of loads, and its work is spread over more threads with every sum in
 // its old order (8 sites, 2 chunks a part: multi-dot 25 -> 6.2 us, band subtraction 14 -> 6.7,
-// update before the product 13 -> 5.6). Above, the vectors' bytes bound a pass and one read
-// of x serves all of a block's vectors.
+// update before the product 13 -> 5.6). Where the vectors' bytes bound a pass, one read of x
+// serves all of a block's vectors. Green functions of one instance in ms, spread out / not:
+// 8 sites (4 chunks) 13.5-15.6 / 20.7, 9 (16) 54-58 / 79, 10 (52) 33 / 52, but also 11 (180)
+// 126 / 153, 12 (716) 140 / 160, and a batch of 8 x 10 sites (416) 166 / 197: the line is on
+// the safe side of the crossing, which lies above 716 chunks.
 constexpr uint32_t kFewBlocks = 128;
 
 // An elementwise pass (D::kElementwise) over a vector that would leave most of the chip idle
-// takes a quarter of that: 8 sites, 3920 amplitudes, are two blocks else. Sums keep one
-// partition, and so one order of their terms, at all sizes.
+// takes a quarter of that: 8 sites, 3920 amplitudes, are two blocks else (9 sites: 54-58 ms
+// against 61 in whole chunks; above the line quarters would still be 4 to 9% better at 11 and
+// 12 sites). Sums keep one partition, and so one order of their terms, at all sizes.
 template <class D>
 __host__ __device__ inline uint64_t chunk_of(uint64_t n) {
   return D::kElementwise && n <= (1u << 17) ? kChunk / 4 : kChunk;
@@ -344,7 +348,10 @@ __global__ __launch_bounds__(kBT) void k_fill0(const VFill* __restrict__ d, int 
 // beta_{k-1}) w_k one pass. (The normalized recurrence took a scaling and a dot pass more,
 // 124 of 700 us for the sectors of 16 plaquettes with 8 bath orbitals, and its replay a
 // pass of 116 us; the 16 problems in all 1.514 -> 1.479 s.) The row form of the product at
-// all sizes: the tiled one, in two passes, has no place for the update.
+// all sizes: the tiled one, in two passes, has no place for the update. Small sectors lose
+// nothing by it: ground states and Green functions of 16 instances of 6 sites 60 -> 51 ms, of
+// 8 sites 135 -> 90 (64 instances 350 -> 288), of 9 sites 350 -> 255, of 8 with 10 sites
+// 260 -> 194 and of 4 with 12 sites 820 -> 640, all changes of these steps together.
 struct LJob {
   static constexpr bool kElementwise = false;
   double* v[2];
@@ -631,8 +638,8 @@ void lanczos_gs_batch(const std::vector<qed_sector*>& S, const std::vector<doubl
     A[j].reset(new DevBuf(n * 8));
     Bv[j].reset(new DevBuf(n * 8));
     QED_HIP(hipMemcpyAsync(A[j]->p, psi[j], n * 8, hipMemcpyDeviceToDevice, stream()));
-    T.add(LJob{{A[j]->as<double>(), Bv[j]->as<double>()}, alpha + (size_t)j * ld, beta + (size_t)j * ld, rows, S[j]->dd, n, 0},
-          n);
+    const size_t at = (size_t)j * ld;
+    T.add(LJob{{A[j]->as<double>(), Bv[j]->as<double>()}, alpha + at, beta + at, rows, S[j]->dd, n, 0}, n);
     rows += S[j]->dd;
     F.add(VFill{Bv[j]->as<double>(), n, 0}, n);
   }
@@ -912,8 +919,8 @@ void band_lanczos_batch(const std::vector<qed_sector*>& S, const std::vector<con
   }
   // staging bounds: per step at most 8 + 2 kBM tables of nj descriptors, the H.v job table
   // and the activity flags
-  const size_t per_table =
-      (size_t)std::max(1, nj) * (std::max({sizeof(MAxpy), sizeof(MTail), sizeof(MRev), sizeof(MDot)}) + sizeof(uint32_t)) + 256;
+  const size_t per_job = std::max({sizeof(MAxpy), sizeof(MTail), sizeof(MRev), sizeof(MDot)}) + sizeof(uint32_t);
+  const size_t per_table = (size_t)std::max(1, nj) * per_job + 256;
   Stager stage1, stage2;
   stage1.init(2 * per_table + 256);
   stage2.init((8 + 2 * (size_t)kBM) * per_table + (size_t)std::max(1, nj) * (sizeof(HvJob) + sizeof(int)) + 4096);

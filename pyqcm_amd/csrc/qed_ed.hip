@@ -629,10 +629,12 @@ QMat sector_qmatrix(qed_sector& T, const double* phi, int p) {
 }
 
 // Sectors whose band Lanczos runs in the batched form, both parts of a Green function in
-// step: factorized, rows in LDS, few start vectors, and small enough that the host round
-// trips of the one-sector form cost more than its vectors (and that twice the vectors are
-// no burden). The products take the row form, so that the result does not depend on the
-// launch shape that is timed to be the fastest.
+// step: factorized, rows in LDS, few start vectors, and small enough that twice the vectors
+// are no burden (2 x 21 of 33 MB at the limit). One-sector form / batched, ms for G of one
+// instance: 6 sites 34 / 9.1, 8 100 / 15, 9 450 / 58, 10 361 / 34, 11 809 / 152, 12 778 / 161,
+// 13 (2.2 million states per part) 2335 / 940: the line is set by memory, not by time. The
+// products take the row form, so that the result does not depend on the launch shape that is
+// timed to be the fastest.
 bool batched_band(const qed_sector& T, int p) {
   return T.factorized() && p + 1 <= kBandVectors && T.D <= (1u << 22) && T.du <= 4096;
 }

@@ -161,7 +161,8 @@ template <int EP, int LOOK, class... Step>
 __global__ __launch_bounds__(256) void k_hv_general(const uint64_t* __restrict__ st, uint32_t n, LocateTables loc,
                                                     int L, const GHop* __restrict__ hops, int end_up, int end_dn,
                                                     int end_hop, const GDiag* __restrict__ diags, int ndiag,
-                                                    const double* __restrict__ x, double* __restrict__ y, Step... step) {
+                                                    const double* __restrict__ x, double* __restrict__ y,
+                                                    Step... step) {
   const LzStep& lz = step_of<LzStep>(step...);
   __shared__ uint16_t ranks[LOOK == kTablesLds ? 1 << kLdsRank : 1];
   if constexpr (LOOK == kTablesLds) {

@@ -130,17 +130,17 @@ struct KsumArgs {
   double* part;
 };
 
-__device__ __forceinline__ uint32_t dpp_max(uint32_t v, uint32_t w) { return v > w ? v : w; }
+__device__ __forceinline__ uint32_t larger(uint32_t v, uint32_t w) { return v > w ? v : w; }
 
 // the maximum of v over the LN lanes of a group (LN = 1, 2, 4, 8; aligned groups)
 template <int LN>
 __device__ __forceinline__ uint32_t group_max(uint32_t v) {
   if constexpr (LN >= 2)  // quad_perm [1,0,3,2]
-    v = dpp_max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xf, 0xf, true));
+    v = larger(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xf, 0xf, true));
   if constexpr (LN >= 4)  // quad_perm [2,3,0,1]
-    v = dpp_max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x4E, 0xf, 0xf, true));
+    v = larger(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x4E, 0xf, 0xf, true));
   if constexpr (LN >= 8)  // row_half_mirror: lane i of eight <-> 7 - i
-    v = dpp_max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x141, 0xf, 0xf, true));
+    v = larger(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x141, 0xf, 0xf, true));
   return v;
 }
 
@@ -195,7 +195,7 @@ __device__ __forceinline__ void eliminate(cplx (&a)[N / LN][N], int q, double2* 
     for (int s = 0; s < R; ++s) {
       const uint32_t mag = WIDE ? mag_bits_wide(a[s][k]) : mag_bits(a[s][k]);
       const uint32_t m = (mag & ~31u) | 16u | (uint32_t)(q + LN * s);
-      key = dpp_max(key, step[s] < 0 ? m : 0u);
+      key = larger(key, step[s] < 0 ? m : 0u);
     }
     key = group_max<LN>(key);
     const int p = (int)(key & 15u);
@@ -287,7 +287,8 @@ __global__ __launch_bounds__(256) void k_vk(int n, int nterm, int nk, const doub
       if (t < tc) {
         const double* v = nv + 3 * (t0 + t);
         double s, c;
-        sincospi(2.0 * (kk[3 * (size_t)kq] * v[0] + kk[3 * (size_t)kq + 1] * v[1] + kk[3 * (size_t)kq + 2] * v[2]), &s, &c);
+        const double* k3 = kk + 3 * (size_t)kq;
+        sincospi(2.0 * (k3[0] * v[0] + k3[1] * v[1] + k3[2] * v[2]), &s, &c);
         ph[u / TB][t] = make_double2(c, s);
       }
     }
@@ -484,7 +485,8 @@ __global__ __launch_bounds__(64) void k_ksum_reduce(int parts, int n, int N, con
     }
     re = wave_sum(re);
     im = wave_sum(im);
-    if (lane == 0) reinterpret_cast<double2*>(out)[(size_t)w * n * n + (size_t)j * n + i] = make_double2(re * scale, im * scale);
+    if (lane == 0)
+      reinterpret_cast<double2*>(out)[(size_t)w * n * n + (size_t)j * n + i] = make_double2(re * scale, im * scale);
   }
 }
 
@@ -601,7 +603,8 @@ void copy_out(unsigned char* dst, const unsigned char* src_dev, size_t bytes, un
   auto send = [&](size_t i) {
     const size_t o = i * piece;
     if (o < bytes)
-      QED_HIP(hipMemcpyAsync(pin + (i & 1) * piece, src_dev + o, std::min(piece, bytes - o), hipMemcpyDeviceToHost, stream()));
+      QED_HIP(hipMemcpyAsync(pin + (i & 1) * piece, src_dev + o, std::min(piece, bytes - o), hipMemcpyDeviceToHost,
+                             stream()));
   };
   send(0);
   for (size_t i = 0; i * piece < bytes; ++i) {
@@ -629,7 +632,8 @@ void ksum(int n, int nw, const double* Gc, const double* V0, int nterm, const do
   int parts = 0;
   for (int k0 = 0; k0 < nk; k0 += kmax)
     if (mode >= 2) parts += ((std::min(kmax, nk - k0) + G - 1) / G + chunk - 1) / chunk;
-  const size_t out_len = mode == 0 ? (size_t)nw * nk * n2 : mode == 1 ? (size_t)nw * nk * 2 : mode == 2 ? nw * n2 : (size_t)nw;
+  const size_t nwk = (size_t)nw * nk;
+  const size_t out_len = mode == 0 ? nwk * n2 : mode == 1 ? nwk * 2 : mode == 2 ? nw * n2 : (size_t)nw;
   // inputs in the order of the upload, then the device's own arrays (doubles)
   size_t off = 0;
   auto take = [&](size_t len) {
@@ -684,7 +688,8 @@ void ksum(int n, int nw, const double* Gc, const double* V0, int nterm, const do
       A.vk = d + o_vk;
       A.out = d + o_out;
       A.part = d + o_part;
-      k_vk<M><<<(A.nk + 7) / 8, 256, 0, st>>>(n, nterm, A.nk, d + o_v0, d + o_vt, d + o_nv, d + o_k + 3 * (size_t)k0, d + o_vk);
+      k_vk<M><<<(A.nk + 7) / 8, 256, 0, st>>>(n, nterm, A.nk, d + o_v0, d + o_vt, d + o_nv, d + o_k + 3 * (size_t)k0,
+                                              d + o_vk);
       launch_ksum<M>(A, mode, (mode < 2 ? nkb : nw) * A.nchunk);
       if (mode >= 2) part0 += A.nchunk;
     }
@@ -706,8 +711,8 @@ void ksum(int n, int nw, const double* Gc, const double* V0, int nterm, const do
       for (int w = 0; w < nw; ++w) out[w] += h[w];
   } else {
     std::vector<double> logdet(h, h + nw);
-    copy_out(reinterpret_cast<unsigned char*>(out), reinterpret_cast<const unsigned char*>(d + o_out), out_len * 8, L->pin,
-             2 * piece);
+    copy_out(reinterpret_cast<unsigned char*>(out), reinterpret_cast<const unsigned char*>(d + o_out), out_len * 8,
+             L->pin, 2 * piece);
     if (mode == 3)
       for (int w = 0; w < nw; ++w) out[w] += logdet[w];
   }

@@ -1129,8 +1129,9 @@ void hv_batch_step(const HvBatch& B, const HvBatchConfig& cfg, int parity, const
   const uint32_t* tj = B.tile_job.as<uint32_t>();
   auto go = [&](auto bs) {
     constexpr int BS = decltype(bs)::value;
-    if (L.kind == 1) k_hv_ell_batch<BS, 1><<<grid, BS, B.lds, stream()>>>(B.jobs, B.njobs, B.ntiles, parity, active, tj, L);
-    else k_hv_ell_batch<BS, 2><<<grid, BS, B.lds, stream()>>>(B.jobs, B.njobs, B.ntiles, parity, active, tj, L);
+    hipStream_t st = stream();
+    if (L.kind == 1) k_hv_ell_batch<BS, 1><<<grid, BS, B.lds, st>>>(B.jobs, B.njobs, B.ntiles, parity, active, tj, L);
+    else k_hv_ell_batch<BS, 2><<<grid, BS, B.lds, st>>>(B.jobs, B.njobs, B.ntiles, parity, active, tj, L);
   };
   if (cfg.block == 1024) go(std::integral_constant<int, 1024>{});
   else if (cfg.block == 512) go(std::integral_constant<int, 512>{});

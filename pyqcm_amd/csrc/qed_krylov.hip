@@ -120,9 +120,9 @@ __global__ __launch_bounds__(RB) void k_axpy_nrm(double a, const double* __restr
 // w_{k+1} = y - alpha_k v_k with alpha_k = <w_k, y> / beta_{k-1}; the parts of |w_{k+1}|^2.
 // Bound by its 24 bytes per element; each wave adds up the product's parts by itself, so
 // that a step is two launches and no scalar kernel (at most kLzParts parts).
-__global__ __launch_bounds__(RB) void k_lz_axpy_nrm(LzStep lz, int na, double* __restrict__ alpha, double* __restrict__ beta,
-                                                    const double* __restrict__ x, double* __restrict__ y, uint64_t n,
-                                                    double* __restrict__ part) {
+__global__ __launch_bounds__(RB) void k_lz_axpy_nrm(LzStep lz, int na, double* __restrict__ alpha,
+                                                    double* __restrict__ beta, const double* __restrict__ x,
+                                                    double* __restrict__ y, uint64_t n, double* __restrict__ part) {
   __shared__ double sh[RB / 64];
   const double b = lz.k == 0 ? 1.0 : sqrt(lz_sum(lz.pb, lz.nb));
   const double inv = lz_inv(b);

@@ -527,7 +527,8 @@ static int launch_mixed(const qed_sector& s, const double* x, double* y, const S
   auto k = T->packed ? (vl ? k_hv_mixed<true, true, EP, Step...> : k_hv_mixed<true, false, EP, Step...>)
                      : (vl ? k_hv_mixed<false, true, EP, Step...> : k_hv_mixed<false, false, EP, Step...>);
   k<<<grid, 256, 0, stream()>>>(view(b), b.up_ell.as<uint32_t>(), b.up_w, b.dn_ell.as<uint32_t>(), b.dn_w,
-                                T->full_of.as<uint32_t>(), T->len.as<uint32_t>(), T->code.as<uint32_t>(), n, b.dn_nvals, x, y, step...);
+                                T->full_of.as<uint32_t>(), T->len.as<uint32_t>(), T->code.as<uint32_t>(), n, b.dn_nvals,
+                                x, y, step...);
   QED_HIP(hipGetLastError());
   return (int)grid;
 }

@@ -239,11 +239,13 @@ def test_combine_mcf_from_qmatrix_matches_lehmann(gpu_lib, qr, seed):
         move = np.zeros(len(zs))
         for _ in range(8):
             eps = np.finfo(float).eps / 2
-            Gp, _n = _rewritten(e * (1 + eps * rng.choice([-1, 1], e.shape)), Q * (1 + eps * rng.choice([-1, 1], Q.shape)), qr, zs)
+            near = [a * (1 + eps * rng.choice([-1, 1], a.shape)) for a in (e, Q)]
+            Gp, _ = _rewritten(*near, qr, zs)
             move = np.maximum(move, np.abs(Gp - Go).max((1, 2)))
         err_o = np.abs(GC[s] - Go).max((1, 2))
         print("spin %d: %d floors (oracle %d), max |G_combined - G_L| = %.3g, vs oracle %s, its own moves %s"
-              % (s, len(A), floors, err, " ".join("%.1e" % x for x in err_o), " ".join("%.1e" % x for x in move)), flush=True)
+              % (s, len(A), floors, err, " ".join("%.1e" % x for x in err_o), " ".join("%.1e" % x for x in move)),
+              flush=True)
         assert (err_o <= 10 * move + 1e-14).all()
         assert err < 1e-5
 
