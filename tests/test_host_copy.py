@@ -67,6 +67,6 @@ def test_copy_with_and_without_helpers(tmp_path, limited):
     subprocess.check_call(["g++", "-O1", "-std=c++17", "-pthread", "-I", os.path.join(ROOT, "pyqcm_amd", "csrc"),
                            str(src), "-o", str(exe)])
     # a new thread's stack is as large as this limit when the program starts
-    cmd = "ulimit -s 131072 && exec %s limited" % exe if limited else str(exe)
+    cmd = "ulimit -s 131072; exec %s limited" % exe if limited else str(exe)
     r = subprocess.run(["bash", "-c", cmd], capture_output=True, text=True, timeout=100)
     assert r.returncode == 0, (r.returncode, r.stdout, r.stderr)
